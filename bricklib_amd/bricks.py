@@ -313,10 +313,23 @@ class Plan:
         self.handle = h.value
         self.shape = shape
         self.kcol = int(kcol)
+        self.boxed = False  # set_box ran
         nu, nc = C.c_uint32(), C.c_uint32()
         check(load().bk_plan_query(_vp(self.handle), C.byref(nu), None, None, C.byref(nc)))
         self.nunits = nu.value
         self.ncovered = nc.value
+
+    def set_box(self, info: BrickInfo, nb, ids: np.ndarray, pairs: np.ndarray) -> None:
+        """Declare the plan's bricks a periodic box (bk_plan_set_box): ``ids``
+        its nb[0] x nb[1] x nb[2] bricks in grid order (k slowest), ``pairs``
+        the (dst, src) ghost pairs, flat.  Sequences of sweeps that refresh
+        with those pairs may then take several sweeps per pass."""
+        ids = np.ascontiguousarray(ids, np.uint32)
+        pairs = np.ascontiguousarray(pairs, np.uint32)
+        check(load().bk_plan_set_box(_vp(self.handle), info.adj.ctypes.data_as(_lib.u32p),
+                                     longs(nb), ids.ctypes.data_as(_lib.u32p),
+                                     pairs.ctypes.data_as(_lib.u32p), pairs.size // 2))
+        self.boxed = True
 
     def __del__(self):
         try:
@@ -363,6 +376,8 @@ DEFAULT_PLANS = {
     (2, BK_BF16): ("quad", 8),
     (3, BK_F64): ("quad", 6), (3, BK_F32): ("quad", 6), (3, BK_BF16): ("quad", 6),
 }
+# Stencils whose sequences may take several sweeps per pass (bk_plan_set_box).
+STEP_STENCILS = (_lib.BK_STAR7, _lib.BK_COND7)
 # lane_shift of the quad star kernels per (stencil, dtype); absent = 0 (the
 # i-taps from the LDS tile).
 DEFAULT_LANE_SHIFT: dict = {}
@@ -459,6 +474,16 @@ class PeriodicGrid:
             blist = np.arange(self.nbricks, dtype=np.uint32) if every else self.sweep_list
             self._plans[key] = Plan(self.info, blist, shape, kcol)
         return self._plans[key]
+
+    def _declare_box(self, plan) -> None:
+        """Declare one of this grid's own quad plans a periodic box, once,
+        ahead of a sequence that may take several sweeps per pass."""
+        if plan.shape != "quad" or plan.boxed or not any(plan is p for p in self._plans.values()):
+            return
+        try:
+            plan.set_box(self.info, self.nb, self.interior, self.pairs)
+        except _lib.BrickError:  # not a periodic box (changed tables): one sweep per pass
+            plan.boxed = True
 
     @property
     def ghost_images(self):
@@ -669,6 +694,8 @@ def sweeps(st: Stencil, a: Brick, b: Brick, grid: PeriodicGrid, nsweeps: int,
     d = _desc(st, b, a, grid, keep, plan=plan, wg_bricks=wg_bricks, lane_shift=lane_shift)
     pairs = grid.d_pairs.ptr if (refresh and grid.d_pairs is not None) else None
     npairs = grid.npairs if refresh else 0
+    if nsweeps > 3 and keep[-1] is not None and st.kind in STEP_STENCILS and ghost_iters == 1:
+        grid._declare_box(keep[-1])
     if fused:
         if ghost_iters != 1:
             raise ValueError("the fused refresh refreshes every sweep (ghost_iters = 1)")

@@ -46,6 +46,10 @@ struct PlanView {
   const uint32_t *start;
   uint32_t nbricks;  // bricks of the adjacency the plan was built on
   uint64_t id;       // unique per plan (graph-cache key), never 0
+  // periodic box (bk_plan_set_box): its brick ids in grid order, or null
+  const uint32_t *box_ids;
+  uint32_t box_nb[3];
+  uint32_t box_npairs;  // ghost pairs that refresh its ghost bricks
 };
 const PlanView plan_view(const bk_plan_s *p);
 
@@ -66,6 +70,12 @@ hipError_t launch_star_columns(const SweepLaunch &L, const PlanView &P, hipStrea
 // Stars over 2x2 column quads: four waves share one LDS tile of the block.
 hipError_t launch_star_quads(const SweepLaunch &L, const PlanView &P, hipStream_t s);
 hipError_t launch_cube_quads(const SweepLaunch &L, const PlanView &P, hipStream_t s);
+// Several sweeps per pass over a periodic box (bk_steps.hip): whether the
+// kernels take the sweep (plan, stencil, alignment), the passes' costs, and
+// one pass of ts sweeps, 3 or 4, from L.in to L.out.
+bool steps_fit(const SweepLaunch &L, const PlanView &P);
+void steps_costs(const SweepLaunch &L, const PlanView &P, float cost[5]);
+hipError_t launch_star_steps(const SweepLaunch &L, const PlanView &P, int ts, hipStream_t s);
 
 int plan_fail(int code, const char *msg);
 

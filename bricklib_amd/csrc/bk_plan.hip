@@ -18,8 +18,8 @@
 #include <array>
 #include <atomic>
 #include <cstring>
+#include <new>
 #include <string>
-#include <unordered_map>
 #include <vector>
 
 #include "bk_api.h"
@@ -27,9 +27,6 @@
 
 namespace bk {
 int plan_fail(int code, const char *msg);
-int plan_build(const uint32_t *h_adj, uint32_t nbricks, const uint32_t *h_list, uint32_t nlist,
-               int shape, uint32_t kcol, uint32_t *h_anchor, uint32_t *h_len, uint32_t *h_mask,
-               uint32_t *h_flat, uint32_t *h_start, uint32_t *nunits, uint32_t *ncovered);
 void graphs_forget_plan(uint64_t plan_id);
 }
 
@@ -38,6 +35,7 @@ struct bk_plan_s {
   uint32_t kcol = 1;
   uint32_t nunits = 0;
   uint32_t ncovered = 0;
+  uint32_t *d_arrays = nullptr;  // one allocation holding the arrays below
   uint32_t *d_anchor = nullptr;  // [nunits] level-0 anchor
   uint32_t *d_len = nullptr;     // [nunits] levels in the unit
   uint32_t *d_mask = nullptr;    // [nunits * kcol] member store mask per level
@@ -46,6 +44,11 @@ struct bk_plan_s {
   uint32_t nbricks = 0;          // bricks of the adjacency the plan was built on
   int device = 0;
   uint64_t id = 0;               // unique per plan for the process's lifetime (never 0)
+  std::vector<bool> covered;     // [nbricks] the covered bricks
+  // periodic box (bk_plan_set_box): brick ids in grid order, in HBM
+  uint32_t *d_box = nullptr;
+  uint32_t box_nb[3] = {0, 0, 0};
+  uint32_t box_npairs = 0;
 };
 
 namespace {
@@ -67,6 +70,9 @@ const PlanView plan_view(const bk_plan_s *p) {
   v.start = p->d_start;
   v.nbricks = p->nbricks;
   v.id = p->id;
+  v.box_ids = p->d_box;
+  for (int a = 0; a < 3; ++a) v.box_nb[a] = p->box_nb[a];
+  v.box_npairs = p->box_npairs;
   return v;
 }
 
@@ -74,45 +80,50 @@ const PlanView plan_view(const bk_plan_s *p) {
 
 namespace {
 
-struct Unit {
-  uint32_t anchor;
-  std::vector<uint32_t> masks;
+constexpr uint32_t kNone = UINT32_MAX;
+
+// The units of a plan: unit u has its level-0 anchor and masks
+// mask[first[u]] .. mask[first[u + 1] - 1], one per level.
+struct Units {
+  std::vector<uint32_t> anchor, first, mask;
+  uint32_t count() const { return (uint32_t)anchor.size(); }
+  uint32_t levels(uint32_t u) const { return first[u + 1] - first[u]; }
 };
 
 // Build k-chains of "cells" (a cell = one brick for columns, one quad level
 // for quads) keyed by their anchor brick, then cut them into units.
-void chain_cells(const uint32_t *adj, const std::vector<uint32_t> &cell_anchor,
-                 const std::vector<uint32_t> &cell_mask, uint32_t kcol,
-                 std::vector<Unit> &units) {
-  std::unordered_map<uint32_t, uint32_t> by_anchor;
-  by_anchor.reserve(cell_anchor.size() * 2);
-  for (uint32_t c = 0; c < cell_anchor.size(); ++c) by_anchor.emplace(cell_anchor[c], c);
-  std::vector<char> used(cell_anchor.size(), 0);
+void chain_cells(const uint32_t *adj, uint32_t nbricks, const std::vector<uint32_t> &cell_anchor,
+                 const std::vector<uint32_t> &cell_mask, uint32_t kcol, Units &units) {
+  std::vector<uint32_t> by_anchor(nbricks, kNone);  // an anchor's unused cell
+  for (uint32_t c = 0; c < cell_anchor.size(); ++c) by_anchor[cell_anchor[c]] = c;
+  units.first.push_back(0);
+  units.mask.reserve(cell_anchor.size());
   for (uint32_t c = 0; c < cell_anchor.size(); ++c) {
-    if (used[c]) continue;
+    if (by_anchor[cell_anchor[c]] == kNone) continue;
     // walk up from c while the k+1 anchor is an unused cell
     uint32_t cur = c;
-    Unit u;
-    u.anchor = cell_anchor[cur];
+    uint32_t anchor = cell_anchor[cur];
     for (;;) {
-      used[cur] = 1;
-      u.masks.push_back(cell_mask[cur]);
-      if (u.masks.size() == kcol) {
-        units.push_back(u);
-        u.masks.clear();
+      by_anchor[cell_anchor[cur]] = kNone;
+      units.mask.push_back(cell_mask[cur]);
+      if (units.mask.size() - units.first.back() == kcol) {
+        units.anchor.push_back(anchor);
+        units.first.push_back((uint32_t)units.mask.size());
       }
       const uint32_t up = adj[(size_t)cell_anchor[cur] * 27 + 22];
-      auto it = by_anchor.find(up);
-      if (it == by_anchor.end() || used[it->second]) break;
+      if (by_anchor[up] == kNone) break;
       // the kernels hand a level's top planes to the next level as its k-1
       // face: link only where the adjacency agrees both ways (it does not
       // on the outer layer of a non-periodic grid, whose out-of-range
       // entries stand for no brick)
       if (adj[(size_t)up * 27 + 4] != cell_anchor[cur]) break;
-      cur = it->second;
-      if (u.masks.empty()) u.anchor = cell_anchor[cur];
+      cur = by_anchor[up];
+      if (units.mask.size() == units.first.back()) anchor = cell_anchor[cur];
     }
-    if (!u.masks.empty()) units.push_back(u);
+    if (units.mask.size() != units.first.back()) {
+      units.anchor.push_back(anchor);
+      units.first.push_back((uint32_t)units.mask.size());
+    }
   }
 }
 
@@ -125,11 +136,11 @@ void chain_cells(const uint32_t *adj, const std::vector<uint32_t> &cell_anchor,
 // every level are what those tables give -- always on a periodic grid and
 // on the interior of a padded one, not on the outer layer of a
 // non-periodic grid.
-bool quad_unit_consistent(const uint32_t *adj, const Unit &u) {
+bool quad_unit_consistent(const uint32_t *adj, uint32_t anchor, const uint32_t *masks, int L,
+                          std::vector<std::array<uint32_t, 16>> &T) {
   auto A = [adj](uint32_t b, int s) { return adj[(size_t)b * 27 + s]; };
-  const uint32_t m0 = u.anchor, m1 = A(m0, 14), m2 = A(m0, 16), m3 = A(m1, 16);
-  const int L = (int)u.masks.size();
-  std::vector<std::array<uint32_t, 16>> T((size_t)L + 2);  // T[l + 1]: level l
+  const uint32_t m0 = anchor, m1 = A(m0, 14), m2 = A(m0, 16), m3 = A(m1, 16);
+  T.resize((size_t)L + 2);  // T[l + 1]: level l
   for (int e = 0; e < 16; ++e) {
     const int r = e >> 2, c = e & 3;
     const uint32_t m = r < 3 ? (c < 3 ? m0 : m1) : (c < 3 ? m2 : m3);
@@ -144,7 +155,7 @@ bool quad_unit_consistent(const uint32_t *adj, const Unit &u) {
     if (l > 0)
       for (auto &b : om) b = A(b, 22);
     for (int mm = 0; mm < 4; ++mm) {
-      if (!((u.masks[l] >> mm) & 1u)) continue;
+      if (!((masks[l] >> mm) & 1u)) continue;
       for (int kd = 0; kd < 3; ++kd)
         for (int jd = 0; jd < 3; ++jd)
           for (int id = 0; id < 3; ++id)
@@ -158,23 +169,15 @@ bool quad_unit_consistent(const uint32_t *adj, const Unit &u) {
 
 }  // namespace
 
-extern "C" {
+namespace {
 
-int bk_plan_build_host(const uint32_t *h_adj, uint32_t nbricks, const uint32_t *h_list,
-                       uint32_t nlist, int shape, uint32_t kcol, uint32_t *h_anchor,
-                       uint32_t *h_len, uint32_t *h_mask, uint32_t *h_flat, uint32_t *nunits,
-                       uint32_t *ncovered) {
-  return bk::plan_build(h_adj, nbricks, h_list, nlist, shape, kcol, h_anchor, h_len, h_mask,
-                        h_flat, nullptr, nunits, ncovered);
-}
+// A plan's arrays on the host.
+struct PlanArrays {
+  std::vector<uint32_t> anchor, len, mask, flat, start;
+};
 
-}  // extern "C"
-
-namespace bk {
 int plan_build(const uint32_t *h_adj, uint32_t nbricks, const uint32_t *h_list, uint32_t nlist,
-               int shape, uint32_t kcol, uint32_t *h_anchor, uint32_t *h_len, uint32_t *h_mask,
-               uint32_t *h_flat, uint32_t *h_start, uint32_t *nunits, uint32_t *ncovered) {
-  if (!nunits || !ncovered) return bk::plan_fail(BK_ERR_ARG, "bk_plan_build_host: null count pointer");
+               int shape, uint32_t kcol, PlanArrays &out) {
   if (!h_adj || (nlist && !h_list))
     return bk::plan_fail(BK_ERR_ARG, "bk_plan_build_host: null pointer");
   if (shape != BK_PLAN_COLUMN && shape != BK_PLAN_QUAD)
@@ -182,11 +185,15 @@ int plan_build(const uint32_t *h_adj, uint32_t nbricks, const uint32_t *h_list, 
   if (kcol == 0 || kcol > 4096) return bk::plan_fail(BK_ERR_ARG, "bk_plan: kcol in [1, 4096]");
   for (uint32_t l = 0; l < nlist; ++l)
     if (h_list[l] >= nbricks) return bk::plan_fail(BK_ERR_ARG, "bk_plan: list entry out of range");
-  for (size_t q = 0; q < (size_t)nbricks * 27; ++q)
-    if (h_adj[q] >= nbricks) return bk::plan_fail(BK_ERR_ARG, "bk_plan: adjacency entry out of range");
+  uint32_t most = 0;
+  for (size_t q = 0; q < (size_t)nbricks * 27; ++q) most = std::max(most, h_adj[q]);
+  if (nbricks && most >= nbricks)
+    return bk::plan_fail(BK_ERR_ARG, "bk_plan: adjacency entry out of range");
 
-  std::vector<uint8_t> listed(nbricks, 0), covered(nbricks, 0);
-  for (uint32_t l = 0; l < nlist; ++l) listed[h_list[l]] = 1;
+  // an entry's first position in the list (kNone: not listed)
+  std::vector<uint32_t> pos(nbricks, kNone);
+  for (uint32_t l = nlist; l-- > 0;) pos[h_list[l]] = l;
+  std::vector<uint8_t> covered(nbricks, 0);
 
   std::vector<uint32_t> cell_anchor, cell_mask;
   for (uint32_t l = 0; l < nlist; ++l) {
@@ -204,7 +211,7 @@ int plan_build(const uint32_t *h_adj, uint32_t nbricks, const uint32_t *h_list, 
       for (int q = 0; q < 4; ++q) {
         bool dup = false;
         for (int p = 0; p < q; ++p) dup = dup || mem[p] == mem[q];
-        if (!dup && listed[mem[q]] && !covered[mem[q]]) {
+        if (!dup && pos[mem[q]] != kNone && !covered[mem[q]]) {
           covered[mem[q]] = 1;
           mask |= 1u << q;
         }
@@ -213,65 +220,80 @@ int plan_build(const uint32_t *h_adj, uint32_t nbricks, const uint32_t *h_list, 
       cell_mask.push_back(mask);
     }
   }
-  std::vector<Unit> units;
-  chain_cells(h_adj, cell_anchor, cell_mask, kcol, units);
-  if (shape == BK_PLAN_QUAD)
-    for (const Unit &u : units)
-      if (!quad_unit_consistent(h_adj, u))
+  Units units;
+  chain_cells(h_adj, nbricks, cell_anchor, cell_mask, kcol, units);
+  const uint32_t nu = units.count();
+  if (shape == BK_PLAN_QUAD) {
+    std::vector<std::array<uint32_t, 16>> tables;
+    for (uint32_t u = 0; u < nu; ++u)
+      if (!quad_unit_consistent(h_adj, units.anchor[u], &units.mask[units.first[u]],
+                                (int)units.levels(u), tables))
         return bk::plan_fail(BK_ERR_UNSUPPORTED,
                              "bk_plan: a quad of the list has neighbours the adjacency does not "
                              "place consistently (the outer layer of a non-periodic grid); use "
                              "a column plan or no plan for such lists");
+  }
   // emit units in the list order of their anchors (for a grid-ordered list:
   // k-segment by k-segment, so units that run together are neighbours)
-  {
-    std::unordered_map<uint32_t, uint32_t> pos;
-    pos.reserve((size_t)nlist * 2);
-    for (uint32_t l = 0; l < nlist; ++l) pos.emplace(h_list[l], l);
-    std::vector<std::pair<uint32_t, uint32_t>> key(units.size());
-    for (uint32_t u = 0; u < units.size(); ++u) {
-      auto it = pos.find(units[u].anchor);
-      key[u] = {it == pos.end() ? UINT32_MAX : it->second, u};
-    }
-    std::stable_sort(key.begin(), key.end());
-    std::vector<Unit> sorted;
-    sorted.reserve(units.size());
-    for (auto &k : key) sorted.push_back(std::move(units[k.second]));
-    units.swap(sorted);
-  }
+  std::vector<std::pair<uint32_t, uint32_t>> key(nu);
+  for (uint32_t u = 0; u < nu; ++u) key[u] = {pos[units.anchor[u]], u};
+  std::stable_sort(key.begin(), key.end());
 
-  uint32_t nf = 0;
-  for (size_t u = 0; u < units.size(); ++u) {
-    if (h_start) h_start[u] = nf;
-    if (h_anchor) h_anchor[u] = units[u].anchor;
-    if (h_len) h_len[u] = (uint32_t)units[u].masks.size();
-    uint32_t a = units[u].anchor;
-    for (size_t l = 0; l < kcol; ++l) {
-      const uint32_t m = l < units[u].masks.size() ? units[u].masks[l] : 0u;
-      if (h_mask) h_mask[u * kcol + l] = m;
-      if (l >= units[u].masks.size()) continue;
+  out.anchor.resize(nu);
+  out.len.resize(nu);
+  out.start.resize(nu);
+  out.mask.assign((size_t)nu * kcol, 0u);
+  out.flat.clear();
+  out.flat.reserve(nlist);
+  for (uint32_t q = 0; q < nu; ++q) {
+    const uint32_t u = key[q].second, L = units.levels(u);
+    uint32_t a = units.anchor[u];
+    out.start[q] = (uint32_t)out.flat.size();
+    out.anchor[q] = a;
+    out.len[q] = L;
+    for (uint32_t l = 0; l < L; ++l) {
+      const uint32_t m = units.mask[units.first[u] + l];
+      out.mask[(size_t)q * kcol + l] = m;
       if (shape == BK_PLAN_COLUMN) {
-        if (m & 1u) {
-          if (h_flat) h_flat[nf] = a;
-          ++nf;
-        }
+        if (m & 1u) out.flat.push_back(a);
       } else {
         const uint32_t m1 = h_adj[(size_t)a * 27 + 14];
         const uint32_t mem[4] = {a, m1, h_adj[(size_t)a * 27 + 16], h_adj[(size_t)m1 * 27 + 16]};
-        for (int q = 0; q < 4; ++q)
-          if (m & (1u << q)) {
-            if (h_flat) h_flat[nf] = mem[q];
-            ++nf;
-          }
+        for (int b = 0; b < 4; ++b)
+          if (m & (1u << b)) out.flat.push_back(mem[b]);
       }
       a = h_adj[(size_t)a * 27 + 22];
     }
   }
-  *nunits = (uint32_t)units.size();
-  *ncovered = nf;
   return BK_OK;
 }
-}  // namespace bk
+
+}  // namespace
+
+extern "C" {
+
+int bk_plan_build_host(const uint32_t *h_adj, uint32_t nbricks, const uint32_t *h_list,
+                       uint32_t nlist, int shape, uint32_t kcol, uint32_t *h_anchor,
+                       uint32_t *h_len, uint32_t *h_mask, uint32_t *h_flat, uint32_t *nunits,
+                       uint32_t *ncovered) {
+  if (!nunits || !ncovered)
+    return bk::plan_fail(BK_ERR_ARG, "bk_plan_build_host: null count pointer");
+  PlanArrays A;
+  const int rc = plan_build(h_adj, nbricks, h_list, nlist, shape, kcol, A);
+  if (rc != BK_OK) return rc;
+  auto put = [](uint32_t *dst, const std::vector<uint32_t> &v) {
+    if (dst) std::copy(v.begin(), v.end(), dst);
+  };
+  put(h_anchor, A.anchor);
+  put(h_len, A.len);
+  put(h_mask, A.mask);
+  put(h_flat, A.flat);
+  *nunits = (uint32_t)A.anchor.size();
+  *ncovered = (uint32_t)A.flat.size();
+  return BK_OK;
+}
+
+}  // extern "C"
 
 extern "C" {
 
@@ -279,40 +301,43 @@ int bk_plan_create(const uint32_t *h_adj, uint32_t nbricks, const uint32_t *h_li
                    uint32_t nlist, int shape, uint32_t kcol, bk_plan *out) {
   if (!out) return bk::plan_fail(BK_ERR_ARG, "bk_plan_create: null out pointer");
   *out = nullptr;
-  uint32_t nu = 0, nc = 0;
-  // sizes first (nunits <= nlist), then the arrays
-  int rc = bk::plan_build(h_adj, nbricks, h_list, nlist, shape, kcol, nullptr, nullptr, nullptr,
-                          nullptr, nullptr, &nu, &nc);
-  if (rc != BK_OK) return rc;
-  std::vector<uint32_t> anchor(nu), len(nu), mask((size_t)nu * kcol), flat(nc), start(nu);
-  rc = bk::plan_build(h_adj, nbricks, h_list, nlist, shape, kcol, anchor.data(), len.data(),
-                      mask.data(), flat.data(), start.data(), &nu, &nc);
+  PlanArrays A;
+  const int rc = plan_build(h_adj, nbricks, h_list, nlist, shape, kcol, A);
   if (rc != BK_OK) return rc;
 
   bk_plan_s *p = new bk_plan_s();
   p->shape = shape;
   p->kcol = kcol;
-  p->nunits = nu;
-  p->ncovered = nc;
+  p->nunits = (uint32_t)A.anchor.size();
+  p->ncovered = (uint32_t)A.flat.size();
   p->nbricks = nbricks;
   p->id = g_next_plan_id.fetch_add(1);
   (void)hipGetDevice(&p->device);  // the current device owns the arrays below
-  auto up = [](uint32_t **dst, const std::vector<uint32_t> &v) -> hipError_t {
-    if (v.empty()) return hipSuccess;
-    hipError_t e = hipMalloc(dst, v.size() * sizeof(uint32_t));
-    if (e != hipSuccess) return e;
-    return hipMemcpy(*dst, v.data(), v.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
-  };
-  hipError_t e = up(&p->d_anchor, anchor);
-  if (e == hipSuccess) e = up(&p->d_len, len);
-  if (e == hipSuccess) e = up(&p->d_mask, mask);
-  if (e == hipSuccess) e = up(&p->d_flat, flat);
-  if (e == hipSuccess) e = up(&p->d_start, start);
-  if (e != hipSuccess) {
-    bk_plan_destroy(p);
-    std::string m = std::string("bk_plan_create: ") + hipGetErrorString(e);
-    return bk::plan_fail(e == hipErrorOutOfMemory ? BK_ERR_NOMEM : BK_ERR_HIP, m.c_str());
+  // one allocation and one copy for all arrays, each from a 256-byte boundary
+  const std::vector<uint32_t> *arr[5] = {&A.anchor, &A.len, &A.mask, &A.flat, &A.start};
+  uint32_t **dst[5] = {&p->d_anchor, &p->d_len, &p->d_mask, &p->d_flat, &p->d_start};
+  size_t at[5], total = 0;
+  for (int q = 0; q < 5; ++q) {
+    at[q] = total;
+    total += (arr[q]->size() + 63) & ~(size_t)63;
   }
+  if (total) {
+    std::vector<uint32_t> all(total, 0u);
+    for (int q = 0; q < 5; ++q)
+      std::copy(arr[q]->begin(), arr[q]->end(), all.begin() + (ptrdiff_t)at[q]);
+    hipError_t e = hipMalloc(&p->d_arrays, total * sizeof(uint32_t));
+    if (e == hipSuccess)
+      e = hipMemcpy(p->d_arrays, all.data(), total * sizeof(uint32_t), hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+      bk_plan_destroy(p);
+      std::string m = std::string("bk_plan_create: ") + hipGetErrorString(e);
+      return bk::plan_fail(e == hipErrorOutOfMemory ? BK_ERR_NOMEM : BK_ERR_HIP, m.c_str());
+    }
+    for (int q = 0; q < 5; ++q)
+      if (!arr[q]->empty()) *dst[q] = p->d_arrays + at[q];
+  }
+  p->covered.assign(nbricks, false);
+  for (uint32_t b : A.flat) p->covered[b] = true;
   *out = p;
   return BK_OK;
 }
@@ -321,12 +346,81 @@ int bk_plan_destroy(bk_plan p) {
   if (!p) return BK_OK;
   // cached graphs captured the plan's device arrays: drop them first
   bk::graphs_forget_plan(p->id);
-  (void)hipFree(p->d_anchor);
-  (void)hipFree(p->d_len);
-  (void)hipFree(p->d_mask);
-  (void)hipFree(p->d_flat);
-  (void)hipFree(p->d_start);
+  (void)hipFree(p->d_arrays);
+  (void)hipFree(p->d_box);
   delete p;
+  return BK_OK;
+}
+
+int bk_plan_set_box(bk_plan p, const uint32_t *h_adj, const long nb[3], const uint32_t *h_ids,
+                    const uint32_t *h_pairs, uint32_t npairs) {
+  if (!p || !h_adj || !nb || !h_ids || (npairs && !h_pairs))
+    return bk::plan_fail(BK_ERR_ARG, "bk_plan_set_box: null pointer");
+  if (p->d_box) return bk::plan_fail(BK_ERR_ARG, "bk_plan_set_box: the plan has a box already");
+  for (int a = 0; a < 3; ++a)
+    if (nb[a] <= 0 || nb[a] > (long)p->nbricks)
+      return bk::plan_fail(BK_ERR_ARG, "bk_plan_set_box: bricks per axis out of range");
+  const uint64_t plane = (uint64_t)nb[0] * (uint64_t)nb[1];
+  if (plane > p->nbricks || plane * (uint64_t)nb[2] != p->ncovered)
+    return bk::plan_fail(BK_ERR_UNSUPPORTED,
+                         "bk_plan_set_box: the box does not have the plan's brick count");
+  // what each brick holds before a sweep: itself, or for a ghost brick the
+  // brick its pair copies onto it
+  std::vector<uint32_t> holds;
+  try {
+    holds.assign(p->nbricks, UINT32_MAX);
+  } catch (const std::bad_alloc &) {
+    return bk::plan_fail(BK_ERR_NOMEM, "bk_plan_set_box: out of host memory");
+  }
+  const size_t n = p->ncovered;
+  for (size_t q = 0; q < n; ++q) {
+    const uint32_t b = h_ids[q];
+    if (b >= p->nbricks || !p->covered[b] || holds[b] != UINT32_MAX)
+      return bk::plan_fail(BK_ERR_UNSUPPORTED,
+                           "bk_plan_set_box: the box is not the plan's bricks, each once");
+    holds[b] = b;
+  }
+  for (uint32_t q = 0; q < npairs; ++q) {
+    const uint32_t dst = h_pairs[2 * q], src = h_pairs[2 * q + 1];
+    if (dst >= p->nbricks || src >= p->nbricks || p->covered[dst])
+      return bk::plan_fail(BK_ERR_UNSUPPORTED,
+                           "bk_plan_set_box: a pair does not copy onto a ghost brick");
+    holds[dst] = src;
+  }
+  // every neighbour of every box brick holds the brick the wrapped box has
+  // there, so sweeps may read that brick instead
+  size_t q = 0;
+  for (long k = 0; k < nb[2]; ++k)
+    for (long j = 0; j < nb[1]; ++j) {
+      const uint32_t *row[9];
+      for (int e = 0; e < 9; ++e) {
+        const long kk = (k + e / 3 - 1 + nb[2]) % nb[2], jj = (j + e % 3 - 1 + nb[1]) % nb[1];
+        row[e] = h_ids + ((size_t)kk * (size_t)nb[1] + (size_t)jj) * (size_t)nb[0];
+      }
+      for (long i = 0; i < nb[0]; ++i, ++q) {
+        const uint32_t *ab = h_adj + (size_t)h_ids[q] * 27;
+        const long at[3] = {i ? i - 1 : nb[0] - 1, i, i + 1 < nb[0] ? i + 1 : 0};
+        for (int e = 0; e < 9; ++e)
+          for (int d = 0; d < 3; ++d) {
+            const uint32_t b = ab[e * 3 + d];
+            if (b >= p->nbricks || holds[b] != row[e][at[d]])
+              return bk::plan_fail(BK_ERR_UNSUPPORTED,
+                                   "bk_plan_set_box: the adjacency and pairs are not those of a "
+                                   "periodic box in this order");
+          }
+      }
+    }
+  uint32_t *d = nullptr;
+  hipError_t e = hipMalloc(&d, n * sizeof(uint32_t));
+  if (e == hipSuccess) e = hipMemcpy(d, h_ids, n * sizeof(uint32_t), hipMemcpyHostToDevice);
+  if (e != hipSuccess) {
+    (void)hipFree(d);
+    std::string m = std::string("bk_plan_set_box: ") + hipGetErrorString(e);
+    return bk::plan_fail(e == hipErrorOutOfMemory ? BK_ERR_NOMEM : BK_ERR_HIP, m.c_str());
+  }
+  p->d_box = d;
+  for (int a = 0; a < 3; ++a) p->box_nb[a] = (uint32_t)nb[a];
+  p->box_npairs = npairs;
   return BK_OK;
 }
 

@@ -238,6 +238,54 @@ hipError_t launch_sweep(const bk::SweepLaunch &L, const bk_plan_s *plan, hipStre
   return bk::launch_star(L, s);
 }
 
+// Sweeps per pass (bk_steps.hip) of a sequence whose last sweep runs by
+// itself: next() gives the sweeps of each pass over the n before it, 1 = one
+// plain sweep, 0 = none left.  The number of passes has the parity of n, so
+// the two fields end up holding what single sweeps leave in them -- the
+// result where the caller expects it and the sweep before it in the other
+// field.  The cheapest such split by the passes' measured costs.
+class SweepSplit {
+  static constexpr int kTable = 24;
+  int last_[kTable + 1][2];
+  int left_, par_, top_ = 1, again_ = 0;
+
+ public:
+  SweepSplit(int n, const float cost[5]) : left_(n), par_(n & 1) {
+    float best[kTable + 1][2];
+    for (int m = 0; m <= kTable; ++m)
+      for (int par = 0; par < 2; ++par) {
+        best[m][par] = m == 0 && par == 0 ? 0.0f : 1e30f;
+        last_[m][par] = 0;
+        for (int t = 1; t <= 4 && t <= m; ++t) {
+          const float c = best[m - t][par ^ 1] + cost[t];
+          if (c < best[m][par]) {
+            best[m][par] = c;
+            last_[m][par] = t;
+          }
+        }
+      }
+    // far from the end: the cheapest pass per sweep, in pairs (two passes
+    // and an even number of sweeps leave both parities alone)
+    for (int t = 2; t <= 4; ++t)
+      if (cost[t] * (float)top_ < cost[top_] * (float)t) top_ = t;
+  }
+  int next() {
+    if (again_) {
+      again_ = 0;
+      return top_;
+    }
+    if (left_ > kTable) {
+      left_ -= 2 * top_;
+      again_ = 1;
+      return top_;
+    }
+    const int t = left_ > 0 ? last_[left_][par_] : 0;
+    left_ -= t;
+    par_ ^= 1;
+    return t;
+  }
+};
+
 // Enqueue the ping-pong sequence of bk_sweeps on stream s.
 // The ping-pong sequence: before sweep t the ghost bricks of its input are
 // refreshed when t % ghost_iters == 0; sweep t covers the desc's brick list
@@ -255,6 +303,39 @@ hipError_t enqueue_sweeps(const bk_sweep_desc *d, const uint32_t *pairs, uint32_
   L.img_off = img_off;
   L.img = img;
   const size_t es = (size_t)dt_size(d->dtype);
+  // Several sweeps per pass where the plan's bricks are a periodic box whose
+  // ghost bricks this sequence refreshes before every sweep: the passes read
+  // the periodic image itself, and only the last sweep, which runs by itself,
+  // reads ghost bricks.
+  if (nsweeps > 2 && ghost_iters == 1 && d->plan && d->layout == BK_LAYOUT_8x8x8) {
+    const bk::PlanView P = bk::plan_view(d->plan);
+    if (P.shape == BK_PLAN_QUAD && P.box_npairs == npairs && bk::steps_fit(L, P)) {
+      float cost[5];
+      bk::steps_costs(L, P, cost);
+      SweepSplit split(nsweeps - 1, cost);
+      bool fwd = true, fresh = false;  // fresh: the input's ghost bricks are up to date
+      for (int ts = 1; ts; fwd = !fwd) {
+        ts = split.next();
+        L.in = fwd ? d->d_in : d->d_out;
+        L.in_step = fwd ? d->in_step : d->out_step;
+        L.out = fwd ? d->d_out : const_cast<void *>(d->d_in);
+        L.out_step = fwd ? d->out_step : d->in_step;
+        hipError_t e = hipSuccess;
+        if (ts > 1) {
+          e = bk::launch_star_steps(L, P, ts, s);
+          fresh = false;
+        } else {
+          if (npairs && !fresh)
+            e = bk::launch_ghost_refresh(const_cast<void *>(L.in), L.in_step * es, 512 * es,
+                                         pairs, npairs, s);
+          if (e == hipSuccess) e = launch_sweep(L, d->plan, s);
+          fresh = img_off != nullptr;
+        }
+        if (e != hipSuccess) return e;
+      }
+      return hipSuccess;
+    }
+  }
   for (int t = 0; t < nsweeps; ++t) {
     const bool fwd = (t % 2) == 0;
     void *src = fwd ? const_cast<void *>(d->d_in) : d->d_out;

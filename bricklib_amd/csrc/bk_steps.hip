@@ -1,0 +1,633 @@
+// bk_steps.hip -- several sweeps of a radius-1 stencil (7-point star, cond)
+// per pass over the field, for periodic boxes of 8x8x8 bricks on gfx950.
+//
+// bk_sweeps runs a loop of sweeps (weak/main.hip.cpp:274-279) whose every
+// step reads and writes the whole field: past the caches' size each sweep
+// costs a copy of the field, and a small box costs a launch per sweep.  Here
+// one pass reads the field once, applies TS sweeps in registers and writes
+// the result; the sweeps in between never reach memory.
+//
+// One wave owns a strip of J rows (j) of up to 7 bricks (V = 1; 15 for V = 2)
+// along i and marches along k.  Lane l holds V adjacent cells of every row.
+// The 64 V cells of a row are the strip's and kHalo halo cells a side, laid
+// round the wave as a ring -- strip first, right halo, left halo -- so the
+// i-taps are one-lane wave rotations (DPP) and groups of lanes fall on whole
+// brick rows.  For each sweep s of the pass the wave keeps two planes of the
+// field after s sweeps in registers (rows s .. NR-s-1 of the NR = J + 2 TS
+// input rows).  When a new input plane arrives, each row goes through all TS
+// sweeps at once:
+//   n_{s+1}[r] = stencil of plane s around row r: centre row and rows r +- 1
+//                from the newer kept plane, k+1 from n_s[r] just computed,
+//                k-1 from the older kept plane,
+// and n_s[r] then takes the older plane's place (the two planes swap roles
+// from step to step).  Of sweep 0 the wave keeps the last loaded plane, the
+// next one arriving while this one is used, and its older plane in LDS (each
+// lane its own cells, so no barrier).  A sweep's halo (one row and one cell a
+// side, one plane at either end of a march) is computed again by the
+// neighbours instead of exchanged: no wave waits for another.
+//
+// Per point and sweep the arithmetic is the other star kernels': acc = c0*x,
+// then fma over i+1, i-1, j+1, j-1, k+1, k-1; BF16 rounds after every sweep
+// as a store would.  The bits are those of single sweeps.
+//
+// What bounds it (512^3, 7-point, TS = 4): the VALU and HBM about equally.
+// FP64: 530 VALU instructions per wave and plane, 308 of them the stencil's;
+// without any memory traffic the pass takes 0.40 ms, its 1.31 GB of reads and
+// 1.07 GB of writes at the copy rate 0.45 ms; together 0.56 ms, 0.141 ms per
+// sweep against 0.393 for one sweep per pass (FP32 0.086 against 0.203, BF16
+// 0.089 against 0.117).  Three sweeps per pass: FP64 0.177, FP32 0.107 ms per
+// sweep.  Found on the way: with the strip from the left halo on (lanes
+// across brick edges) and one store per row 0.154; V = 2 in FP32 (fewer
+// rotations, two waves per SIMD instead of three) no faster; issuing the
+// first five taps of the next row among the last ones of this row, two rows
+// per scheduling group, or loads two planes ahead no faster.
+#include <algorithm>
+#include <atomic>
+#include <type_traits>
+
+#include "bk_device.h"
+#include "bk_internal.h"
+
+namespace bk {
+namespace {
+
+constexpr int kHalo = 4;  // halo cells at either end of a row (TS <= 4)
+
+// What the kernel computes: the 7-point star, or cond, keeping in registers
+// the values themselves (taps clamp them at 0) or the clamped ones.  Clamped
+// planes save the clamps of four taps in five; the select of the reference
+// form needs no kept value, and with a threshold theta >= 0 a value exceeds
+// theta exactly where its clamped one does.
+enum Form { kStar = 0, kCondRaw = 1, kCondPos = 2 };
+
+template <class T>
+struct StepArgs {
+  using A = typename acc_of<T>::type;
+  const uint32_t *__restrict__ ids;  // box bricks, ids[(bk*nb1 + bj)*nb0 + bi]
+  const T *__restrict__ in;
+  T *__restrict__ out;
+  uint64_t in_step;
+  uint64_t out_step;
+  uint32_t nb0, nb1, nb2;  // bricks of the box along i, j, k
+  uint32_t nchunk;         // strips along i
+  uint32_t njg;            // strips along j (nb1 * 8 / J)
+  uint32_t njw;            // workgroups along j (four strips each)
+  uint32_t ksegs;          // marches along k
+  int cond_mode;
+  A theta;
+  A c[7];
+};
+
+// V adjacent cells of a lane
+template <class A, int V>
+struct Cells {
+  A v[V];
+};
+
+// The value of the next (UP) or previous lane, the wave a ring of 64.
+template <bool UP>
+__device__ __forceinline__ uint32_t wave_turn32(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, UP ? 0x134 : 0x13c, 0xf, 0xf, true);
+}
+template <bool UP>
+__device__ __forceinline__ float wave_turn(float x) {
+  return __builtin_bit_cast(float, wave_turn32<UP>(__builtin_bit_cast(uint32_t, x)));
+}
+template <bool UP>
+__device__ __forceinline__ double wave_turn(double x) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = wave_turn32<UP>((uint32_t)u), hi = wave_turn32<UP>((uint32_t)(u >> 32));
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// The value of the next (UP) or previous lane of a 16-lane row.
+template <bool UP>
+__device__ __forceinline__ uint32_t row_next32(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, UP ? 0x101 : 0x111, 0xf, 0xf, true);
+}
+template <bool UP>
+__device__ __forceinline__ float row_next(float x) {
+  return __builtin_bit_cast(float, row_next32<UP>(__builtin_bit_cast(uint32_t, x)));
+}
+template <bool UP>
+__device__ __forceinline__ double row_next(double x) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = row_next32<UP>((uint32_t)u), hi = row_next32<UP>((uint32_t)(u >> 32));
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// a lane's V cells from memory
+__device__ __forceinline__ void load_cells(const double *p, Cells<double, 1> &x) { x.v[0] = *p; }
+__device__ __forceinline__ void load_cells(const float *p, Cells<float, 1> &x) { x.v[0] = *p; }
+__device__ __forceinline__ void load_cells(const bf16 *p, Cells<float, 1> &x) {
+  x.v[0] = widen(*p);
+}
+
+// what a store to T and the next sweep's load make of a sweep's values
+// (gfx950's conversion rounds as narrow() does: the same bits for all 2^32
+// inputs)
+template <class T, class A, int V>
+__device__ __forceinline__ void round_cells(Cells<A, V> &x) {
+  if constexpr (std::is_same<T, bf16>::value) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 h2 __attribute__((ext_vector_type(2)));
+    f2 t;
+    t.x = x.v[0];
+    t.y = x.v[V - 1];
+    const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(t, h2));
+    x.v[0] = __uint_as_float(u << 16);
+    if (V > 1) x.v[V - 1] = __uint_as_float(u & 0xffff0000u);
+  }
+}
+
+// Values of the lane `1` or `2` away in its group of four (quad_perm).
+__device__ __forceinline__ uint32_t quad_swap1(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xb1, 0xf, 0xf, true);
+}
+__device__ __forceinline__ uint32_t quad_swap2(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x4e, 0xf, 0xf, true);
+}
+__device__ __forceinline__ double quad_swap1(double x) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = quad_swap1((uint32_t)u), hi = quad_swap1((uint32_t)(u >> 32));
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// Output rows in groups of G, each lane storing 16 bytes of one row of the
+// group (a G x G exchange between G neighbouring lanes): a store instruction
+// then covers 128 contiguous bytes per brick -- a whole line -- where one row
+// is 64 (FP64) or 32 (FP32).  Row by row the FP64 pass took 0.62 ms against
+// 0.58, the FP32 one 0.42 against 0.34.  BF16 keeps one store per row.
+template <class T>
+struct RowStore {
+  static constexpr int G = 1;
+  float x;
+  __device__ __forceinline__ void put(int, float v) { x = v; }
+  __device__ __forceinline__ void store(T *p, int, bool mine) const {
+    if (mine) p->u = (uint16_t)(__float_as_uint(x) >> 16);  // already rounded to BF16
+  }
+};
+template <>
+struct RowStore<double> {
+  static constexpr int G = 2;
+  double x[2];
+  __device__ __forceinline__ void put(int g, double v) { x[g] = v; }
+  // p: the lane's cell in the group's first row
+  __device__ __forceinline__ void store(double *p, int lane, bool mine) const {
+    typedef double d2 __attribute__((ext_vector_type(2)));
+    const bool odd = (lane & 1) != 0;
+    const double got = quad_swap1(odd ? x[0] : x[1]);
+    d2 v;
+    v.x = odd ? got : x[0];
+    v.y = odd ? x[1] : got;
+    if (mine) *reinterpret_cast<d2 *>(p + (odd ? 7 : 0)) = v;
+  }
+};
+template <>
+struct RowStore<float> {
+  static constexpr int G = 4;
+  uint32_t x[4];
+  __device__ __forceinline__ void put(int g, float v) { x[g] = __float_as_uint(v); }
+  __device__ __forceinline__ void store(float *p, int lane, bool mine) const {
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    const bool o1 = (lane & 1) != 0, o2 = (lane & 2) != 0;
+    uint32_t y[4], z[4];
+#pragma unroll
+    for (int q = 0; q < 4; q += 2) {
+      const uint32_t got = quad_swap1(o1 ? x[q] : x[q + 1]);
+      y[q] = o1 ? got : x[q];
+      y[q + 1] = o1 ? x[q + 1] : got;
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const uint32_t got = quad_swap2(o2 ? y[q] : y[q + 2]);
+      z[q] = o2 ? got : y[q];
+      z[q + 2] = o2 ? y[q + 2] : got;
+    }
+    u4 v;
+    v.x = z[0];
+    v.y = z[1];
+    v.z = z[2];
+    v.w = z[3];
+    if (mine) *reinterpret_cast<u4 *>(p + (lane & 3) * 7) = v;
+  }
+};
+
+template <class T, int TS, int J, int FORM>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(2)))
+void star_steps(const StepArgs<T> a) {
+  using A = typename acc_of<T>::type;
+  constexpr int V = 1;
+  using X = Cells<A, V>;
+  constexpr int NR = J + 2 * TS;  // rows of the input planes
+  static_assert(TS >= 1 && TS <= kHalo && TS <= J && (J == 4 || J == 8),
+                "the halo rows of a side lie in one brick");
+  const int lane = threadIdx.x & 63;
+  // each wave's older input plane, rows 1 .. NR-2, a lane its own cells
+  __shared__ X older_all[4 * (NR - 2) * 64];
+  X *older = older_all + (threadIdx.x >> 6) * ((NR - 2) * 64) + lane;
+
+  // workgroup -> (march, four strips along j, strip along i)
+  uint32_t w = xcd_remap(blockIdx.x, gridDim.x);
+  const uint32_t ch = w % a.nchunk;
+  w /= a.nchunk;
+  const uint32_t jg = (w % a.njw) * 4u + uniform(threadIdx.x >> 6);
+  const uint32_t seg = w / a.njw;
+  if (jg >= a.njg) return;  // wave-uniform; nothing below synchronises waves
+
+  // the strip along i: bricks [c0, c1); lane l the cells l V of it, the last
+  // kHalo cells of the ring those before it (lanes past the right halo hold
+  // further cells of the wrapped row, unused)
+  const uint32_t c0 = a.nb0 * ch / a.nchunk, c1 = a.nb0 * (ch + 1) / a.nchunk;
+  const uint32_t n0 = a.nb0 * 8, n1 = a.nb1 * 8, n2 = a.nb2 * 8;
+  const int off = lane * V < 64 * V - kHalo ? lane * V : (lane - 64) * V;
+  const uint32_t cell = (uint32_t)((int)(c0 * 8 + n0) + off) % n0;
+  const uint32_t bi = cell >> 3, io = cell & 7;
+  const bool mine = (uint32_t)(lane * V) < (c1 - c0) * 8;
+  // rows: the strip's in brick row bj, the halo rows below and above in brick
+  // rows bl and bh
+  const uint32_t j0 = jg * J;
+  const uint32_t jl = (j0 + n1 - 1) % n1, jh = (j0 + J) % n1;
+  const uint32_t bj = j0 >> 3, bl = jl >> 3, bh = jh >> 3;
+  // output planes [k0, k1)
+  const uint32_t k0 = (uint32_t)((uint64_t)n2 * seg / a.ksegs),
+                 k1 = (uint32_t)((uint64_t)n2 * (seg + 1) / a.ksegs);
+  const int total = (int)(k1 - k0) + 2 * TS;
+
+  // Input rows r - TS < 0 are read through pl, 0 .. J-1 through pc, J ..
+  // through ph, at + (r - TS) * 8 (the pointers move 64 cells per plane).
+  const int ol = ((int)(jl & 7) + 1) * 8 + (int)io, oc = (int)(j0 & 7) * 8 + (int)io,
+            oh = ((int)(jh & 7) - J) * 8 + (int)io;
+  auto id_of = [&](uint32_t lv, uint32_t b) { return a.ids[(lv * a.nb1 + b) * a.nb0 + bi]; };
+  const uint32_t kf = (k0 + n2 - TS) % n2;  // first input plane (n2 >= 8 > TS)
+  uint32_t lv = kf >> 3, kq = kf & 7;       // level, and the plane last loaded in it
+  const T *pl, *pc, *ph;
+  auto set_rows = [&](uint32_t il, uint32_t ic, uint32_t ih, int kofs) {
+    pl = a.in + (size_t)il * a.in_step + (ol + kofs);
+    pc = a.in + (size_t)ic * a.in_step + (oc + kofs);
+    ph = a.in + (size_t)ih * a.in_step + (oh + kofs);
+  };
+  set_rows(id_of(lv, bl), id_of(lv, bj), id_of(lv, bh), (int)kq * 64);
+  // brick ids one level ahead
+  lv = lv + 1 == a.nb2 ? 0 : lv + 1;
+  uint32_t nl = id_of(lv, bl), nc = id_of(lv, bj), nh = id_of(lv, bh);
+
+  X ea[NR], eb[NR];  // the last input plane and the one arriving
+  auto load_row = [&](int r, X(&e)[NR]) {
+    const T *p = r < TS ? pl : (r < TS + J ? pc : ph);
+    load_cells(p + (r - TS) * 8, e[r]);
+  };
+#pragma unroll
+  for (int r = 0; r < NR; ++r) load_row(r, eb);
+
+  uint32_t ko = k0;  // next output plane
+  T *po = a.out + (size_t)id_of(k0 >> 3, bj) * a.out_step + ((int)(k0 & 7) * 64 + oc);
+
+  X pa[TS][NR], pb[TS][NR];  // the two planes of sweeps 1 .. TS-1
+#pragma unroll
+  for (int r = 0; r < NR; ++r)
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+      ea[r].v[q] = A(0);
+#pragma unroll
+      for (int s = 0; s < TS; ++s) pa[s][r].v[q] = pb[s][r].v[q] = A(0);
+    }
+
+  // values as taps see them: of a kept plane, and of one just computed
+  auto tap = [](A x) -> A {
+    if constexpr (FORM == kCondRaw) return relu_ref(x);
+    else return x;
+  };
+  auto keep = [](X x) -> X {
+    if constexpr (FORM == kCondPos) {
+#pragma unroll
+      for (int q = 0; q < V; ++q) x.v[q] = relu_ref(x.v[q]);
+    }
+    return x;
+  };
+  // one sweep at one row: centre m, rows j+1 and j-1, planes k+1 and k-1
+  auto point = [&](const X &m, const X &jp, const X &jm, const X &kp, const X &km) {
+    X t, o;
+#pragma unroll
+    for (int q = 0; q < V; ++q) t.v[q] = tap(m.v[q]);
+    const A next = wave_turn<true>(t.v[0]), prev = wave_turn<false>(t.v[V - 1]);
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+      A acc = a.c[0] * t.v[q];
+      acc = fmadd(a.c[1], q + 1 < V ? t.v[q + 1 < V ? q + 1 : q] : next, acc);
+      acc = fmadd(a.c[2], q > 0 ? t.v[q > 0 ? q - 1 : 0] : prev, acc);
+      acc = fmadd(a.c[3], tap(jp.v[q]), acc);
+      acc = fmadd(a.c[4], tap(jm.v[q]), acc);
+      acc = fmadd(a.c[5], tap(kp.v[q]), acc);
+      acc = fmadd(a.c[6], tap(km.v[q]), acc);
+      if constexpr (FORM != kStar) {
+        const bool sel = a.cond_mode == 0 ? (acc > A(0)) : (m.v[q] > a.theta);
+        acc = sel ? acc : -acc;
+      }
+      o.v[q] = acc;
+    }
+    round_cells<T>(o);
+    return o;
+  };
+
+  // One input plane F (E the one before it): every row through the TS sweeps.
+  auto step = [&](X(&E)[NR], X(&F)[NR], X(&prv)[TS][NR], X(&cur)[TS][NR], int it) {
+    // the next plane's addresses (past the last one needed, still a plane of
+    // the box)
+    if (++kq == 8) {
+      kq = 0;
+      set_rows(nl, nc, nh, 0);
+      lv = lv + 1 == a.nb2 ? 0 : lv + 1;
+      nl = id_of(lv, bl);
+      nc = id_of(lv, bj);
+      nh = id_of(lv, bh);
+    } else {
+      pl += 64;
+      pc += 64;
+      ph += 64;
+    }
+    const bool emit = it >= 2 * TS, st = emit && mine;
+    // keeps the LDS plane in LDS (the compiler would carry it in registers)
+    asm volatile("" ::: "memory");
+    RowStore<T> rs;
+    X km = older[0];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      X x = F[r] = keep(F[r]);
+#pragma unroll
+      for (int s = 0; s < TS; ++s) {
+        if (r < s || r >= NR - s) continue;            // not a row of sweep s
+        const bool in = r > s && r < NR - s - 1;       // sweep s+1 has the row too
+        const int rm = r > 0 ? r - 1 : 0, rp = r + 1 < NR ? r + 1 : r;
+        X o;
+        if (s == 0) {
+          if (in) {
+            const X k0v = km;
+            if (r + 2 < NR) km = older[r * 64];  // row r+1's
+            o = point(E[r], E[rp], E[rm], x, k0v);
+          }
+          // row r-1 of E is done with: the older plane takes it, the next
+          // plane's row comes in its place
+          if (r > 1) older[(r - 2) * 64] = E[rm];
+          if (r > 0) load_row(rm, E);
+          if (r == NR - 1) load_row(r, E);
+        } else {
+          if (in) o = point(cur[s][r], cur[s][rp], cur[s][rm], x, prv[s][r]);
+          prv[s][r] = x;
+          // defined only here, after the older value's last use: the two can
+          // share a register (the compiler's own copies sit at the loop's end
+          // and doubled the registers held)
+          if (in)
+#pragma unroll
+            for (int q = 0; q < V; ++q) asm volatile("" : "+v"(prv[s][r].v[q]) : "v"(o.v[q]));
+        }
+        if (in) x = s + 1 < TS ? keep(o) : o;
+      }
+      if (r >= TS && r < TS + J) {
+        constexpr int G = RowStore<T>::G;
+        const int q = r - TS;
+        rs.put(q % G, x.v[0]);
+        if (q % G == G - 1) rs.store(po + (q - (G - 1)) * 8, lane, st);
+      }
+      __builtin_amdgcn_sched_barrier(0);  // row by row: bounds the live registers
+    }
+    if (emit) {
+      ++ko;
+      if ((ko & 7) == 0 && it + 1 < total)
+        po = a.out + (size_t)id_of(ko >> 3, bj) * a.out_step + oc;
+      else
+        po += 64;
+    }
+  };
+  for (int it = 0; it < total; it += 2) {
+    step(ea, eb, pa, pb, it);
+    if (it + 1 < total) step(eb, ea, pb, pa, it + 1);
+  }
+}
+
+// Small boxes: one workgroup per brick (BK = 8) or half brick (BK = 4 planes)
+// and pass, so that a few hundred bricks reach every CU.  The workgroup's 256
+// threads are the 16 x 16 columns of the brick's plane and its 4 halo cells a
+// side; a thread keeps its column's BK + 2 TS planes in registers.  Per sweep
+// the columns' values go to LDS, the j-taps come from there, the i-taps by DPP
+// from the 16-lane row (one row of the region), the k-taps from the thread's
+// own registers; two LDS buffers in turn, so one barrier per sweep.
+template <class T, int TS, int BK, int FORM>
+__global__ __launch_bounds__(256) void star_steps_block(const StepArgs<T> a) {
+  using A = typename acc_of<T>::type;
+  constexpr int NP = BK + 2 * TS;  // planes of the input
+  static_assert(TS >= 1 && TS <= kHalo && TS <= BK && (BK == 4 || BK == 8),
+                "the halo planes of a side lie in one level");
+  // buffer s & 1 of sweep s + 1: planes s+1 .. NP-s-2 of the field after s
+  // sweeps, from plane 1 (even s) or 2 (odd s)
+  __shared__ A lds[((NP - 2) + (NP - 4)) * 256];
+  const int t = threadIdx.x, x = t & 15, y = t >> 4;
+  uint32_t w = xcd_remap(blockIdx.x, gridDim.x);
+  const uint32_t bi = w % a.nb0;
+  w /= a.nb0;
+  const uint32_t bj = w % a.nb1;
+  const uint32_t k0 = w / a.nb1 * BK;  // first output plane
+  const uint32_t n0 = a.nb0 * 8, n1 = a.nb1 * 8, n2 = a.nb2 * 8;
+  const uint32_t ci = (bi * 8 + n0 - kHalo + x) % n0, cj = (bj * 8 + n1 - kHalo + y) % n1;
+  const uint32_t kl = (k0 + n2 - 1) % n2, kh = (k0 + BK) % n2;  // planes next to the block
+  const uint32_t row = (cj >> 3) * a.nb0 + (ci >> 3), per = a.nb0 * a.nb1;
+  const uint32_t il = a.ids[(kl >> 3) * per + row], ic = a.ids[(k0 >> 3) * per + row],
+                 ih = a.ids[(kh >> 3) * per + row];
+  const int e = (int)((cj & 7) * 8 + (ci & 7));
+  const T *pl = a.in + (size_t)il * a.in_step + (e + ((int)(kl & 7) + 1) * 64);
+  const T *pc = a.in + (size_t)ic * a.in_step + (e + (int)(k0 & 7) * 64);
+  const T *ph = a.in + (size_t)ih * a.in_step + (e + ((int)(kh & 7) - BK) * 64);
+  A c[NP];
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    const T *q = p < TS ? pl : (p < TS + BK ? pc : ph);
+    c[p] = widen(q[(p - TS) * 64]);
+  }
+  auto tap = [](A v) -> A {
+    if constexpr (FORM != kStar) return relu_ref(v);
+    else return v;
+  };
+  const int yp = (y < 15 ? t + 16 : t), ym = (y > 0 ? t - 16 : t);
+#pragma unroll
+  for (int s = 0; s < TS; ++s) {
+    A *buf = lds + (s & 1 ? (NP - 2) * 256 : 0);
+    const int p0 = (s & 1) + 1;
+#pragma unroll
+    for (int p = s + 1; p < NP - s - 1; ++p) buf[(p - p0) * 256 + t] = tap(c[p]);
+    __syncthreads();
+    A below = tap(c[s]);
+#pragma unroll
+    for (int p = s + 1; p < NP - s - 1; ++p) {
+      const A m = tap(c[p]);
+      A acc = a.c[0] * m;
+      acc = fmadd(a.c[1], row_next<true>(m), acc);
+      acc = fmadd(a.c[2], row_next<false>(m), acc);
+      acc = fmadd(a.c[3], buf[(p - p0) * 256 + yp], acc);
+      acc = fmadd(a.c[4], buf[(p - p0) * 256 + ym], acc);
+      acc = fmadd(a.c[5], tap(c[p + 1]), acc);
+      acc = fmadd(a.c[6], below, acc);
+      if constexpr (FORM != kStar) {
+        const bool sel = a.cond_mode == 0 ? (acc > A(0)) : (c[p] > a.theta);
+        acc = sel ? acc : -acc;
+      }
+      Cells<A, 1> o;
+      o.v[0] = acc;
+      round_cells<T>(o);
+      below = m;
+      c[p] = o.v[0];
+    }
+  }
+  if (x >= kHalo && x < kHalo + 8 && y >= kHalo && y < kHalo + 8) {
+    T *po = a.out + (size_t)ic * a.out_step + (e + (int)(k0 & 7) * 64);
+#pragma unroll
+    for (int p = TS; p < TS + BK; ++p) narrow(po[(p - TS) * 64], c[p]);
+  }
+}
+
+// Workgroups (four strips each) the device holds at once.
+template <class T, int TS, int J, int FORM>
+uint32_t steps_slots() {
+  static std::atomic<uint32_t> known{0};
+  uint32_t n = known.load(std::memory_order_relaxed);
+  if (n == 0) {
+    int dev = 0, cus = 256, per = 0;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        &per, reinterpret_cast<const void *>(&star_steps<T, TS, J, FORM>), 256, 0);
+    n = (uint32_t)(cus * std::max(1, per));
+    known.store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
+
+// Whether a box goes by blocks (one workgroup per brick) or by strips.  The
+// strips' long serial marches need a few thousand of them to fill the device;
+// the blocks compute 2.9 times the points a pass keeps.  Equal at (us a sweep,
+// blocks / strips): FP64 7-point 128^3 6.9 / 7.1, 160^3 12.4 / 10.4; cond
+// 160^3 16.5 / 17.6, 192^3 27.0 / 19.7; FP32 7-point 160^3 7.3 / 8.5, 192^3
+// 11.2 / 11.2; BF16 160^3 8.4 / 9.9, 192^3 12.9 / 12.8.
+bool steps_by_block(const SweepLaunch &L, const PlanView &P) {
+  const uint32_t most = L.dtype != BK_F64 ? 12000 : L.stencil == BK_COND7 ? 8000 : 5000;
+  return P.ncovered <= most;
+}
+
+bool clamped_form(const SweepLaunch &L) {
+  return L.cond_mode == BK_COND_REFERENCE || L.theta >= 0.0;
+}
+
+// Strips of four FP64 sweeps with unclamped cond planes spill (0.75 ms a
+// sweep against 0.22 with three): not built.
+template <class T, int TS, int FORM>
+constexpr bool strip_built() {
+  return !(std::is_same<T, double>::value && TS == 4 && FORM == kCondRaw);
+}
+
+template <class T, int TS, int FORM>
+hipError_t launch_steps_t(const SweepLaunch &L, const PlanView &P, hipStream_t s) {
+  using A = typename acc_of<T>::type;
+  StepArgs<T> a;
+  a.ids = P.box_ids;
+  a.in = static_cast<const T *>(L.in);
+  a.out = static_cast<T *>(L.out);
+  a.in_step = L.in_step;
+  a.out_step = L.out_step;
+  a.nb0 = P.box_nb[0];
+  a.nb1 = P.box_nb[1];
+  a.nb2 = P.box_nb[2];
+  a.cond_mode = L.cond_mode;
+  a.theta = (A)L.theta;
+  for (int q = 0; q < 7; ++q) a.c[q] = (A)L.coeff[q];
+  a.nchunk = a.njg = a.njw = a.ksegs = 0;
+  if (steps_by_block(L, P)) {
+    // half bricks while whole ones would leave half of the 256 CUs without a
+    // workgroup (64 bricks: 1.43 us a sweep against 1.58; 216: 1.72 / 1.70)
+    if (P.ncovered <= 128)
+      hipLaunchKernelGGL((star_steps_block<T, TS, 4, FORM>), dim3(P.ncovered * 2), dim3(256), 0,
+                         s, a);
+    else
+      hipLaunchKernelGGL((star_steps_block<T, TS, 8, FORM>), dim3(P.ncovered), dim3(256), 0, s,
+                         a);
+    return hipGetLastError();
+  }
+  if constexpr (!strip_built<T, TS, FORM>()) {
+    return hipErrorInvalidValue;
+  } else {
+  constexpr int J = 8;
+  const uint32_t most = (64 - 2 * kHalo) / 8;  // bricks of a strip along i
+  a.nchunk = (a.nb0 + most - 1) / most;
+  a.njg = a.nb1 * 8 / J;
+  a.njw = (a.njg + 3) / 4;
+  const uint64_t per = (uint64_t)a.nchunk * a.njw;  // workgroups of a march
+  // marches: enough to fill the device once, of at most 64 planes (shorter
+  // ones read and compute more halo planes; 512^3 FP64, TS = 4: 0.563 ms a
+  // pass with 64 planes, 0.579 with 171, 0.604 with 32) and at least 8
+  const uint64_t segs = std::max<uint64_t>(steps_slots<T, TS, J, FORM>() / per, a.nb2 / 8);
+  a.ksegs = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(segs, a.nb2));
+  const uint64_t nblk = per * a.ksegs;
+  if (nblk > 0x7fffffffull) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((star_steps<T, TS, J, FORM>), dim3((uint32_t)nblk), dim3(256), 0, s, a);
+  return hipGetLastError();
+  }
+}
+
+template <class T, int FORM>
+hipError_t launch_steps_dt(const SweepLaunch &L, const PlanView &P, int ts, hipStream_t s) {
+  switch (ts) {
+    case 3: return launch_steps_t<T, 3, FORM>(L, P, s);
+    case 4: return launch_steps_t<T, 4, FORM>(L, P, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+template <class T>
+hipError_t launch_steps_st(const SweepLaunch &L, const PlanView &P, int ts, hipStream_t s) {
+  if (L.stencil == BK_STAR7) return launch_steps_dt<T, kStar>(L, P, ts, s);
+  if (L.stencil == BK_COND7)
+    return clamped_form(L) ? launch_steps_dt<T, kCondPos>(L, P, ts, s)
+                           : launch_steps_dt<T, kCondRaw>(L, P, ts, s);
+  return hipErrorInvalidValue;
+}
+
+}  // namespace
+
+bool steps_fit(const SweepLaunch &L, const PlanView &P) {
+  if (!P.box_ids || (L.stencil != BK_STAR7 && L.stencil != BK_COND7)) return false;
+  // both fields take 16-byte stores (single ones in BF16)
+  const size_t es = L.dtype == BK_F64 ? 8 : L.dtype == BK_F32 ? 4 : 2;
+  const uintptr_t bits = reinterpret_cast<uintptr_t>(L.in) | reinterpret_cast<uintptr_t>(L.out) |
+                         (uintptr_t)(L.in_step * es) | (uintptr_t)(L.out_step * es);
+  return es == 2 || bits % 16 == 0;
+}
+
+// The cost of a pass of 1, 3 and 4 sweeps (passes of two are never needed:
+// see SweepSplit) in units of one sweep by itself, refresh included.  By
+// strips, 512^3, ms a pass: FP64 7-point 0.42 / 0.53 / 0.57, FP32 0.235 /
+// 0.318 / 0.353, BF16 0.130 / 0.310 / 0.359; cond with clamped planes FP64
+// 0.42 / 0.59 / 0.74, FP32 0.235 / 0.38 / 0.51, BF16 0.145 / 0.40 / 0.57,
+// unclamped 0.66, 0.42, 0.44 for three.  By blocks, 32^3: 3.3 us / 5.5 us.
+void steps_costs(const SweepLaunch &L, const PlanView &P, float cost[5]) {
+  static const float star[3][2] = {{1.25f, 1.35f}, {1.35f, 1.5f}, {2.4f, 2.8f}};
+  static const float pos[3][2] = {{1.4f, 1.76f}, {1.6f, 2.2f}, {2.7f, 4.0f}};
+  static const float raw[3][2] = {{1.56f, 9.0f}, {1.8f, 2.9f}, {3.1f, 5.0f}};
+  const int dt = L.dtype == BK_F64 ? 0 : L.dtype == BK_F32 ? 1 : 2;
+  const float(*t)[2] = L.stencil == BK_STAR7 ? star : clamped_form(L) ? pos : raw;
+  const bool block = steps_by_block(L, P);
+  cost[0] = 0.0f;
+  cost[1] = 1.0f;
+  cost[2] = 9.0f;
+  cost[3] = block ? 1.4f : t[dt][0];
+  cost[4] = block ? 1.6f : t[dt][1];
+}
+
+hipError_t launch_star_steps(const SweepLaunch &L, const PlanView &P, int ts, hipStream_t s) {
+  switch (L.dtype) {
+    case BK_F64: return launch_steps_st<double>(L, P, ts, s);
+    case BK_F32: return launch_steps_st<float>(L, P, ts, s);
+    case BK_BF16: return launch_steps_st<bf16>(L, P, ts, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace bk

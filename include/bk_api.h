@@ -298,6 +298,23 @@ int bk_plan_build_host(const uint32_t *h_adj, uint32_t nbricks,
                        uint32_t kcol, uint32_t *h_anchor, uint32_t *h_len,
                        uint32_t *h_mask, uint32_t *h_flat, uint32_t *nunits,
                        uint32_t *ncovered);
+/* Declare the plan's bricks a periodic box of nb[0] x nb[1] x nb[2] bricks
+ * (i, j, k; i fastest in h_ids): h_ids[(k*nb[1] + j)*nb[0] + i] is the brick
+ * at (i, j, k), h_pairs the (dst, src) ghost pairs that refresh the ghost
+ * bricks before every sweep (none where the adjacency itself wraps).
+ * Checked against h_adj, the adjacency the plan was built on: every
+ * neighbour of every box brick must be the brick of the wrapped box, or a
+ * ghost brick that a pair makes its copy -- BK_ERR_UNSUPPORTED otherwise, and
+ * the plan stays as it was.  A sequence of sweeps over such a quad plan that
+ * refreshes with these pairs (bk_sweeps, bk_sweeps_fused called with npairs
+ * pairs) may take several sweeps per pass over the field.  Both fields' box
+ * bricks then hold what single sweeps leave in them, bit for bit, and so do
+ * the ghost bricks of the input field of the last sweep (of both fields, for
+ * bk_sweeps_fused); the ghost bricks of a bk_sweeps result are not refreshed
+ * and hold older values.  No counterpart in the reference.  Allocates device
+ * memory. */
+int bk_plan_set_box(bk_plan plan, const uint32_t *h_adj, const long nb[3],
+                    const uint32_t *h_ids, const uint32_t *h_pairs, uint32_t npairs);
 int bk_plan_query(bk_plan plan, uint32_t *nunits, uint32_t *kcol, int *shape,
                   uint32_t *ncovered);
 /* Copy the plan's arrays to the host (any pointer may be NULL):
