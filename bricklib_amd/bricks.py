@@ -364,7 +364,7 @@ class Plan:
 #   0.131 / 0.145 against 0.146 / 0.158), the 25-point in blocks of 8
 #   levels (0.177-0.180 / 0.183-0.187 against one brick per wave 0.184-0.186
 #   / 0.186-0.187).
-#   cube: quads of 6 levels (kernel at 512^3: FP64 0.613 ms against 0.628
+#   cube: by size (auto_plan); at 512^3 quads of 6 levels (kernel: FP64 0.613 ms against 0.628
 #   with 4 levels, 0.646 with 2 and 0.635 with 8; FP32 0.514 against 0.520
 #   / 0.521 / 0.540).
 DEFAULT_PLANS = {
@@ -521,12 +521,19 @@ class PeriodicGrid:
         choice = DEFAULT_PLANS.get((int(stencil_kind), int(dtype)))
         if choice is None:
             return None
-        if int(stencil_kind) == _lib.BK_CUBE125 and self.interior.size > (1 << 20):
-            # large grids: 8 levels (1024^3 FP64: 4.76 ms per sweep on one
-            # host against 5.0-6.2 with 4; on most hosts every schedule lands
-            # at 5.8-6.1 ms -- 4, 5, 6, 8 and 12 levels within 1.5 % of each
-            # other on one -- and 8 levels were never the slower)
-            choice = ("quad", 8)
+        if int(stencil_kind) == _lib.BK_CUBE125:
+            # levels per unit by size: one wave marches a unit, so small grids
+            # need short units to fill the device (up to 2000 to 14000 bricks
+            # the library takes a workgroup per level).  us a sweep: FP64
+            # 160^3 1 level 30, 2 levels 37, 6 levels 91; 256^3 2 levels 98, 1
+            # level 103, 6 levels 136; 320^3 2 levels 197, 6 levels 205; 384^3
+            # 4 levels 329, 6 levels 346; FP32 256^3 84 / 86 / 137, 384^3 3
+            # levels 239, 6 levels 272.  1024^3 FP64: 4, 5, 6, 8 and 12 levels
+            # within 1.5 % on one host, 8 never the slower.
+            n = self.interior.size
+            wide = 4 if dtype == BK_F64 else 3
+            choice = ("quad", 8 if n > (1 << 20) else 6 if n > 200000 else wide if n > 80000
+                      else 2 if n > 9000 else 1)
         return self.plan(*choice)
 
     def auto_wg_bricks(self, stencil_kind: int) -> int:

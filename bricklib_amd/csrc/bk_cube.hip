@@ -614,6 +614,134 @@ __device__ __forceinline__ void cube_quad_unit_dma(
   }
 }
 
+// Block form for small and middle-sized grids: one workgroup per plan level
+// (2x2 bricks, 8 planes), its 12 padded input planes staged in LDS at once by
+// all waves, each wave computing KO of the 8 output planes from there -- no
+// march, so a level takes the time of KO + 4 windows after one load latency
+// instead of 12 dependent planes, and a grid gives 8 / KO waves per quad level
+// instead of one wave per unit.  The windows are the marching form's (2x2
+// points a lane, 6x6 cells), but every wave that needs a plane reads it again
+// (18 16-byte reads per plane: KO = 2 keeps LDS 86 % busy while it computes,
+// KO = 1 more), so past the sizes where waves are scarce the marching form is
+// the faster one.  Per point the taps go (dk, dj, di) lexicographic.
+//
+// us a sweep, block KO = 1 / KO = 2 / best marching plan / one brick a wave
+// (the six-level plans of large grids took 85 to 137 us at these sizes):
+//   FP64  64^3 7.9 / 8.6 / 18.0 / 10.1, 128^3 22.2 / 20.1 / 21.7 / 36.5,
+//         160^3 36 / 32 / 30, 256^3 138 / 121 / 98
+//   FP32  64^3 6.7 / 8.3 / 23.1 / 7.9, 128^3 15.4 / 15.6 / 27.3 / 18.1,
+//         192^3 41.3 / 40.6 / 48.4 / 52, 256^3 88.0 / 84.6 / 83.7
+//   BF16 as FP32.
+// A row stride of 20 cells (four instead of three FP64 workgroups a CU) and
+// touching the coefficients' lines ahead of the loads were no faster.
+template <class T, int KO>
+__global__ __launch_bounds__(64 * (8 / KO)) void cube_sweep_block(const CubeArgs<T> a) {
+  using A = typename acc_of<T>::type;
+  typedef A A2 __attribute__((ext_vector_type(2)));
+  static_assert(KO == 1 || KO == 2, "eight planes over whole waves");
+  constexpr int NT = 64 * (8 / KO);
+  constexpr int CPR = kQuadPW / 2, NCH = 12 * kQuadPW * CPR, NLD = (NCH + NT - 1) / NT;
+  __shared__ __attribute__((aligned(16))) A planes[12 * kQuadCells];
+  __shared__ uint32_t tbl[48];
+  const int t = threadIdx.x, lane = t & 63;
+  const uint32_t item = xcd_remap(blockIdx.x, gridDim.x);
+  const uint32_t u = item / a.kcol, l = item - u * a.kcol;
+  if (l >= a.len[u]) return;  // the whole workgroup
+  const uint32_t stored = a.mask[(size_t)u * a.kcol + l];
+  uint32_t m0 = a.anchor[u];
+  for (uint32_t q = 0; q < l; ++q) m0 = a.adj[(size_t)m0 * 27 + 22];
+  m0 = uniform(m0);
+  // The 4x4 block of columns at the level below, this one and the one above,
+  // each entry from a stored member that has it as a neighbour (the plan's
+  // check makes them agree); entries of no stored member are not needed.
+  if (t < 48) {
+    const int kd = t >> 4, r = (t >> 2) & 3, c = t & 3;
+    const uint32_t *a0 = a.adj + (size_t)m0 * 27;
+    int mj = r == 3, mi = c == 3;
+    if (!((stored >> (2 * mj + mi)) & 1u)) {
+      // the other member that reaches a middle row or column
+      if (r == 1 || r == 2) mj = 1;
+      else if (c == 1 || c == 2) mi = 1;
+    }
+    const bool ok = (stored >> (2 * mj + mi)) & 1u;
+    const uint32_t m = !ok ? m0 : (mj ? (mi ? a0[17] : a0[16]) : (mi ? a0[14] : m0));
+    tbl[t] = ok ? a.adj[(size_t)m * 27 + kd * 9 + (r - mj) * 3 + (c - mi)] : m0;
+  }
+  __syncthreads();
+  {
+    const uint32_t st32 = (uint32_t)a.in_step;
+    A2 v[NLD];
+#pragma unroll
+    for (int q = 0; q < NLD; ++q) {
+      const int ch = t + q * NT;
+      if (ch < NCH) {
+        const int p = ch / (kQuadPW * CPR), rem = ch - p * (kQuadPW * CPR);
+        const int J = rem / CPR + 6, I = (rem % CPR) * 2 + 6, K = p + 6;  // cell + 8
+        const uint32_t e = tbl[(K >> 3) * 16 + (J >> 3) * 4 + (I >> 3)] * st32 +
+                           (uint32_t)((K & 7) * 64 + (J & 7) * 8 + (I & 7));
+        const Pair<T> w = *reinterpret_cast<const Pair<T> *>(a.in + e);
+        v[q].x = widen(w.a);
+        v[q].y = widen(w.b);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < NLD; ++q) {
+      const int ch = t + q * NT;
+      if (ch < NCH) {
+        const int p = ch / (kQuadPW * CPR), rem = ch - p * (kQuadPW * CPR);
+        *reinterpret_cast<A2 *>(
+            &planes[p * kQuadCells + (rem / CPR) * kQuadStride + (rem % CPR) * 2]) = v[q];
+      }
+    }
+  }
+  __syncthreads();
+  const kconst_ptr<A> cp0 =
+      (kconst_ptr<A>)((kconst_ptr<char>)__builtin_amdgcn_kernarg_segment_ptr() +
+                      offsetof(CubeArgs<T>, c));
+  const int o0 = (int)uniform(t >> 6) * KO;
+  const int lj = lane >> 3, li = lane & 7;
+  const int xo = o0 * kQuadCells + (2 * lj) * kQuadStride + 2 * li;
+  const int mm = (lj >> 2) * 2 + (li >> 2);
+  const bool mine = (stored >> mm) & 1u;
+  T *po = a.out + (size_t)tbl[16 + ((mm >> 1) + 1) * 4 + (mm & 1) + 1] * a.out_step + o0 * 64 +
+          ((2 * lj) & 7) * 8 + ((2 * li) & 7);
+  A acc[5][2][2];
+#pragma unroll
+  for (int s = 0; s < 5; ++s)
+#pragma unroll
+    for (int pj = 0; pj < 2; ++pj)
+#pragma unroll
+      for (int pi = 0; pi < 2; ++pi) acc[s][pj][pi] = A(0);
+  // not unrolled: the windows of several planes would be read ahead and held
+#pragma unroll 1
+  for (int P = -2; P < KO + 2; ++P) {
+    A x[6][6];
+#pragma unroll
+    for (int r = 0; r < 6; ++r)
+#pragma unroll
+      for (int c = 0; c < 6; c += 2) {
+        const A2 v = *reinterpret_cast<const A2 *>(
+            &planes[xo + (P + 2) * kQuadCells + r * kQuadStride + c]);
+        x[r][c] = v.x;
+        x[r][c + 1] = v.y;
+      }
+    quad_plane_window<A>(x, cp0, P, KO, acc);
+    if (P >= 2 && mine) {  // slot 0 is complete
+      T *pp = po + (P - 2) * 64;
+      narrow(pp[0], acc[0][0][0]);
+      narrow(pp[1], acc[0][0][1]);
+      narrow(pp[8], acc[0][1][0]);
+      narrow(pp[9], acc[0][1][1]);
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int pj = 0; pj < 2; ++pj)
+#pragma unroll
+        for (int pi = 0; pi < 2; ++pi) acc[s][pj][pi] = acc[s + 1][pj][pi];
+  }
+}
+
 // FP64: 3 waves per SIMD (135 VGPRs); capping at 128 for a fourth wave
 // spills and runs slower
 template <class T>
@@ -707,6 +835,16 @@ hipError_t launch_quads_t(const SweepLaunch &L, const PlanView &P, hipStream_t s
   a.kcol = P.kcol;
   for (int q = 0; q < 125; ++q) a.c[q] = (A)L.coeff[q];
   if (P.nunits == 0) return hipSuccess;
+  // blocks while waves are scarce (the measured crossings above)
+  const uint32_t one = sizeof(T) == 8 ? 2000 : 8000, two = sizeof(T) == 8 ? 4500 : 14000;
+  const uint64_t levels = (uint64_t)P.nunits * P.kcol;
+  if (!P.march && P.ncovered <= two && levels <= 0x7fffffffull) {
+    if (P.ncovered <= one)
+      hipLaunchKernelGGL((cube_sweep_block<T, 1>), dim3((uint32_t)levels), dim3(512), 0, s, a);
+    else
+      hipLaunchKernelGGL((cube_sweep_block<T, 2>), dim3((uint32_t)levels), dim3(256), 0, s, a);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL((cube_sweep_quads<T>), dim3(P.nunits), dim3(64), 0, s, a);
   return hipGetLastError();
 }

@@ -50,8 +50,12 @@ struct PlanView {
   const uint32_t *box_ids;
   uint32_t box_nb[3];
   uint32_t box_npairs;  // ghost pairs that refresh its ghost bricks
+  bool march;           // cube: march the units at every size (plan_march)
 };
 const PlanView plan_view(const bk_plan_s *p);
+// Keep cube sweeps over the plan to the marching form, the one the batched
+// kernel runs (the tuner times it for them).
+void plan_march(bk_plan_s *p);
 
 // The quad schedule addresses its input through 32-bit element offsets:
 // brick * step + element must stay below 2^32.

@@ -49,6 +49,7 @@ struct bk_plan_s {
   uint32_t *d_box = nullptr;
   uint32_t box_nb[3] = {0, 0, 0};
   uint32_t box_npairs = 0;
+  bool march = false;  // the cube marches the units at every size
 };
 
 namespace {
@@ -73,8 +74,11 @@ const PlanView plan_view(const bk_plan_s *p) {
   v.box_ids = p->d_box;
   for (int a = 0; a < 3; ++a) v.box_nb[a] = p->box_nb[a];
   v.box_npairs = p->box_npairs;
+  v.march = p->march;
   return v;
 }
+
+void plan_march(bk_plan_s *p) { p->march = true; }
 
 }  // namespace bk
 

@@ -260,9 +260,11 @@ int bk_tune_sweep(int stencil, int dtype, const double *h_coeff, double theta, i
     candidates_of(l, stencil, flags, mine);
     std::vector<Plan> plans(mine.size());
     for (size_t q = 0; q < mine.size(); ++q)
-      if (mine[q].plan_shape)
+      if (mine[q].plan_shape) {
         BK_TRY(bk_plan_create(g.adj.data(), g.nbricks, g.list.data(), g.nlist,
                               mine[q].plan_shape, mine[q].kcol, &plans[q].p));
+        if (flags & BK_TUNE_BATCH_SCHEDULES) bk::plan_march(plans[q].p);
+      }
     d.layout = l;
     d.d_adj = static_cast<const uint32_t *>(g.d_adj.p);
     d.d_list = static_cast<const uint32_t *>(g.d_list.p);
