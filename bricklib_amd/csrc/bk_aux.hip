@@ -1,5 +1,7 @@
 // bk_aux.hip -- ghost refresh, fills, FP64 reductions and array<->brick
 // conversion kernels for gfx950.
+#include <algorithm>
+
 #include "bk_device.h"
 #include "bk_internal.h"
 
@@ -325,37 +327,71 @@ struct CopyGeom {
   int64_t nk, nj, ni;        // bricks per axis in the iteration
 };
 
+// 16 bytes of cells, aligned as the element type (array rows start anywhere).
+template <size_t ES> struct CellVec;
+template <> struct CellVec<8> { typedef u32x4 type __attribute__((aligned(8))); };
+template <> struct CellVec<4> { typedef u32x4 type __attribute__((aligned(4))); };
+template <> struct CellVec<2> { typedef u32x4 type __attribute__((aligned(2))); };
+
+// One wave moves R rows of B bricks side by side along i, 16 bytes a lane,
+// for all eight planes (eight loads in flight): a load or store covers 128 to
+// 512 contiguous bytes of every array row and 128 or 256 of every brick it
+// touches.  HBM bound, at the copy rate.  One element a lane (a brick plane a
+// wave: 64-byte pieces of eight array rows, half lines when storing to the
+// array) against this, 400x264x312, us to bricks / back: FP64 142 / 152 ->
+// 99 / 101 (rows off 16 bytes 144 / 168 -> 102 / 143), FP32 108 / 144 -> 51 /
+// 53, BF16 103 / 102 -> 25 / 24.  R = 2 storing FP64 to the array: its rows
+// may start anywhere, and longer runs leave fewer lines to two waves (off 16
+// bytes 143 against 154 with R = 4; 8-byte-aligned otherwise equal).
+constexpr int copy_rows(size_t es, bool to_brick) {
+  return es == 2 ? 8 : es == 8 && !to_brick ? 2 : 4;
+}
+
 template <class T, bool TO_BRICK>
 __global__ __launch_bounds__(256) void copy_brick(CopyGeom g, T *arr, const uint32_t *grid,
                                                   T *dat, uint64_t step) {
-  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t nbr = (uint64_t)g.nk * g.nj * g.ni;
-  if (t >= nbr * 512) return;
-  const uint64_t bi = t >> 9;
-  const int e = (int)(t & 511);
-  const int64_t ti = g.i0 + (int64_t)(bi % g.ni);
-  const int64_t tj = g.j0 + (int64_t)((bi / g.ni) % g.nj);
-  const int64_t tk = g.k0 + (int64_t)(bi / ((uint64_t)g.ni * g.nj));
-  const int k = e >> 6, j = (e >> 3) & 7, i = e & 7;
-  const size_t b = grid[ti + tj * g.sb1 + tk * g.sb2];
-  const size_t ai = (size_t)((g.pad0 + ti * 8 + i) + (g.pad1 + tj * 8 + j) * g.sa1 +
-                             (g.pad2 + tk * 8 + k) * g.sa2);
-  if constexpr (TO_BRICK) dat[b * step + e] = arr[ai];
-  else arr[ai] = dat[b * step + e];
+  typedef typename CellVec<sizeof(T)>::type Vec;
+  constexpr int CPL = 16 / (int)sizeof(T), LPR = 8 / CPL;          // cells, lanes per row
+  constexpr int R = copy_rows(sizeof(T), TO_BRICK), B = 64 / (LPR * R);  // rows, bricks of a wave
+  constexpr int NRG = 8 / R;                                       // row groups of a brick
+  const int lane = threadIdx.x & 63;
+  const uint32_t w = blockIdx.x * 4u + uniform(threadIdx.x >> 6);
+  const int64_t bi = (int64_t)(w / NRG) * B + (lane / LPR) % B;
+  if (bi >= g.ni) return;
+  const int row = (int)(w % NRG) * R + lane / (LPR * B), i = (lane % LPR) * CPL;
+  const int64_t ti = g.i0 + bi;
+  for (int64_t nk = blockIdx.z; nk < g.nk; nk += gridDim.z)
+    for (int64_t nj = blockIdx.y; nj < g.nj; nj += gridDim.y) {
+      const int64_t tj = g.j0 + nj, tk = g.k0 + nk;
+      const size_t b = grid[ti + tj * g.sb1 + tk * g.sb2];
+      T *pb = dat + b * step + row * 8 + i;
+      T *pa = arr + ((g.pad0 + ti * 8 + i) + (g.pad1 + tj * 8 + row) * g.sa1 +
+                     (g.pad2 + tk * 8) * g.sa2);
+      Vec v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        v[k] = *reinterpret_cast<const Vec *>(TO_BRICK ? pa + k * g.sa2 : pb + k * 64);
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        *reinterpret_cast<Vec *>(TO_BRICK ? pb + k * 64 : pa + k * g.sa2) = v[k];
+    }
 }
 
 template <class T>
 hipError_t launch_copy_t(int to_brick, const CopyGeom &g, void *arr, const uint32_t *grid,
                          void *dat, size_t step, hipStream_t s) {
-  const uint64_t n = (uint64_t)g.nk * g.nj * g.ni * 512;
-  if (n == 0) return hipSuccess;
-  const uint64_t nblk = (n + 255) / 256;
+  if (g.nk <= 0 || g.nj <= 0 || g.ni <= 0) return hipSuccess;
+  // waves along i: groups of 4 or 8 bricks, times the row groups (see the kernel)
+  const int64_t R = copy_rows(sizeof(T), to_brick), B = 64 / (8 * (int64_t)sizeof(T) / 16 * R), NRG = 8 / R;
+  const int64_t nx = ((g.ni + B - 1) / B * NRG + 3) / 4;
+  const dim3 blocks((uint32_t)nx, (uint32_t)std::min<int64_t>(g.nj, 65535),
+                    (uint32_t)std::min<int64_t>(g.nk, 65535));
   if (to_brick)
-    hipLaunchKernelGGL((copy_brick<T, true>), dim3((uint32_t)nblk), dim3(256), 0, s, g,
-                       static_cast<T *>(arr), grid, static_cast<T *>(dat), (uint64_t)step);
+    hipLaunchKernelGGL((copy_brick<T, true>), blocks, dim3(256), 0, s, g, static_cast<T *>(arr),
+                       grid, static_cast<T *>(dat), (uint64_t)step);
   else
-    hipLaunchKernelGGL((copy_brick<T, false>), dim3((uint32_t)nblk), dim3(256), 0, s, g,
-                       static_cast<T *>(arr), grid, static_cast<T *>(dat), (uint64_t)step);
+    hipLaunchKernelGGL((copy_brick<T, false>), blocks, dim3(256), 0, s, g, static_cast<T *>(arr),
+                       grid, static_cast<T *>(dat), (uint64_t)step);
   return hipGetLastError();
 }
 
