@@ -220,100 +220,234 @@ __global__ __launch_bounds__(256) void fill_uniform(T *__restrict__ dat, uint64_
 }
 
 // ---------------------------------------------------------------------------
-// FP64 reductions: pass 1 writes one partial per block, pass 2 combines them
-// in a fixed order (results do not depend on scheduling).
+// FP64 reductions: every block reduces its share and writes one partial per
+// value, the last block to finish combines the partials in block order
+// (results do not depend on scheduling).  A thread takes C adjacent elements
+// of four bricks at a time (16-byte loads where the element type allows, four
+// in flight); the brick of a chunk is a shift away, not a division per
+// element, and one ratio in compare's maximum needs its FP64 division only
+// when it can be a new maximum of the wave.  256 blocks of 1024 threads: the
+// last block starts from the count of blocks done, whose 1024 additions from
+// smaller blocks took 7 us.  HBM bound: 256^3, us for the statistics of an
+// FP32 field / the comparison of an FP32 with an FP64 one, 17.7 / 38 (3.8 and
+// 5.3 TB/s) against 55 / 99 for one element a thread, a 64-bit division each
+// and a second kernel.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double ld64(int dt, const void *p, size_t idx) {
-  if (dt == BK_F64) return static_cast<const double *>(p)[idx];
-  if (dt == BK_F32) return (double)static_cast<const float *>(p)[idx];
-  return (double)widen(static_cast<const bf16 *>(p)[idx]);
+constexpr int kReduceThreads = 1024;
+
+template <class T> struct Elem;
+template <> struct Elem<double> { typedef double type; };
+template <> struct Elem<float> { typedef float type; };
+template <> struct Elem<bf16> { typedef uint16_t type; };
+
+__device__ __forceinline__ double to64(double x) { return x; }
+__device__ __forceinline__ double to64(float x) { return (double)x; }
+__device__ __forceinline__ double to64(uint16_t x) {
+  return (double)__uint_as_float((uint32_t)x << 16);
 }
 
+// C adjacent elements at p (aligned as the element type)
+template <class T, int C>
+__device__ __forceinline__ void load64(const void *p, size_t at, double (&x)[C]) {
+  typedef typename Elem<T>::type E;
+  struct Chunk {
+    E v[C];
+  };
+  const Chunk t = *reinterpret_cast<const Chunk *>(static_cast<const E *>(p) + at);
+#pragma unroll
+  for (int q = 0; q < C; ++q) x[q] = to64(t.v[q]);
+}
+
+// The largest value of the wave, NaN ignored, in every lane.
+__device__ __forceinline__ double wave_max(double v) {
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) v = fmax(v, __shfl_xor(v, m));
+  return v;
+}
+
+// Sum (or maximum) of each value over the block's threads, in a fixed order,
+// to thread 0.
 template <int NV>
-__device__ void block_reduce(double (&v)[NV], const bool (&is_max)[NV], double *out) {
-  __shared__ double sh[NV][256];
-#pragma unroll
-  for (int q = 0; q < NV; ++q) sh[q][threadIdx.x] = v[q];
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) {
-#pragma unroll
-      for (int q = 0; q < NV; ++q) {
-        const double o = sh[q][threadIdx.x + s];
-        sh[q][threadIdx.x] = is_max[q] ? fmax(sh[q][threadIdx.x], o) : sh[q][threadIdx.x] + o;
-      }
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int q = 0; q < NV; ++q) out[q] = sh[q][0];
-  }
-}
-
-__global__ __launch_bounds__(256) void stats_pass1(int dt, const void *dat, uint64_t step,
-                                                   const uint32_t *list, uint32_t nlist,
-                                                   uint32_t brick_elems, double *part) {
-  double v[3] = {0.0, 0.0, 0.0};
-  const uint64_t total = (uint64_t)nlist * brick_elems;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += stride) {
-    const uint64_t l = t / brick_elems, e = t - l * brick_elems;
-    const double x = ld64(dt, dat, (size_t)list[l] * step + e);
-    v[0] += x;
-    v[1] += x * x;
-    v[2] = fmax(v[2], fabs(x));
-  }
-  const bool mx[3] = {false, false, true};
-  block_reduce<3>(v, mx, part + (size_t)blockIdx.x * 3);
-}
-
-__global__ __launch_bounds__(256) void compare_pass1(int dta, const void *a, uint64_t sa,
-                                                     int dtr, const void *r, uint64_t sr,
-                                                     const uint32_t *list, uint32_t nlist,
-                                                     uint32_t brick_elems, double floor_,
-                                                     double atol, double rtol,
-                                                     double *part) {
-  double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  const uint64_t total = (uint64_t)nlist * brick_elems;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += stride) {
-    const uint64_t l = t / brick_elems, e = t - l * brick_elems;
-    const size_t b = list[l];
-    const double xa = ld64(dta, a, b * sa + e);
-    const double xr = ld64(dtr, r, b * sr + e);
-    const double d = fabs(xa - xr);
-    const double den = fmax(fabs(xr), floor_);
-    v[0] = fmax(v[0], d);
-    v[1] = fmax(v[1], d / den);
-    v[2] += d * d;
-    v[3] += xr * xr;
-    v[4] += (d > atol + rtol * fabs(xr)) ? 1.0 : 0.0;
-  }
-  const bool mx[5] = {true, true, false, false, false};
-  block_reduce<5>(v, mx, part + (size_t)blockIdx.x * 5);
-}
-
-template <int NV>
-__global__ __launch_bounds__(256) void reduce_pass2(const double *part, int nblocks, double *out,
-                                                    int m0, int m1, int m2, int m3, int m4) {
-  double v[NV];
-  const int ms[5] = {m0, m1, m2, m3, m4};
-  bool mx[NV];
+__device__ __forceinline__ void block_reduce(double (&v)[NV], const bool (&is_max)[NV],
+                                             double (&sh)[NV][kReduceThreads / 64]) {
+  auto across = [&](int q, int m) {
+    const double o = __shfl_xor(v[q], m);
+    v[q] = is_max[q] ? fmax(v[q], o) : v[q] + o;
+  };
 #pragma unroll
   for (int q = 0; q < NV; ++q) {
-    v[q] = 0.0;
-    mx[q] = ms[q] != 0;
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) across(q, m);
+    if ((threadIdx.x & 63) == 0) sh[q][threadIdx.x >> 6] = v[q];
   }
-  for (int t = threadIdx.x; t < nblocks; t += 256) {
+  __syncthreads();
+  if (threadIdx.x < 64) {
 #pragma unroll
     for (int q = 0; q < NV; ++q) {
-      const double o = part[(size_t)t * NV + q];
-      v[q] = mx[q] ? fmax(v[q], o) : v[q] + o;
+      v[q] = sh[q][threadIdx.x % (kReduceThreads / 64)];
+#pragma unroll
+      for (int m = 1; m < kReduceThreads / 64; m <<= 1) across(q, m);
     }
   }
   __syncthreads();
-  block_reduce<NV>(v, mx, out);  // out may be part itself: every read precedes the write
+}
+
+// A block's partials to part[block][NV]; the last block combines them all into
+// out[0 .. NV).  *count holds the blocks that are done; it wraps back to 0
+// with the last one.
+template <int NV>
+__device__ __forceinline__ void finish(double (&v)[NV], const bool (&is_max)[NV], double *part,
+                                       uint32_t *count, double *out) {
+  __shared__ double sh[NV][kReduceThreads / 64];
+  __shared__ uint32_t last;
+  block_reduce<NV>(v, is_max, sh);
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int q = 0; q < NV; ++q)
+      __hip_atomic_store(&part[(size_t)blockIdx.x * NV + q], v[q], __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    // the partials, written through to memory every XCD reads, are there
+    // before the count says so (a fence would write all of L2 back)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    last = atomicInc(count, gridDim.x - 1);
+  }
+  __syncthreads();
+  if (last != gridDim.x - 1) return;
+#pragma unroll
+  for (int q = 0; q < NV; ++q) v[q] = 0.0;
+  for (uint32_t t = threadIdx.x; t < gridDim.x; t += kReduceThreads) {
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+      const double o = __hip_atomic_load(&part[(size_t)t * NV + q], __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+      v[q] = is_max[q] ? fmax(v[q], o) : v[q] + o;
+    }
+  }
+  block_reduce<NV>(v, is_max, sh);
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int q = 0; q < NV; ++q) out[q] = v[q];
+  }
+}
+
+// Calls body(bricks, chunks) for every chunk this thread owns of the listed
+// bricks' `per` chunks each, U at a time (arrays of U, or of one at the end).
+template <int U, class Body>
+__device__ __forceinline__ void walk_chunks(const uint32_t *list, uint32_t nlist, uint32_t per,
+                                            Body body) {
+  if (per <= kReduceThreads && kReduceThreads % per == 0) {
+    // several bricks a block at once, or one: no division in the loop
+    const uint32_t bpb = kReduceThreads / per, sub = threadIdx.x / per, c = threadIdx.x - sub * per;
+    const uint64_t stride = (uint64_t)gridDim.x * bpb;
+    uint64_t l = (uint64_t)blockIdx.x * bpb + sub;
+    for (; l + (U - 1) * stride < nlist; l += U * stride) {
+      uint32_t b[U], e[U];
+#pragma unroll
+      for (int q = 0; q < U; ++q) {
+        b[q] = list[l + q * stride];
+        e[q] = c;
+      }
+      body(b, e);
+    }
+    for (; l < nlist; l += stride) {
+      const uint32_t b[1] = {list[l]}, e[1] = {c};
+      body(b, e);
+    }
+  } else {
+    const uint64_t total = (uint64_t)nlist * per, stride = (uint64_t)gridDim.x * kReduceThreads;
+    for (uint64_t t = (uint64_t)blockIdx.x * kReduceThreads + threadIdx.x; t < total; t += stride) {
+      const uint64_t l = t / per;
+      const uint32_t b[1] = {list[l]}, e[1] = {(uint32_t)(t - l * per)};
+      body(b, e);
+    }
+  }
+}
+
+template <class T, int C>
+__global__ __launch_bounds__(kReduceThreads) void stats_kernel(const void *dat, uint64_t step,
+                                                    const uint32_t *list, uint32_t nlist,
+                                                    uint32_t per, double *part, uint32_t *count,
+                                                    double *out) {
+  double s0[C] = {}, s1[C] = {}, s2[C] = {};
+  walk_chunks<4>(list, nlist, per, [&](const auto &b, const auto &e) {
+    constexpr int U = sizeof(b) / sizeof(b[0]);
+    double x[U][C];
+#pragma unroll
+    for (int q = 0; q < U; ++q) load64<T, C>(dat, (size_t)b[q] * step + (size_t)e[q] * C, x[q]);
+#pragma unroll
+    for (int q = 0; q < U; ++q)
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        s0[c] += x[q][c];
+        s1[c] += x[q][c] * x[q][c];
+        s2[c] = fmax(s2[c], fabs(x[q][c]));
+      }
+  });
+  double v[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    v[0] += s0[c];
+    v[1] += s1[c];
+    v[2] = fmax(v[2], s2[c]);
+  }
+  const bool mx[3] = {false, false, true};
+  finish<3>(v, mx, part, count, out);
+}
+
+template <class TA, class TR, int C>
+__global__ __launch_bounds__(kReduceThreads) void compare_kernel(const void *a, uint64_t sa, const void *r,
+                                                      uint64_t sr, const uint32_t *list,
+                                                      uint32_t nlist, uint32_t per,
+                                                      double floor_, double atol, double rtol,
+                                                      double *part, uint32_t *count,
+                                                      double *out) {
+  double s0[C] = {}, s2[C] = {}, s3[C] = {};
+  double ratio = 0.0, top = 0.0;  // this lane's largest ratio; a bound below the wave's
+  uint64_t bad = 0;
+  walk_chunks<2>(list, nlist, per, [&](const auto &b, const auto &e) {
+    constexpr int U = sizeof(b) / sizeof(b[0]);
+    double xa[U][C], xr[U][C];
+#pragma unroll
+    for (int q = 0; q < U; ++q) {
+      load64<TA, C>(a, (size_t)b[q] * sa + (size_t)e[q] * C, xa[q]);
+      load64<TR, C>(r, (size_t)b[q] * sr + (size_t)e[q] * C, xr[q]);
+    }
+    double d[U][C], den[U][C];
+    bool more = false;
+#pragma unroll
+    for (int q = 0; q < U; ++q)
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        d[q][c] = fabs(xa[q][c] - xr[q][c]);
+        const double m = fabs(xr[q][c]);
+        den[q][c] = fmax(m, floor_);
+        s0[c] = fmax(s0[c], d[q][c]);
+        s2[c] += d[q][c] * d[q][c];
+        s3[c] += xr[q][c] * xr[q][c];
+        bad += (d[q][c] > atol + rtol * m) ? 1 : 0;
+        // d / den can exceed top only where this holds (the product's
+        // rounding is covered by the factor; a zero or underflowing product
+        // holds too)
+        more = more || d[q][c] >= top * den[q][c] * (1.0 - 0x1p-50);
+      }
+    if (__any(more)) {
+#pragma unroll
+      for (int q = 0; q < U; ++q)
+#pragma unroll
+        for (int c = 0; c < C; ++c) ratio = fmax(ratio, d[q][c] / den[q][c]);
+      // lanes out of bricks would hand on anything: then each lane its own
+      top = __ballot(1) == ~0ull ? wave_max(ratio) : ratio;
+    }
+  });
+  double v[5] = {0.0, ratio, 0.0, 0.0, (double)bad};
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    v[0] = fmax(v[0], s0[c]);
+    v[2] += s2[c];
+    v[3] += s3[c];
+  }
+  const bool mx[5] = {true, true, false, false, false};
+  finish<5>(v, mx, part, count, out);
 }
 
 // ---------------------------------------------------------------------------
@@ -518,26 +652,91 @@ hipError_t launch_fill_uniform(int layout, int dtype, void *dat, size_t step, co
   return hipGetLastError();
 }
 
-hipError_t launch_field_stats(int dtype, const void *dat, size_t step, const uint32_t *list,
-                              uint32_t nlist, size_t brick_elems, double *scratch, double *out,
-                              hipStream_t s) {
-  hipLaunchKernelGGL(stats_pass1, dim3(kReduceBlocks), dim3(256), 0, s, dtype, dat,
-                     (uint64_t)step, list, nlist, (uint32_t)brick_elems, scratch);
-  hipLaunchKernelGGL(reduce_pass2<3>, dim3(1), dim3(256), 0, s, scratch, kReduceBlocks,
-                     out ? out : scratch, 0, 0, 1, 0, 0);
+namespace {
+
+template <class T>
+hipError_t launch_stats_t(const void *dat, size_t step, const uint32_t *list, uint32_t nlist,
+                          size_t elems, double *part, uint32_t *count, double *out,
+                          hipStream_t s) {
+  constexpr int C = sizeof(T) == 8 ? 2 : sizeof(T) == 4 ? 4 : 8;  // 16 bytes
+  if (elems % C == 0)
+    hipLaunchKernelGGL((stats_kernel<T, C>), dim3(kReduceBlocks), dim3(kReduceThreads), 0, s, dat,
+                       (uint64_t)step, list, nlist, (uint32_t)(elems / C), part, count, out);
+  else
+    hipLaunchKernelGGL((stats_kernel<T, 1>), dim3(kReduceBlocks), dim3(kReduceThreads), 0, s, dat,
+                       (uint64_t)step, list, nlist, (uint32_t)elems, part, count, out);
   return hipGetLastError();
+}
+
+template <class TA, class TR>
+hipError_t launch_compare_t(const void *a, size_t sa, const void *r, size_t sr,
+                            const uint32_t *list, uint32_t nlist, size_t elems, double floor_,
+                            double atol, double rtol, double *part, uint32_t *count, double *out,
+                            hipStream_t s) {
+  // 16 bytes of the narrower type, at most four elements
+  constexpr int C = sizeof(TA) == 8 && sizeof(TR) == 8 ? 2 : 4;
+  if (elems % C == 0)
+    hipLaunchKernelGGL((compare_kernel<TA, TR, C>), dim3(kReduceBlocks), dim3(kReduceThreads), 0, s, a,
+                       (uint64_t)sa, r, (uint64_t)sr, list, nlist, (uint32_t)(elems / C), floor_,
+                       atol, rtol, part, count, out);
+  else
+    hipLaunchKernelGGL((compare_kernel<TA, TR, 1>), dim3(kReduceBlocks), dim3(kReduceThreads), 0, s, a,
+                       (uint64_t)sa, r, (uint64_t)sr, list, nlist, (uint32_t)elems, floor_, atol,
+                       rtol, part, count, out);
+  return hipGetLastError();
+}
+
+template <class TA>
+hipError_t launch_compare_a(int dtr, const void *a, size_t sa, const void *r, size_t sr,
+                            const uint32_t *list, uint32_t nlist, size_t elems, double floor_,
+                            double atol, double rtol, double *part, uint32_t *count, double *out,
+                            hipStream_t s) {
+  switch (dtr) {
+    case BK_F64:
+      return launch_compare_t<TA, double>(a, sa, r, sr, list, nlist, elems, floor_, atol, rtol,
+                                          part, count, out, s);
+    case BK_F32:
+      return launch_compare_t<TA, float>(a, sa, r, sr, list, nlist, elems, floor_, atol, rtol,
+                                         part, count, out, s);
+    case BK_BF16:
+      return launch_compare_t<TA, bf16>(a, sa, r, sr, list, nlist, elems, floor_, atol, rtol,
+                                        part, count, out, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace
+
+hipError_t launch_field_stats(int dtype, const void *dat, size_t step, const uint32_t *list,
+                              uint32_t nlist, size_t brick_elems, double *scratch,
+                              uint32_t *count, double *out, hipStream_t s) {
+  switch (dtype) {
+    case BK_F64:
+      return launch_stats_t<double>(dat, step, list, nlist, brick_elems, scratch, count, out, s);
+    case BK_F32:
+      return launch_stats_t<float>(dat, step, list, nlist, brick_elems, scratch, count, out, s);
+    case BK_BF16:
+      return launch_stats_t<bf16>(dat, step, list, nlist, brick_elems, scratch, count, out, s);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 hipError_t launch_field_compare(int dta, const void *a, size_t step_a, int dtr, const void *r,
                                 size_t step_r, const uint32_t *list, uint32_t nlist,
                                 size_t brick_elems, double floor_, double atol, double rtol,
-                                double *scratch, hipStream_t s) {
-  hipLaunchKernelGGL(compare_pass1, dim3(kReduceBlocks), dim3(256), 0, s, dta, a,
-                     (uint64_t)step_a, dtr, r, (uint64_t)step_r, list, nlist,
-                     (uint32_t)brick_elems, floor_, atol, rtol, scratch);
-  hipLaunchKernelGGL(reduce_pass2<5>, dim3(1), dim3(256), 0, s, scratch, kReduceBlocks, scratch,
-                     1, 1, 0, 0, 0);
-  return hipGetLastError();
+                                double *scratch, uint32_t *count, double *out, hipStream_t s) {
+  switch (dta) {
+    case BK_F64:
+      return launch_compare_a<double>(dtr, a, step_a, r, step_r, list, nlist, brick_elems,
+                                      floor_, atol, rtol, scratch, count, out, s);
+    case BK_F32:
+      return launch_compare_a<float>(dtr, a, step_a, r, step_r, list, nlist, brick_elems, floor_,
+                                     atol, rtol, scratch, count, out, s);
+    case BK_BF16:
+      return launch_compare_a<bf16>(dtr, a, step_a, r, step_r, list, nlist, brick_elems, floor_,
+                                    atol, rtol, scratch, count, out, s);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 hipError_t launch_copy_brick(int to_brick, int dtype, const long dims[3], const long padding[3],

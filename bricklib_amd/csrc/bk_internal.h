@@ -139,20 +139,20 @@ hipError_t launch_valu_probe(int dtype, int chains, uint32_t nblocks, uint32_t i
 hipError_t launch_fill_uniform(int layout, int dtype, void *dat, size_t step,
                                const long nb[3], int ghost, uint64_t seed,
                                double lo, double hi, hipStream_t s);
-// Deterministic two-pass FP64 reductions; `scratch` holds kReduceBlocks*nout
-// doubles (pass-1 partials).  Results land in scratch[0 .. nout), or in
-// out[0 .. nout) for launch_field_stats when `out` is not null.
-constexpr int kReduceBlocks = 1024;
+// Deterministic FP64 reductions; `scratch` holds kReduceBlocks*nout doubles
+// (the blocks' partials), *count is 0 and returns to 0.  Results land in
+// out[0 .. nout) (device memory, or pinned host memory).
+constexpr int kReduceBlocks = 256;
 hipError_t launch_field_stats(int dtype, const void *dat, size_t step,
                               const uint32_t *list, uint32_t nlist,
-                              size_t brick_elems, double *scratch, double *out,
-                              hipStream_t s);
+                              size_t brick_elems, double *scratch, uint32_t *count,
+                              double *out, hipStream_t s);
 hipError_t launch_field_compare(int dta, const void *a, size_t step_a,
                                 int dtr, const void *r, size_t step_r,
                                 const uint32_t *list, uint32_t nlist,
                                 size_t brick_elems, double floor_,
-                                double atol, double rtol, double *scratch,
-                                hipStream_t s);
+                                double atol, double rtol, double *scratch, uint32_t *count,
+                                double *out, hipStream_t s);
 hipError_t launch_copy_brick(int to_brick, int dtype, const long dims[3],
                              const long padding[3], const long ghost[3],
                              void *arr, const uint32_t *grid, void *dat,

@@ -60,42 +60,59 @@ void layout_ext(int l, int e[3]) {
 int dt_size(int dt) { return dt == BK_F64 ? 8 : dt == BK_F32 ? 4 : dt == BK_BF16 ? 2 : 0; }
 
 // Per-device FP64 reduction scratch, allocated once and guarded by a mutex;
-// the guarded section ends with a stream sync, so calls do not overlap.
+// the guarded section ends with a stream sync, so calls do not overlap.  The
+// results go straight to pinned host memory: no copy after the kernel.
+struct ReduceScratch {
+  double *part = nullptr;     // the blocks' partials
+  uint32_t *count = nullptr;  // blocks done, 0 between calls
+  double *host = nullptr;     // results, pinned
+};
 struct Scratch {
   std::mutex mu;
-  std::map<int, double *> buf;
+  std::map<int, ReduceScratch> buf;
 };
 Scratch &reduce_scratch() {
   static Scratch s;
   return s;
 }
 
-int get_scratch(double **p) {
+int get_scratch(ReduceScratch **p) {
   int dev = 0;
   BK_HIP(hipGetDevice(&dev));
   auto &sc = reduce_scratch();
   auto it = sc.buf.find(dev);
-  if (it != sc.buf.end()) {
-    *p = it->second;
-    return BK_OK;
+  if (it == sc.buf.end()) {
+    ReduceScratch r;
+    void *q = nullptr, *h = nullptr;
+    const size_t part = sizeof(double) * bk::kReduceBlocks * 5;
+    BK_HIP(hipMalloc(&q, part + 64));
+    hipError_t e = hipMemset(static_cast<char *>(q) + part, 0, 64);
+    if (e == hipSuccess) e = hipHostMalloc(&h, 8 * sizeof(double), hipHostMallocDefault);
+    if (e == hipSuccess) e = hipDeviceSynchronize();
+    if (e != hipSuccess) {
+      (void)hipFree(q);
+      (void)hipHostFree(h);
+      return hip_fail(e, "reduction scratch");
+    }
+    r.part = static_cast<double *>(q);
+    r.count = reinterpret_cast<uint32_t *>(static_cast<char *>(q) + part);
+    r.host = static_cast<double *>(h);
+    it = sc.buf.emplace(dev, r).first;
   }
-  void *q = nullptr;
-  BK_HIP(hipMalloc(&q, sizeof(double) * bk::kReduceBlocks * 8));
-  sc.buf[dev] = static_cast<double *>(q);
-  *p = static_cast<double *>(q);
+  *p = &it->second;
   return BK_OK;
 }
 
 }  // namespace
 
-// Pass-1 partials of bk_field_stats_noalloc: a file-scope device array, one
-// copy per GPU at its own address, held until the process ends (24 KiB).
-// Its size does not depend on the input: the first pass is grid-stride over
-// a fixed kReduceBlocks blocks, each writing its own three partials, and the
-// second pass reads all of them, so every slot is rewritten by every call
-// and nothing needs clearing.  Calls that overlap on one GPU share it and
-// race.
-constexpr size_t kStaticScratchDoubles = (size_t)bk::kReduceBlocks * 3;
+// Partials of bk_field_stats_noalloc: a file-scope device array, one copy per
+// GPU at its own address, held until the process ends (6 KiB).  Its size does
+// not depend on the input: a fixed kReduceBlocks blocks each write their own
+// three partials and the last one reads all of them, so every slot is
+// rewritten by every call.  Behind them the count of blocks done: 0 when the
+// library is loaded, and again after every call.  Calls that overlap on one
+// GPU share the array and race.
+constexpr size_t kStaticScratchDoubles = (size_t)bk::kReduceBlocks * 3 + 1;
 static __device__ __align__(256) double scratch[kStaticScratchDoubles];
 
 namespace {
@@ -938,20 +955,20 @@ int bk_field_stats(int dtype, const void *d_dat, size_t step, const uint32_t *d_
     return fail(BK_ERR_ARG, "bk_field_stats: brick_elems must be in [1, step]");
   auto &sc = reduce_scratch();
   std::lock_guard<std::mutex> lock(sc.mu);
-  double *buf = nullptr;
+  ReduceScratch *buf = nullptr;
   int rc = get_scratch(&buf);
   if (rc != BK_OK) return rc;
-  BK_HIP(bk::launch_field_stats(dtype, d_dat, step, d_list, nlist, brick_elems, buf, nullptr,
-                                S(s)));
-  BK_HIP(hipMemcpyAsync(h_out, buf, 3 * sizeof(double), hipMemcpyDeviceToHost, S(s)));
+  BK_HIP(bk::launch_field_stats(dtype, d_dat, step, d_list, nlist, brick_elems, buf->part,
+                                buf->count, buf->host, S(s)));
   BK_HIP(hipStreamSynchronize(S(s)));
+  std::copy(buf->host, buf->host + 3, h_out);
   return BK_OK;
 }
 
 int bk_field_stats_noalloc(int dtype, const void *d_dat, size_t step, const uint32_t *d_list,
                            uint32_t nlist, size_t brick_elems, double *d_out, bk_stream s) {
-  static_assert((size_t)bk::kReduceBlocks * 3 <= kStaticScratchDoubles,
-                "pass-1 partials exceed the static scratch array");
+  static_assert((size_t)bk::kReduceBlocks * 3 + 1 <= kStaticScratchDoubles,
+                "partials and count exceed the static scratch array");
   if (!valid_dtype(dtype))
     return fail(BK_ERR_ARG, "bk_field_stats_noalloc: unknown dtype %d", dtype);
   if (!d_out) return fail(BK_ERR_ARG, "bk_field_stats_noalloc: null output");
@@ -962,7 +979,9 @@ int bk_field_stats_noalloc(int dtype, const void *d_dat, size_t step, const uint
   double *buf = nullptr;
   int rc = static_scratch_ptr(&buf);
   if (rc != BK_OK) return rc;
-  BK_HIP(bk::launch_field_stats(dtype, d_dat, step, d_list, nlist, brick_elems, buf, d_out, S(s)));
+  BK_HIP(bk::launch_field_stats(dtype, d_dat, step, d_list, nlist, brick_elems, buf,
+                                reinterpret_cast<uint32_t *>(buf + bk::kReduceBlocks * 3), d_out,
+                                S(s)));
   return BK_OK;
 }
 
@@ -977,13 +996,14 @@ int bk_field_compare(int dtype_a, const void *d_a, size_t step_a, int dtype_r, c
     return fail(BK_ERR_ARG, "bk_field_compare: brick_elems must be in [1, step]");
   auto &sc = reduce_scratch();
   std::lock_guard<std::mutex> lock(sc.mu);
-  double *buf = nullptr;
+  ReduceScratch *buf = nullptr;
   int rc = get_scratch(&buf);
   if (rc != BK_OK) return rc;
   BK_HIP(bk::launch_field_compare(dtype_a, d_a, step_a, dtype_r, d_r, step_r, d_list, nlist,
-                                  brick_elems, floor_, atol, rtol, buf, S(s)));
-  BK_HIP(hipMemcpyAsync(h_out, buf, 5 * sizeof(double), hipMemcpyDeviceToHost, S(s)));
+                                  brick_elems, floor_, atol, rtol, buf->part, buf->count,
+                                  buf->host, S(s)));
   BK_HIP(hipStreamSynchronize(S(s)));
+  std::copy(buf->host, buf->host + 5, h_out);
   return BK_OK;
 }
 

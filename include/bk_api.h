@@ -636,8 +636,8 @@ int bk_field_stats(int dtype, const void *d_dat, size_t step,
 /* bk_field_stats without any allocation: no counterpart in the reference
  * (it has no GPU reductions); for callers that cannot allocate device memory
  * -- code under HIP graph capture, tight serving loops, harnesses that forbid
- * hipMalloc.  The same kernels and the same results as bk_field_stats, but
- * the pass-1 partials live in a static 24 KiB device array of the library
+ * hipMalloc.  The same kernel and the same results as bk_field_stats, but
+ * the blocks' partials live in a static 6 KiB device array of the library
  * (one per GPU, whatever the input size) and the three results are written
  * to device memory d_out[3], stream-ordered on s with no host wait.  Calls
  * that overlap on one GPU share that array and race: order them on one
