@@ -2,7 +2,9 @@
 //
 // A batch holds one device table per (stencil, dtype) group and one per
 // dtype for the ghost refresh.  bk_batch_set() writes the current requests
-// into those tables (pinned staging, then stream-ordered copies into HBM);
+// into those tables (pinned staging, then one stream-ordered kernel that
+// fetches the parts in use into HBM: 49 copies, most of empty tables, took
+// 0.5 ms of a batch's set, one launch 12 us);
 // bk_batch_run() launches, per tick, one persistent refresh kernel per dtype
 // and one persistent sweep kernel per group -- each serving the
 // concatenated work of all its requests -- optionally captured once into a
@@ -11,6 +13,8 @@
 // tables between runs (continuous batching).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cstddef>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -32,6 +36,36 @@ namespace {
 constexpr int kStencils = 5, kDtypes = 3, kScheds = 3, kGroups = kStencils * kDtypes * kScheds;
 static_assert(kGroups <= 64, "the non-empty groups form a 64-bit mask");
 constexpr size_t kCoeffSlot = 125;  // doubles per request in the coefficient pool
+// above the groups' bits of a sweep mask: two bits per dtype with the planes a
+// wave of the cube's block form (0: marching form), so that a captured run's
+// key tells the kernels it launches
+constexpr int kPlaneBits = kGroups;
+static_assert(kPlaneBits + 2 * kDtypes <= 64, "the cube's forms fit the mask");
+
+constexpr int cube_planes(uint64_t mask, int dtype) {
+  return (int)(mask >> (kPlaneBits + 2 * dtype)) & 3;
+}
+
+// Tables and coefficients lie at the same offsets of one pinned and one device
+// allocation.
+constexpr size_t kTableStride = (sizeof(bk::BatchTable) + 255) & ~(size_t)255;
+constexpr size_t kCoeffAt = kTableStride * (kGroups + kDtypes);
+
+// Byte ranges of the staging memory in use, in units of 16 bytes.
+constexpr int kMaxRanges = 2 * (kGroups + kDtypes) + 1;
+struct Ranges {
+  uint32_t at[kMaxRanges], len[kMaxRanges];
+};
+static_assert(offsetof(bk::BatchTable, seg) % 16 == 0 && sizeof(bk::BatchSeg) % 16 == 0,
+              "table parts are ranges of 16-byte units");
+
+// Copies range blockIdx.y from the (pinned) staging memory.
+__global__ __launch_bounds__(256) void fetch_ranges(const uint4 *__restrict__ from,
+                                                    uint4 *__restrict__ to, const Ranges r) {
+  const uint32_t at = r.at[blockIdx.y], len = r.len[blockIdx.y];
+  for (uint32_t q = blockIdx.x * 256 + threadIdx.x; q < len; q += gridDim.x * 256)
+    to[at + q] = from[at + q];
+}
 
 constexpr int group_of(int stencil, int dtype, int sched) {
   return (stencil * kDtypes + dtype) * kScheds + sched;
@@ -41,6 +75,8 @@ constexpr int group_of(int stencil, int dtype, int sched) {
 struct bk_batch_s {
   int device = 0;
   uint32_t max_reqs = 0;
+  char *d_mem = nullptr;  // the tables and the coefficient pool
+  char *h_mem = nullptr;  // their staging copy, pinned
   bk::BatchTable *d_sweep[kGroups] = {};
   bk::BatchTable *h_sweep[kGroups] = {};
   bk::BatchTable *d_ref[kDtypes] = {};
@@ -74,8 +110,6 @@ int hipfail(hipError_t e, const char *what) {
     if (e_ != hipSuccess) return hipfail(e_, #call);  \
   } while (0)
 
-size_t table_head_bytes() { return offsetof(bk::BatchTable, seg); }
-
 hipError_t enqueue_run(bk_batch_s *b, uint32_t nticks, hipStream_t s) {
   for (uint32_t t = 0; t < nticks; ++t) {
     for (int d = 0; d < kDtypes; ++d)
@@ -89,7 +123,8 @@ hipError_t enqueue_run(bk_batch_s *b, uint32_t nticks, hipStream_t s) {
         const int sched = g % kScheds;
         hipError_t e =
             stencil == BK_CUBE125
-                ? bk::launch_cube_batched(dtype, b->d_sweep[g], t, s)
+                ? bk::launch_cube_batched(dtype, cube_planes(b->sweep_mask, dtype), b->d_sweep[g],
+                                          t, s)
                 : sched == 1 ? bk::launch_star_columns_batched(stencil, dtype, b->d_sweep[g], t, s)
                 : sched == 2 ? bk::launch_star_quads_batched(stencil, dtype, b->d_sweep[g], t, s)
                              : bk::launch_star_batched(stencil, dtype, b->d_sweep[g], t, s);
@@ -106,16 +141,8 @@ extern "C" {
 int bk_batch_destroy(bk_batch b) {
   if (!b) return BK_OK;
   (void)b->graphs.clear();
-  for (int g = 0; g < kGroups; ++g) {
-    (void)hipFree(b->d_sweep[g]);
-    (void)hipHostFree(b->h_sweep[g]);
-  }
-  for (int d = 0; d < kDtypes; ++d) {
-    (void)hipFree(b->d_ref[d]);
-    (void)hipHostFree(b->h_ref[d]);
-  }
-  (void)hipFree(b->d_coeff);
-  (void)hipHostFree(b->h_coeff);
+  (void)hipFree(b->d_mem);
+  (void)hipHostFree(b->h_mem);
   if (b->staged) (void)hipEventDestroy(b->staged);
   if (b->capture) (void)hipStreamDestroy(b->capture);
   delete b;
@@ -134,35 +161,22 @@ int bk_batch_create(uint32_t max_reqs, bk_batch *out) {
     bk_batch_destroy(b);
     return rc;
   };
-  const size_t tb = sizeof(bk::BatchTable);
-  for (int g = 0; g < kGroups; ++g) {
-    if (hipMalloc(&b->d_sweep[g], tb) != hipSuccess ||
-        hipHostMalloc(&b->h_sweep[g], tb, hipHostMallocDefault) != hipSuccess)
-      return cleanup(fail(BK_ERR_NOMEM, "bk_batch_create: table allocation failed"));
+  const size_t bytes = kCoeffAt + sizeof(double) * kCoeffSlot * max_reqs + 16;
+  if (hipMalloc(&b->d_mem, bytes) != hipSuccess ||
+      hipHostMalloc(&b->h_mem, bytes, hipHostMallocDefault) != hipSuccess)
+    return cleanup(fail(BK_ERR_NOMEM, "bk_batch_create: table allocation failed"));
+  // (a table is launched over only once a set has filled it)
+  for (int g = 0; g < kGroups + kDtypes; ++g) {
+    auto *d = reinterpret_cast<bk::BatchTable *>(b->d_mem + kTableStride * g);
+    auto *h = reinterpret_cast<bk::BatchTable *>(b->h_mem + kTableStride * g);
+    (g < kGroups ? b->d_sweep[g] : b->d_ref[g - kGroups]) = d;
+    (g < kGroups ? b->h_sweep[g] : b->h_ref[g - kGroups]) = h;
   }
-  for (int d = 0; d < kDtypes; ++d) {
-    if (hipMalloc(&b->d_ref[d], tb) != hipSuccess ||
-        hipHostMalloc(&b->h_ref[d], tb, hipHostMallocDefault) != hipSuccess)
-      return cleanup(fail(BK_ERR_NOMEM, "bk_batch_create: table allocation failed"));
-  }
-  const size_t cb = sizeof(double) * kCoeffSlot * max_reqs;
-  if (hipMalloc(&b->d_coeff, cb) != hipSuccess ||
-      hipHostMalloc(&b->h_coeff, cb, hipHostMallocDefault) != hipSuccess)
-    return cleanup(fail(BK_ERR_NOMEM, "bk_batch_create: coefficient pool allocation failed"));
+  b->d_coeff = reinterpret_cast<double *>(b->d_mem + kCoeffAt);
+  b->h_coeff = reinterpret_cast<double *>(b->h_mem + kCoeffAt);
   if (hipEventCreateWithFlags(&b->staged, hipEventDisableTiming) != hipSuccess ||
       hipStreamCreateWithFlags(&b->capture, hipStreamNonBlocking) != hipSuccess)
     return cleanup(fail(BK_ERR_HIP, "bk_batch_create: event/stream creation failed"));
-  // empty tables on the device, so a run before the first set is a no-op
-  for (int g = 0; g < kGroups; ++g) std::memset(b->h_sweep[g], 0, table_head_bytes());
-  for (int d = 0; d < kDtypes; ++d) std::memset(b->h_ref[d], 0, table_head_bytes());
-  for (int g = 0; g < kGroups; ++g)
-    if (hipMemcpy(b->d_sweep[g], b->h_sweep[g], table_head_bytes(), hipMemcpyHostToDevice) !=
-        hipSuccess)
-      return cleanup(fail(BK_ERR_HIP, "bk_batch_create: table upload failed"));
-  for (int d = 0; d < kDtypes; ++d)
-    if (hipMemcpy(b->d_ref[d], b->h_ref[d], table_head_bytes(), hipMemcpyHostToDevice) !=
-        hipSuccess)
-      return cleanup(fail(BK_ERR_HIP, "bk_batch_create: table upload failed"));
   *out = b;
   return BK_OK;
 }
@@ -207,8 +221,9 @@ int bk_batch_set(bk_batch b, const bk_batch_req *reqs, uint32_t n, bk_stream str
       return fail(BK_ERR_ARG, "bk_batch_set: unknown cond mode");
   }
   uint32_t count[kGroups] = {}, rcount[kDtypes] = {};
-  for (int g = 0; g < kGroups; ++g) b->h_sweep[g]->prefix[0] = 0;
-  for (int d = 0; d < kDtypes; ++d) b->h_ref[d]->prefix[0] = 0;
+  uint64_t cube_bricks[kDtypes] = {};
+  for (int g = 0; g < kGroups; ++g) b->h_sweep[g]->prefix[0] = b->h_sweep[g]->levels = 0;
+  for (int d = 0; d < kDtypes; ++d) b->h_ref[d]->prefix[0] = b->h_ref[d]->levels = 0;
   for (uint32_t r = 0; r < n; ++r) {
     const bk_batch_req &q = reqs[r];
     const int sched = (q.stencil == BK_CUBE125 || !q.plan) ? 0
@@ -240,6 +255,8 @@ int bk_batch_set(bk_batch b, const bk_batch_req *reqs, uint32_t n, bk_stream str
       sg.mask = P.mask;
       sg.nitems = P.nunits;
       sg.kcol = P.kcol;
+      b->h_sweep[g]->levels = std::max(b->h_sweep[g]->levels, P.kcol);
+      if (q.stencil == BK_CUBE125) cube_bricks[q.dtype] += P.ncovered;
     } else {
       sg.items = q.d_list;
       sg.nitems = q.nlist;
@@ -261,27 +278,42 @@ int bk_batch_set(bk_batch b, const bk_batch_req *reqs, uint32_t n, bk_stream str
   }
   b->sweep_mask = 0;
   b->ref_mask = 0;
+  Ranges ranges;
+  uint32_t nranges = 0, longest = 0;
+  auto add = [&](size_t at, size_t bytes) {
+    const uint32_t n = (uint32_t)((bytes + 15) / 16);
+    ranges.at[nranges] = (uint32_t)(at / 16);
+    ranges.len[nranges++] = n;
+    longest = std::max(longest, n);
+  };
+  auto add_table = [&](int slot, const bk::BatchTable *t) {
+    add(kTableStride * slot, offsetof(bk::BatchTable, prefix) + 4 * ((size_t)t->nsegs + 1));
+    add(kTableStride * slot + offsetof(bk::BatchTable, seg), sizeof(bk::BatchSeg) * t->nsegs);
+  };
   for (int g = 0; g < kGroups; ++g) {
     bk::BatchTable *t = b->h_sweep[g];
     t->nsegs = count[g];
-    if (count[g] && t->prefix[count[g]]) b->sweep_mask |= 1ull << g;
-    BKB_HIP(hipMemcpyAsync(b->d_sweep[g], t, table_head_bytes(), hipMemcpyHostToDevice, s));
-    if (count[g])
-      BKB_HIP(hipMemcpyAsync(&b->d_sweep[g]->seg[0], &t->seg[0], sizeof(bk::BatchSeg) * count[g],
-                             hipMemcpyHostToDevice, s));
+    if (!count[g] || !t->prefix[count[g]]) continue;  // never launched
+    b->sweep_mask |= 1ull << g;
+    add_table(g, t);
   }
   for (int d = 0; d < kDtypes; ++d) {
     bk::BatchTable *t = b->h_ref[d];
     t->nsegs = rcount[d];
-    if (rcount[d] && t->prefix[rcount[d]]) b->ref_mask |= 1u << d;
-    BKB_HIP(hipMemcpyAsync(b->d_ref[d], t, table_head_bytes(), hipMemcpyHostToDevice, s));
-    if (rcount[d])
-      BKB_HIP(hipMemcpyAsync(&b->d_ref[d]->seg[0], &t->seg[0], sizeof(bk::BatchSeg) * rcount[d],
-                             hipMemcpyHostToDevice, s));
+    if (cube_bricks[d])
+      b->sweep_mask |= (uint64_t)bk::cube_batched_planes(d, cube_bricks[d])
+                       << (kPlaneBits + 2 * d);
+    if (!rcount[d] || !t->prefix[rcount[d]]) continue;
+    b->ref_mask |= 1u << d;
+    add_table(kGroups + d, t);
   }
-  if (n)
-    BKB_HIP(hipMemcpyAsync(b->d_coeff, b->h_coeff, sizeof(double) * kCoeffSlot * n,
-                           hipMemcpyHostToDevice, s));
+  if (n) add(kCoeffAt, sizeof(double) * kCoeffSlot * n);
+  if (nranges) {
+    hipLaunchKernelGGL(fetch_ranges, dim3((longest + 255) / 256, nranges), dim3(256), 0, s,
+                       reinterpret_cast<const uint4 *>(b->h_mem),
+                       reinterpret_cast<uint4 *>(b->d_mem), ranges);
+    BKB_HIP(hipGetLastError());
+  }
   BKB_HIP(hipEventRecord(b->staged, s));
   return BK_OK;
 }

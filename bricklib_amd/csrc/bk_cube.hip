@@ -635,110 +635,162 @@ __device__ __forceinline__ void cube_quad_unit_dma(
 // A row stride of 20 cells (four instead of three FP64 workgroups a CU) and
 // touching the coefficients' lines ahead of the loads were no faster.
 template <class T, int KO>
-__global__ __launch_bounds__(64 * (8 / KO)) void cube_sweep_block(const CubeArgs<T> a) {
+struct CubeBlock {
   using A = typename acc_of<T>::type;
-  typedef A A2 __attribute__((ext_vector_type(2)));
   static_assert(KO == 1 || KO == 2, "eight planes over whole waves");
-  constexpr int NT = 64 * (8 / KO);
-  constexpr int CPR = kQuadPW / 2, NCH = 12 * kQuadPW * CPR, NLD = (NCH + NT - 1) / NT;
-  __shared__ __attribute__((aligned(16))) A planes[12 * kQuadCells];
-  __shared__ uint32_t tbl[48];
-  const int t = threadIdx.x, lane = t & 63;
-  const uint32_t item = xcd_remap(blockIdx.x, gridDim.x);
-  const uint32_t u = item / a.kcol, l = item - u * a.kcol;
-  if (l >= a.len[u]) return;  // the whole workgroup
-  const uint32_t stored = a.mask[(size_t)u * a.kcol + l];
-  uint32_t m0 = a.anchor[u];
-  for (uint32_t q = 0; q < l; ++q) m0 = a.adj[(size_t)m0 * 27 + 22];
-  m0 = uniform(m0);
-  // The 4x4 block of columns at the level below, this one and the one above,
-  // each entry from a stored member that has it as a neighbour (the plan's
-  // check makes them agree); entries of no stored member are not needed.
-  if (t < 48) {
-    const int kd = t >> 4, r = (t >> 2) & 3, c = t & 3;
-    const uint32_t *a0 = a.adj + (size_t)m0 * 27;
-    int mj = r == 3, mi = c == 3;
-    if (!((stored >> (2 * mj + mi)) & 1u)) {
-      // the other member that reaches a middle row or column
-      if (r == 1 || r == 2) mj = 1;
-      else if (c == 1 || c == 2) mi = 1;
+  static constexpr int NT = 64 * (8 / KO);
+  struct Lds {
+    __attribute__((aligned(16))) A planes[12 * kQuadCells];
+    uint32_t tbl[48];
+  };
+
+  // one level: member m0, the members to store (bit mm)
+  static __device__ __forceinline__ void level(const uint32_t *__restrict__ adj,
+                                               const T *__restrict__ in, T *__restrict__ out,
+                                               size_t st, size_t ost, uint32_t m0,
+                                               uint32_t stored, kconst_ptr<A> cp0, Lds &lds) {
+    typedef A A2 __attribute__((ext_vector_type(2)));
+    constexpr int CPR = kQuadPW / 2, NCH = 12 * kQuadPW * CPR, NLD = (NCH + NT - 1) / NT;
+    A *planes = lds.planes;
+    uint32_t *tbl = lds.tbl;
+    const int t = threadIdx.x, lane = t & 63;
+    // The 4x4 block of columns at the level below, this one and the one above,
+    // each entry from a stored member that has it as a neighbour (the plan's
+    // check makes them agree); entries of no stored member are not needed.
+    if (t < 48) {
+      const int kd = t >> 4, r = (t >> 2) & 3, c = t & 3;
+      const uint32_t *a0 = adj + (size_t)m0 * 27;
+      int mj = r == 3, mi = c == 3;
+      if (!((stored >> (2 * mj + mi)) & 1u)) {
+        // the other member that reaches a middle row or column
+        if (r == 1 || r == 2) mj = 1;
+        else if (c == 1 || c == 2) mi = 1;
+      }
+      const bool ok = (stored >> (2 * mj + mi)) & 1u;
+      const uint32_t m = !ok ? m0 : (mj ? (mi ? a0[17] : a0[16]) : (mi ? a0[14] : m0));
+      tbl[t] = ok ? adj[(size_t)m * 27 + kd * 9 + (r - mj) * 3 + (c - mi)] : m0;
     }
-    const bool ok = (stored >> (2 * mj + mi)) & 1u;
-    const uint32_t m = !ok ? m0 : (mj ? (mi ? a0[17] : a0[16]) : (mi ? a0[14] : m0));
-    tbl[t] = ok ? a.adj[(size_t)m * 27 + kd * 9 + (r - mj) * 3 + (c - mi)] : m0;
-  }
-  __syncthreads();
-  {
-    const uint32_t st32 = (uint32_t)a.in_step;
-    A2 v[NLD];
+    __syncthreads();
+    {
+      const uint32_t st32 = (uint32_t)st;
+      A2 v[NLD];
 #pragma unroll
-    for (int q = 0; q < NLD; ++q) {
-      const int ch = t + q * NT;
-      if (ch < NCH) {
-        const int p = ch / (kQuadPW * CPR), rem = ch - p * (kQuadPW * CPR);
-        const int J = rem / CPR + 6, I = (rem % CPR) * 2 + 6, K = p + 6;  // cell + 8
-        const uint32_t e = tbl[(K >> 3) * 16 + (J >> 3) * 4 + (I >> 3)] * st32 +
-                           (uint32_t)((K & 7) * 64 + (J & 7) * 8 + (I & 7));
-        const Pair<T> w = *reinterpret_cast<const Pair<T> *>(a.in + e);
-        v[q].x = widen(w.a);
-        v[q].y = widen(w.b);
+      for (int q = 0; q < NLD; ++q) {
+        const int ch = t + q * NT;
+        if (ch < NCH) {
+          const int p = ch / (kQuadPW * CPR), rem = ch - p * (kQuadPW * CPR);
+          const int J = rem / CPR + 6, I = (rem % CPR) * 2 + 6, K = p + 6;  // cell + 8
+          const uint32_t e = tbl[(K >> 3) * 16 + (J >> 3) * 4 + (I >> 3)] * st32 +
+                             (uint32_t)((K & 7) * 64 + (J & 7) * 8 + (I & 7));
+          const Pair<T> w = *reinterpret_cast<const Pair<T> *>(in + e);
+          v[q].x = widen(w.a);
+          v[q].y = widen(w.b);
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < NLD; ++q) {
+        const int ch = t + q * NT;
+        if (ch < NCH) {
+          const int p = ch / (kQuadPW * CPR), rem = ch - p * (kQuadPW * CPR);
+          *reinterpret_cast<A2 *>(
+              &planes[p * kQuadCells + (rem / CPR) * kQuadStride + (rem % CPR) * 2]) = v[q];
+        }
       }
     }
+    __syncthreads();
+    const int o0 = (int)uniform(t >> 6) * KO;
+    const int lj = lane >> 3, li = lane & 7;
+    const int xo = o0 * kQuadCells + (2 * lj) * kQuadStride + 2 * li;
+    const int mm = (lj >> 2) * 2 + (li >> 2);
+    const bool mine = (stored >> mm) & 1u;
+    T *po = out + (size_t)tbl[16 + ((mm >> 1) + 1) * 4 + (mm & 1) + 1] * ost + o0 * 64 +
+            ((2 * lj) & 7) * 8 + ((2 * li) & 7);
+    A acc[5][2][2];
 #pragma unroll
-    for (int q = 0; q < NLD; ++q) {
-      const int ch = t + q * NT;
-      if (ch < NCH) {
-        const int p = ch / (kQuadPW * CPR), rem = ch - p * (kQuadPW * CPR);
-        *reinterpret_cast<A2 *>(
-            &planes[p * kQuadCells + (rem / CPR) * kQuadStride + (rem % CPR) * 2]) = v[q];
-      }
-    }
-  }
-  __syncthreads();
-  const kconst_ptr<A> cp0 =
-      (kconst_ptr<A>)((kconst_ptr<char>)__builtin_amdgcn_kernarg_segment_ptr() +
-                      offsetof(CubeArgs<T>, c));
-  const int o0 = (int)uniform(t >> 6) * KO;
-  const int lj = lane >> 3, li = lane & 7;
-  const int xo = o0 * kQuadCells + (2 * lj) * kQuadStride + 2 * li;
-  const int mm = (lj >> 2) * 2 + (li >> 2);
-  const bool mine = (stored >> mm) & 1u;
-  T *po = a.out + (size_t)tbl[16 + ((mm >> 1) + 1) * 4 + (mm & 1) + 1] * a.out_step + o0 * 64 +
-          ((2 * lj) & 7) * 8 + ((2 * li) & 7);
-  A acc[5][2][2];
-#pragma unroll
-  for (int s = 0; s < 5; ++s)
-#pragma unroll
-    for (int pj = 0; pj < 2; ++pj)
-#pragma unroll
-      for (int pi = 0; pi < 2; ++pi) acc[s][pj][pi] = A(0);
-  // not unrolled: the windows of several planes would be read ahead and held
-#pragma unroll 1
-  for (int P = -2; P < KO + 2; ++P) {
-    A x[6][6];
-#pragma unroll
-    for (int r = 0; r < 6; ++r)
-#pragma unroll
-      for (int c = 0; c < 6; c += 2) {
-        const A2 v = *reinterpret_cast<const A2 *>(
-            &planes[xo + (P + 2) * kQuadCells + r * kQuadStride + c]);
-        x[r][c] = v.x;
-        x[r][c + 1] = v.y;
-      }
-    quad_plane_window<A>(x, cp0, P, KO, acc);
-    if (P >= 2 && mine) {  // slot 0 is complete
-      T *pp = po + (P - 2) * 64;
-      narrow(pp[0], acc[0][0][0]);
-      narrow(pp[1], acc[0][0][1]);
-      narrow(pp[8], acc[0][1][0]);
-      narrow(pp[9], acc[0][1][1]);
-    }
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
+    for (int s = 0; s < 5; ++s)
 #pragma unroll
       for (int pj = 0; pj < 2; ++pj)
 #pragma unroll
-        for (int pi = 0; pi < 2; ++pi) acc[s][pj][pi] = acc[s + 1][pj][pi];
+        for (int pi = 0; pi < 2; ++pi) acc[s][pj][pi] = A(0);
+    // not unrolled: the windows of several planes would be read ahead and held
+#pragma unroll 1
+    for (int P = -2; P < KO + 2; ++P) {
+      A x[6][6];
+#pragma unroll
+      for (int r = 0; r < 6; ++r)
+#pragma unroll
+        for (int c = 0; c < 6; c += 2) {
+          const A2 v = *reinterpret_cast<const A2 *>(
+              &planes[xo + (P + 2) * kQuadCells + r * kQuadStride + c]);
+          x[r][c] = v.x;
+          x[r][c + 1] = v.y;
+        }
+      quad_plane_window<A>(x, cp0, P, KO, acc);
+      if (P >= 2 && mine) {  // slot 0 is complete
+        T *pp = po + (P - 2) * 64;
+        narrow(pp[0], acc[0][0][0]);
+        narrow(pp[1], acc[0][0][1]);
+        narrow(pp[8], acc[0][1][0]);
+        narrow(pp[9], acc[0][1][1]);
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int pj = 0; pj < 2; ++pj)
+#pragma unroll
+          for (int pi = 0; pi < 2; ++pi) acc[s][pj][pi] = acc[s + 1][pj][pi];
+    }
+  }
+
+  // the anchor of level l of a unit
+  static __device__ __forceinline__ uint32_t walk(const uint32_t *__restrict__ adj, uint32_t m0,
+                                                  uint32_t l) {
+    for (uint32_t q = 0; q < l; ++q) m0 = adj[(size_t)m0 * 27 + 22];
+    return uniform(m0);
+  }
+};
+
+template <class T, int KO>
+__global__ __launch_bounds__(64 * (8 / KO)) void cube_sweep_block(const CubeArgs<T> a) {
+  using A = typename acc_of<T>::type;
+  using B = CubeBlock<T, KO>;
+  __shared__ typename B::Lds lds;
+  const uint32_t item = xcd_remap(blockIdx.x, gridDim.x);
+  const uint32_t u = item / a.kcol, l = item - u * a.kcol;
+  if (l >= a.len[u]) return;  // the whole workgroup
+  const kconst_ptr<A> cp =
+      (kconst_ptr<A>)((kconst_ptr<char>)__builtin_amdgcn_kernarg_segment_ptr() +
+                      offsetof(CubeArgs<T>, c));
+  B::level(a.adj, a.in, a.out, a.in_step, a.out_step, B::walk(a.adj, a.anchor[u], l),
+           a.mask[(size_t)u * a.kcol + l], cp, lds);
+}
+
+// Batched block form, for lightly loaded groups: one persistent launch, work
+// item = one level of one unit of one request (tab->levels levels a unit, the
+// longest of the group's plans; missing ones are skipped).
+template <class T, int KO>
+__global__ __launch_bounds__(64 * (8 / KO)) void cube_block_batched(const BatchTable *tab_,
+                                                                    uint32_t tick) {
+  using A = typename acc_of<T>::type;
+  using B = CubeBlock<T, KO>;
+  __shared__ typename B::Lds lds;
+  const kconst_ptr<BatchTable> tab = (kconst_ptr<BatchTable>)tab_;
+  const uint32_t nsegs = tab->nsegs, levels = tab->levels;
+  const uint32_t total = tab->prefix[nsegs] * levels;
+  SegCursor cur;
+  for (uint32_t w = xcd_remap(blockIdx.x, gridDim.x); w < total; w += gridDim.x) {
+    const uint32_t u = w / levels, l = w - u * levels;
+    cur.seek(tab->prefix, nsegs, u);
+    const auto &sg = tab->seg[cur.s];
+    if (tick >= sg.ticks) continue;  // the same item for every wave: uniform
+    const uint32_t ul = u - cur.lo;
+    if (l >= sg.len[ul]) continue;
+    const bool odd = ((sg.parity + tick) & 1u) != 0;
+    const T *in = static_cast<const T *>(odd ? sg.f1 : sg.f0);
+    T *out = static_cast<T *>(odd ? sg.f0 : sg.f1);
+    __syncthreads();  // the last item's LDS is done with
+    B::level(sg.adj, in, out, sg.step, sg.step, B::walk(sg.adj, sg.items[ul], l),
+             sg.mask[(size_t)ul * sg.kcol + l], (kconst_ptr<A>)sg.coeff, lds);
   }
 }
 
@@ -817,6 +869,29 @@ hipError_t launch_cube_batched_t(const BatchTable *tab, uint32_t tick, hipStream
   return hipGetLastError();
 }
 
+template <class T, int KO>
+hipError_t launch_block_batched(const BatchTable *tab, uint32_t tick, hipStream_t s) {
+  static int nblk = 0;
+  if (nblk == 0) {
+    int dev = 0, cus = 256, per = 1;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        &per, reinterpret_cast<const void *>(&cube_block_batched<T, KO>), CubeBlock<T, KO>::NT, 0);
+    nblk = cus * (per > 0 ? per : 1);
+  }
+  hipLaunchKernelGGL((cube_block_batched<T, KO>), dim3(nblk), dim3(CubeBlock<T, KO>::NT), 0, s,
+                     tab, tick);
+  return hipGetLastError();
+}
+
+// Planes a wave of the block form for `bricks` bricks swept together, 0 = the
+// marching form (the measured crossings at the kernel).
+int block_planes(size_t es, uint64_t bricks) {
+  if (bricks <= (es == 8 ? 2000u : 8000u)) return 1;
+  return bricks <= (es == 8 ? 4500u : 14000u) ? 2 : 0;
+}
+
 template <class T>
 hipError_t launch_quads_t(const SweepLaunch &L, const PlanView &P, hipStream_t s) {
   using A = typename acc_of<T>::type;
@@ -835,17 +910,14 @@ hipError_t launch_quads_t(const SweepLaunch &L, const PlanView &P, hipStream_t s
   a.kcol = P.kcol;
   for (int q = 0; q < 125; ++q) a.c[q] = (A)L.coeff[q];
   if (P.nunits == 0) return hipSuccess;
-  // blocks while waves are scarce (the measured crossings above)
-  const uint32_t one = sizeof(T) == 8 ? 2000 : 8000, two = sizeof(T) == 8 ? 4500 : 14000;
   const uint64_t levels = (uint64_t)P.nunits * P.kcol;
-  if (!P.march && P.ncovered <= two && levels <= 0x7fffffffull) {
-    if (P.ncovered <= one)
-      hipLaunchKernelGGL((cube_sweep_block<T, 1>), dim3((uint32_t)levels), dim3(512), 0, s, a);
-    else
-      hipLaunchKernelGGL((cube_sweep_block<T, 2>), dim3((uint32_t)levels), dim3(256), 0, s, a);
-    return hipGetLastError();
-  }
-  hipLaunchKernelGGL((cube_sweep_quads<T>), dim3(P.nunits), dim3(64), 0, s, a);
+  const int ko = P.march || levels > 0x7fffffffull ? 0 : block_planes(sizeof(T), P.ncovered);
+  if (ko == 1)
+    hipLaunchKernelGGL((cube_sweep_block<T, 1>), dim3((uint32_t)levels), dim3(512), 0, s, a);
+  else if (ko == 2)
+    hipLaunchKernelGGL((cube_sweep_block<T, 2>), dim3((uint32_t)levels), dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((cube_sweep_quads<T>), dim3(P.nunits), dim3(64), 0, s, a);
   return hipGetLastError();
 }
 
@@ -888,11 +960,22 @@ uint32_t cube_batched_capacity(int dtype) {
   }
 }
 
-hipError_t launch_cube_batched(int dtype, const BatchTable *tab, uint32_t tick, hipStream_t s) {
-  switch (dtype) {
-    case BK_F64: return launch_cube_batched_t<double>(tab, tick, s);
-    case BK_F32: return launch_cube_batched_t<float>(tab, tick, s);
-    case BK_BF16: return launch_cube_batched_t<bf16>(tab, tick, s);
+int cube_batched_planes(int dtype, uint64_t bricks) {
+  return block_planes(dtype == BK_F64 ? 8 : 4, bricks);
+}
+
+hipError_t launch_cube_batched(int dtype, int planes, const BatchTable *tab, uint32_t tick,
+                               hipStream_t s) {
+  switch (dtype * 3 + planes) {
+    case BK_F64 * 3: return launch_cube_batched_t<double>(tab, tick, s);
+    case BK_F64 * 3 + 1: return launch_block_batched<double, 1>(tab, tick, s);
+    case BK_F64 * 3 + 2: return launch_block_batched<double, 2>(tab, tick, s);
+    case BK_F32 * 3: return launch_cube_batched_t<float>(tab, tick, s);
+    case BK_F32 * 3 + 1: return launch_block_batched<float, 1>(tab, tick, s);
+    case BK_F32 * 3 + 2: return launch_block_batched<float, 2>(tab, tick, s);
+    case BK_BF16 * 3: return launch_cube_batched_t<bf16>(tab, tick, s);
+    case BK_BF16 * 3 + 1: return launch_block_batched<bf16, 1>(tab, tick, s);
+    case BK_BF16 * 3 + 2: return launch_block_batched<bf16, 2>(tab, tick, s);
     default: return hipErrorInvalidValue;
   }
 }

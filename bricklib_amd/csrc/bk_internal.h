@@ -111,7 +111,7 @@ struct BatchSeg {
 
 struct BatchTable {
   uint32_t nsegs;
-  uint32_t pad;
+  uint32_t levels;  // levels of the longest plan (cube, block form)
   uint32_t prefix[kBatchMaxSegs + 1];  // items before segment s
   BatchSeg seg[kBatchMaxSegs];
 };
@@ -122,7 +122,11 @@ hipError_t launch_star_columns_batched(int stencil, int dtype, const BatchTable 
                                        uint32_t tick, hipStream_t s);
 hipError_t launch_star_quads_batched(int stencil, int dtype, const BatchTable *tab,
                                      uint32_t tick, hipStream_t s);
-hipError_t launch_cube_batched(int dtype, const BatchTable *tab, uint32_t tick, hipStream_t s);
+// The cube's batched form for `bricks` bricks of a group: planes a wave of the
+// block form (1 or 2), or 0 for units marched by one wave each.
+int cube_batched_planes(int dtype, uint64_t bricks);
+hipError_t launch_cube_batched(int dtype, int planes, const BatchTable *tab, uint32_t tick,
+                               hipStream_t s);
 // quad units the persistent batched cube kernel holds at once (one per wave)
 uint32_t cube_batched_capacity(int dtype);
 // quad units the persistent batched star kernel holds at once (one per workgroup)
