@@ -17,7 +17,9 @@
 #include <cstddef>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <tuple>
 #include <utility>
 
@@ -70,6 +72,12 @@ __global__ __launch_bounds__(256) void fetch_ranges(const uint4 *__restrict__ fr
 constexpr int group_of(int stencil, int dtype, int sched) {
   return (stencil * kDtypes + dtype) * kScheds + sched;
 }
+constexpr int dtype_of(int group) { return (group / kScheds) % kDtypes; }
+
+using Span = std::pair<uintptr_t, uintptr_t>;  // a field's bytes
+
+// Side streams of a run whose chains go side by side.
+constexpr int kSide = 3;
 }  // namespace
 
 struct bk_batch_s {
@@ -87,6 +95,11 @@ struct bk_batch_s {
   uint32_t ref_mask = 0;    // non-empty refresh tables
   hipEvent_t staged = nullptr;
   hipStream_t capture = nullptr;
+  hipStream_t side[kSide] = {};  // captured runs whose groups go side by side
+  hipEvent_t forked = nullptr, joined[kSide] = {};
+  std::unique_ptr<Span[]> span;  // bk_batch_set's: 2 * max_reqs
+  bool apart = false;  // the groups of the set may run side by side
+  uint64_t bricks = 0;  // of the set's requests with sweeps left
   // captured runs keyed by (tick count, sweep and refresh group masks); an
   // exec is destroyed only once its last launch has completed, so a caller
   // may queue the next run while the previous one is still on the device
@@ -110,28 +123,115 @@ int hipfail(hipError_t e, const char *what) {
     if (e_ != hipSuccess) return hipfail(e_, #call);  \
   } while (0)
 
-hipError_t enqueue_run(bk_batch_s *b, uint32_t nticks, hipStream_t s) {
-  for (uint32_t t = 0; t < nticks; ++t) {
-    for (int d = 0; d < kDtypes; ++d)
-      if (b->ref_mask >> d & 1u) {
-        hipError_t e = bk::launch_ghost_batched(d, b->d_ref[d], t, s);
-        if (e != hipSuccess) return e;
-      }
-    for (int g = 0; g < kGroups; ++g)
-      if (b->sweep_mask >> g & 1u) {
-        const int stencil = g / (kScheds * kDtypes), dtype = (g / kScheds) % kDtypes;
-        const int sched = g % kScheds;
-        hipError_t e =
-            stencil == BK_CUBE125
-                ? bk::launch_cube_batched(dtype, cube_planes(b->sweep_mask, dtype), b->d_sweep[g],
-                                          t, s)
-                : sched == 1 ? bk::launch_star_columns_batched(stencil, dtype, b->d_sweep[g], t, s)
-                : sched == 2 ? bk::launch_star_quads_batched(stencil, dtype, b->d_sweep[g], t, s)
-                             : bk::launch_star_batched(stencil, dtype, b->d_sweep[g], t, s);
-        if (e != hipSuccess) return e;
-      }
+// No two requests' fields overlap, as far as the host can tell: a field spans
+// the bricks of its plan's adjacency, or as many as its list and pairs have.
+bool fields_apart(const bk_batch_req *reqs, uint32_t n, Span *span) {
+  uint32_t m = 0;
+  for (uint32_t r = 0; r < n; ++r) {
+    const bk_batch_req &q = reqs[r];
+    uint64_t bricks = (uint64_t)q.nlist + q.npairs;
+    if (q.plan) bricks = std::max<uint64_t>(bricks, bk::plan_view(q.plan).nbricks);
+    const uintptr_t bytes = bricks * q.step * bk_dtype_size(q.dtype);
+    const uintptr_t lo = reinterpret_cast<uintptr_t>(std::min(q.d_f0, q.d_f1));
+    const uintptr_t hi = reinterpret_cast<uintptr_t>(std::max(q.d_f0, q.d_f1));
+    if (lo + bytes > hi) {  // interleaved
+      span[m++] = {lo, hi + bytes};
+    } else {
+      span[m++] = {lo, lo + bytes};
+      span[m++] = {hi, hi + bytes};
+    }
   }
-  return hipSuccess;
+  std::sort(span, span + m);
+  for (uint32_t i = 1; i < m; ++i)
+    if (span[i].first < span[i - 1].second) return false;
+  return true;
+}
+
+// Group g's sweep of tick t.
+hipError_t enqueue_group(bk_batch_s *b, int g, uint32_t t, hipStream_t s) {
+  const int stencil = g / (kScheds * kDtypes), dtype = dtype_of(g), sched = g % kScheds;
+  if (stencil == BK_CUBE125)
+    return bk::launch_cube_batched(dtype, cube_planes(b->sweep_mask, dtype), b->d_sweep[g], t, s);
+  if (sched == 1) return bk::launch_star_columns_batched(stencil, dtype, b->d_sweep[g], t, s);
+  if (sched == 2) return bk::launch_star_quads_batched(stencil, dtype, b->d_sweep[g], t, s);
+  return bk::launch_star_batched(stencil, dtype, b->d_sweep[g], t, s);
+}
+
+// Whether a captured run forks.  Each launch gains 1 us, and another per 200
+// bricks of its group and at most 10; fork and join cost 65 us, and in some
+// processes, by the queues that the runtime maps its branches to, 150.  One
+// stream / forked, in us: 10 groups of 8^3 bricks, 16 ticks 1312 / 721-727, 4
+// ticks 356 / 250-403, 1 tick 117 / 141; 8 groups of 2^3, 16 ticks 556 /
+// 471; 5 groups of 24^3, 4 ticks 1038 / 939-951.  Few launches gain less than
+// several queues take from them: 3 groups of 660 bricks, 16 ticks 419 / 565, 2
+// of 8^3 281 / 599.
+bool forks(const bk_batch_s *b, uint32_t nticks) {
+  if (!b->apart) return false;
+  const int launches = __builtin_popcountll(b->sweep_mask & ((1ull << kGroups) - 1)) +
+                       __builtin_popcount(b->ref_mask);
+  if (launches < 5) return false;
+  const double gain = 1.0 + std::min(10.0, (double)b->bricks / launches / 200.0);
+  return gain * launches * nticks > 150.0;
+}
+
+// What has to run in turn, tick by tick: a type's refresh, if it has one, and
+// sweep groups.
+struct Chain {
+  int refresh = -1;
+  uint64_t groups = 0;  // mask
+};
+
+hipError_t enqueue_chain(bk_batch_s *b, const Chain &c, uint32_t t, hipStream_t s) {
+  hipError_t e = hipSuccess;
+  if (c.refresh >= 0) e = bk::launch_ghost_batched(c.refresh, b->d_ref[c.refresh], t, s);
+  for (int g = 0; g < kGroups && e == hipSuccess; ++g)
+    if (c.groups >> g & 1u) e = enqueue_group(b, g, t, s);
+  return e;
+}
+
+// The launches of a run on stream s.  `fork`: chains that need nothing of each
+// other (a group, or all groups of a type that refreshes ghosts) take all
+// their ticks side by side, on kSide streams and s, one per hardware queue, and
+// join once at the run's end.  A launch of a small group fills a fraction of
+// the chip, and behind one another every tick pays every group's start and
+// drain: 24 mixed requests (up to 32^3 bricks, 16 ticks, 10 groups) 1882 ->
+// 1240 us side by side; with one side stream 1465 us, with seven 1831 (more
+// streams than queues).
+hipError_t enqueue_run(bk_batch_s *b, uint32_t nticks, bool fork, hipStream_t s) {
+  Chain chain[kGroups];
+  int nchains = 0;
+  for (int d = 0; d < kDtypes; ++d)
+    if (b->ref_mask >> d & 1u) chain[nchains++].refresh = d;
+  const int nref = nchains;
+  for (int g = 0; g < kGroups; ++g) {
+    if (!(b->sweep_mask >> g & 1u)) continue;
+    int c = 0;
+    while (c < nref && chain[c].refresh != dtype_of(g)) ++c;
+    if (c == nref) c = nchains++;
+    chain[c].groups |= 1ull << g;
+  }
+  hipError_t e = hipSuccess;
+  if (!fork || nchains < 2) {
+    for (uint32_t t = 0; t < nticks; ++t)
+      for (int c = 0; c < nchains && e == hipSuccess; ++c)
+        e = enqueue_chain(b, chain[c], t, s);
+    return e;
+  }
+  // chain c on side stream c, the first beyond them on s, and so on in turn
+  const int sides = std::min(nchains - 1, kSide);
+  e = hipEventRecord(b->forked, s);
+  for (int l = 0; l < sides && e == hipSuccess; ++l)
+    e = hipStreamWaitEvent(b->side[l], b->forked, 0);
+  for (int c = 0; c < nchains; ++c) {
+    const int l = c % (sides + 1);
+    for (uint32_t t = 0; t < nticks && e == hipSuccess; ++t)
+      e = enqueue_chain(b, chain[c], t, l < sides ? b->side[l] : s);
+  }
+  for (int l = 0; l < sides && e == hipSuccess; ++l) {
+    e = hipEventRecord(b->joined[l], b->side[l]);
+    if (e == hipSuccess) e = hipStreamWaitEvent(s, b->joined[l], 0);
+  }
+  return e;
 }
 
 }  // namespace
@@ -145,6 +245,11 @@ int bk_batch_destroy(bk_batch b) {
   (void)hipHostFree(b->h_mem);
   if (b->staged) (void)hipEventDestroy(b->staged);
   if (b->capture) (void)hipStreamDestroy(b->capture);
+  if (b->forked) (void)hipEventDestroy(b->forked);
+  for (int l = 0; l < kSide; ++l) {
+    if (b->side[l]) (void)hipStreamDestroy(b->side[l]);
+    if (b->joined[l]) (void)hipEventDestroy(b->joined[l]);
+  }
   delete b;
   return BK_OK;
 }
@@ -156,13 +261,14 @@ int bk_batch_create(uint32_t max_reqs, bk_batch *out) {
     return fail(BK_ERR_ARG, "bk_batch_create: max_reqs must be in [1, 2048]");
   bk_batch_s *b = new bk_batch_s();
   b->max_reqs = max_reqs;
+  b->span.reset(new (std::nothrow) Span[2 * (size_t)max_reqs]);
   (void)hipGetDevice(&b->device);
   auto cleanup = [&](int rc) {
     bk_batch_destroy(b);
     return rc;
   };
   const size_t bytes = kCoeffAt + sizeof(double) * kCoeffSlot * max_reqs + 16;
-  if (hipMalloc(&b->d_mem, bytes) != hipSuccess ||
+  if (!b->span || hipMalloc(&b->d_mem, bytes) != hipSuccess ||
       hipHostMalloc(&b->h_mem, bytes, hipHostMallocDefault) != hipSuccess)
     return cleanup(fail(BK_ERR_NOMEM, "bk_batch_create: table allocation failed"));
   // (a table is launched over only once a set has filled it)
@@ -177,6 +283,11 @@ int bk_batch_create(uint32_t max_reqs, bk_batch *out) {
   if (hipEventCreateWithFlags(&b->staged, hipEventDisableTiming) != hipSuccess ||
       hipStreamCreateWithFlags(&b->capture, hipStreamNonBlocking) != hipSuccess)
     return cleanup(fail(BK_ERR_HIP, "bk_batch_create: event/stream creation failed"));
+  bool made = hipEventCreateWithFlags(&b->forked, hipEventDisableTiming) == hipSuccess;
+  for (int l = 0; l < kSide; ++l)
+    made = made && hipStreamCreateWithFlags(&b->side[l], hipStreamNonBlocking) == hipSuccess &&
+           hipEventCreateWithFlags(&b->joined[l], hipEventDisableTiming) == hipSuccess;
+  if (!made) return cleanup(fail(BK_ERR_HIP, "bk_batch_create: event/stream creation failed"));
   *out = b;
   return BK_OK;
 }
@@ -221,7 +332,7 @@ int bk_batch_set(bk_batch b, const bk_batch_req *reqs, uint32_t n, bk_stream str
       return fail(BK_ERR_ARG, "bk_batch_set: unknown cond mode");
   }
   uint32_t count[kGroups] = {}, rcount[kDtypes] = {};
-  uint64_t cube_bricks[kDtypes] = {};
+  uint64_t cube_bricks[kDtypes] = {}, bricks = 0;
   for (int g = 0; g < kGroups; ++g) b->h_sweep[g]->prefix[0] = b->h_sweep[g]->levels = 0;
   for (int d = 0; d < kDtypes; ++d) b->h_ref[d]->prefix[0] = b->h_ref[d]->levels = 0;
   for (uint32_t r = 0; r < n; ++r) {
@@ -248,19 +359,22 @@ int bk_batch_set(bk_batch b, const bk_batch_req *reqs, uint32_t n, bk_stream str
     sg.ticks = q.ticks;
     sg.theta = q.theta;
     sg.cond_mode = q.cond_mode;
+    uint32_t nbricks = q.nlist;
     if (q.stencil == BK_CUBE125 || sched != 0) {
       const bk::PlanView P = bk::plan_view(q.plan);
+      nbricks = P.ncovered;
       sg.items = P.anchor;
       sg.len = P.len;
       sg.mask = P.mask;
       sg.nitems = P.nunits;
       sg.kcol = P.kcol;
       b->h_sweep[g]->levels = std::max(b->h_sweep[g]->levels, P.kcol);
-      if (q.stencil == BK_CUBE125) cube_bricks[q.dtype] += P.ncovered;
+      if (q.stencil == BK_CUBE125) cube_bricks[q.dtype] += nbricks;
     } else {
       sg.items = q.d_list;
       sg.nitems = q.nlist;
     }
+    if (q.ticks) bricks += nbricks;
     bk::BatchTable *t = b->h_sweep[g];
     t->seg[count[g]] = sg;
     t->prefix[count[g] + 1] = t->prefix[count[g]] + sg.nitems;
@@ -307,6 +421,8 @@ int bk_batch_set(bk_batch b, const bk_batch_req *reqs, uint32_t n, bk_stream str
     b->ref_mask |= 1u << d;
     add_table(kGroups + d, t);
   }
+  b->apart = fields_apart(reqs, n, b->span.get());
+  b->bricks = bricks;
   if (n) add(kCoeffAt, sizeof(double) * kCoeffSlot * n);
   if (nranges) {
     hipLaunchKernelGGL(fetch_ranges, dim3((longest + 255) / 256, nranges), dim3(256), 0, s,
@@ -324,13 +440,15 @@ int bk_batch_run(bk_batch b, uint32_t nticks, int use_graph, bk_stream stream) {
   hipStream_t s = static_cast<hipStream_t>(stream);
   std::lock_guard<std::mutex> lock(b->mu);
   if (!use_graph) {
-    BKB_HIP(enqueue_run(b, nticks, s));
+    BKB_HIP(enqueue_run(b, nticks, false, s));
     return BK_OK;
   }
-  const std::tuple<uint32_t, uint64_t, uint32_t> key{nticks, b->sweep_mask, b->ref_mask};
+  const bool fork = forks(b, nticks);
+  const std::tuple<uint32_t, uint64_t, uint32_t> key{
+      nticks, b->sweep_mask, b->ref_mask | (fork ? 1u << kDtypes : 0u)};
   if (!b->graphs.find(key)) {
     BKB_HIP(hipStreamBeginCapture(b->capture, hipStreamCaptureModeThreadLocal));
-    hipError_t e = enqueue_run(b, nticks, b->capture);
+    hipError_t e = enqueue_run(b, nticks, fork, b->capture);
     hipGraph_t g = nullptr;
     hipError_t e2 = hipStreamEndCapture(b->capture, &g);
     if (e != hipSuccess) {
