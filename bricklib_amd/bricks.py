@@ -323,7 +323,8 @@ class Plan:
         """Declare the plan's bricks a periodic box (bk_plan_set_box): ``ids``
         its nb[0] x nb[1] x nb[2] bricks in grid order (k slowest), ``pairs``
         the (dst, src) ghost pairs, flat.  Sequences of sweeps that refresh
-        with those pairs may then take several sweeps per pass."""
+        with those pairs then read the images themselves and may take
+        several sweeps per pass."""
         ids = np.ascontiguousarray(ids, np.uint32)
         pairs = np.ascontiguousarray(pairs, np.uint32)
         check(load().bk_plan_set_box(_vp(self.handle), info.adj.ctypes.data_as(_lib.u32p),
@@ -477,7 +478,7 @@ class PeriodicGrid:
 
     def _declare_box(self, plan) -> None:
         """Declare one of this grid's own quad plans a periodic box, once,
-        ahead of a sequence that may take several sweeps per pass."""
+        ahead of a sequence of sweeps that refresh it."""
         if plan.shape != "quad" or plan.boxed or not any(plan is p for p in self._plans.values()):
             return
         try:
@@ -701,7 +702,8 @@ def sweeps(st: Stencil, a: Brick, b: Brick, grid: PeriodicGrid, nsweeps: int,
     d = _desc(st, b, a, grid, keep, plan=plan, wg_bricks=wg_bricks, lane_shift=lane_shift)
     pairs = grid.d_pairs.ptr if (refresh and grid.d_pairs is not None) else None
     npairs = grid.npairs if refresh else 0
-    if nsweeps > 3 and keep[-1] is not None and st.kind in STEP_STENCILS and ghost_iters == 1:
+    if (nsweeps > 3 and keep[-1] is not None and ghost_iters == 1
+            and (npairs or st.kind in STEP_STENCILS)):
         grid._declare_box(keep[-1])
     if fused:
         if ghost_iters != 1:

@@ -48,6 +48,7 @@ struct PlanView {
   uint64_t id;       // unique per plan (graph-cache key), never 0
   // periodic box (bk_plan_set_box): its brick ids in grid order, or null
   const uint32_t *box_ids;
+  const uint32_t *box_adj;  // with ghost bricks: an adjacency that wraps, or null
   uint32_t box_nb[3];
   uint32_t box_npairs;  // ghost pairs that refresh its ghost bricks
   bool march;           // cube: march the units at every size (plan_march)

@@ -47,6 +47,7 @@ struct bk_plan_s {
   std::vector<bool> covered;     // [nbricks] the covered bricks
   // periodic box (bk_plan_set_box): brick ids in grid order, in HBM
   uint32_t *d_box = nullptr;
+  uint32_t *d_box_adj = nullptr;  // its wrapped adjacency, behind d_box
   uint32_t box_nb[3] = {0, 0, 0};
   uint32_t box_npairs = 0;
   bool march = false;  // the cube marches the units at every size
@@ -72,6 +73,7 @@ const PlanView plan_view(const bk_plan_s *p) {
   v.nbricks = p->nbricks;
   v.id = p->id;
   v.box_ids = p->d_box;
+  v.box_adj = p->d_box_adj;
   for (int a = 0; a < 3; ++a) v.box_nb[a] = p->box_nb[a];
   v.box_npairs = p->box_npairs;
   v.march = p->march;
@@ -174,6 +176,18 @@ bool quad_unit_consistent(const uint32_t *adj, uint32_t anchor, const uint32_t *
 }  // namespace
 
 namespace {
+
+// adj[ids[q]][e]: the wrapped box's brick next to its q-th in direction e.
+__global__ __launch_bounds__(256) void wrap_adjacency(const uint32_t *__restrict__ ids, uint32_t n,
+                                                      uint32_t nb0, uint32_t nb1, uint32_t nb2,
+                                                      uint32_t *__restrict__ adj) {
+  const uint32_t q = blockIdx.x * 256 + threadIdx.x, e = blockIdx.y;
+  if (q >= n) return;
+  const uint32_t i = q % nb0, j = q / nb0 % nb1, k = q / nb0 / nb1;
+  const uint32_t ii = (i + nb0 + e % 3 - 1) % nb0, jj = (j + nb1 + e / 3 % 3 - 1) % nb1,
+                 kk = (k + nb2 + e / 9 - 1) % nb2;
+  adj[(size_t)ids[q] * 27 + e] = ids[(kk * nb1 + jj) * nb0 + ii];
+}
 
 // A plan's arrays on the host.
 struct PlanArrays {
@@ -414,15 +428,28 @@ int bk_plan_set_box(bk_plan p, const uint32_t *h_adj, const long nb[3], const ui
           }
       }
     }
+  // a box with ghost bricks gets an adjacency without them
+  const size_t at = (n + 63) & ~(size_t)63, nadj = npairs ? (size_t)p->nbricks * 27 : 0;
   uint32_t *d = nullptr;
-  hipError_t e = hipMalloc(&d, n * sizeof(uint32_t));
+  hipError_t e = hipMalloc(&d, (at + nadj) * sizeof(uint32_t));
   if (e == hipSuccess) e = hipMemcpy(d, h_ids, n * sizeof(uint32_t), hipMemcpyHostToDevice);
+  if (e == hipSuccess && nadj) {
+    e = hipMemsetAsync(d + at, 0, nadj * sizeof(uint32_t), nullptr);  // ghost bricks' rows: unused
+    if (e == hipSuccess) {
+      hipLaunchKernelGGL(wrap_adjacency, dim3((uint32_t)((n + 255) / 256), 27), dim3(256), 0,
+                         nullptr, d, (uint32_t)n, (uint32_t)nb[0], (uint32_t)nb[1],
+                         (uint32_t)nb[2], d + at);
+      e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+  }
   if (e != hipSuccess) {
     (void)hipFree(d);
     std::string m = std::string("bk_plan_set_box: ") + hipGetErrorString(e);
     return bk::plan_fail(e == hipErrorOutOfMemory ? BK_ERR_NOMEM : BK_ERR_HIP, m.c_str());
   }
   p->d_box = d;
+  p->d_box_adj = nadj ? d + at : nullptr;
   for (int a = 0; a < 3; ++a) p->box_nb[a] = (uint32_t)nb[a];
   p->box_npairs = npairs;
   return BK_OK;

@@ -320,19 +320,25 @@ hipError_t enqueue_sweeps(const bk_sweep_desc *d, const uint32_t *pairs, uint32_
   L.img_off = img_off;
   L.img = img;
   const size_t es = (size_t)dt_size(d->dtype);
-  // Several sweeps per pass where the plan's bricks are a periodic box whose
-  // ghost bricks this sequence refreshes before every sweep: the passes read
-  // the periodic image itself, and only the last sweep, which runs by itself,
-  // reads ghost bricks.
+  // Where the plan's bricks are a periodic box whose ghost bricks this sequence
+  // refreshes before every sweep, sweeps read the periodic image itself and
+  // only the last ones touch ghost bricks: the last sweep's input has them
+  // fresh, and in the fused form its output too.  Ten sweeps, us each, with a
+  // refresh (fused) every time / now: 25-point FP32 384^3 128 (122) / 110, 13-
+  // point FP64 160^3 37.0 (25.5) / 21.6 (20.7), 125-point FP64 160^3 48.9 /
+  // 34.1, 13-point FP32 of 9x7x8 bricks 16.1 (10.7) / 7.0 (6.7).  Stencils of radius 1 take
+  // several sweeps per pass besides; the last sweep runs by itself.
   if (nsweeps > 2 && ghost_iters == 1 && d->plan && d->layout == BK_LAYOUT_8x8x8) {
     const bk::PlanView P = bk::plan_view(d->plan);
-    if (P.shape == BK_PLAN_QUAD && P.box_npairs == npairs && bk::steps_fit(L, P)) {
-      float cost[5];
-      bk::steps_costs(L, P, cost);
+    if (P.shape == BK_PLAN_QUAD && P.box_ids && P.box_npairs == npairs) {
+      const bool many = bk::steps_fit(L, P);
+      float cost[5] = {};
+      if (many) bk::steps_costs(L, P, cost);
       SweepSplit split(nsweeps - 1, cost);
       bool fwd = true, fresh = false;  // fresh: the input's ghost bricks are up to date
-      for (int ts = 1; ts; fwd = !fwd) {
-        ts = split.next();
+      for (int left = nsweeps; left; fwd = !fwd) {
+        const int ts = left == 1 || !many ? 1 : split.next();
+        left -= ts;
         L.in = fwd ? d->d_in : d->d_out;
         L.in_step = fwd ? d->in_step : d->out_step;
         L.out = fwd ? d->d_out : const_cast<void *>(d->d_in);
@@ -340,13 +346,15 @@ hipError_t enqueue_sweeps(const bk_sweep_desc *d, const uint32_t *pairs, uint32_
         hipError_t e = hipSuccess;
         if (ts > 1) {
           e = bk::launch_star_steps(L, P, ts, s);
-          fresh = false;
         } else {
-          if (npairs && !fresh)
+          if (left == 0 && npairs && !fresh)
             e = bk::launch_ghost_refresh(const_cast<void *>(L.in), L.in_step * es, 512 * es,
                                          pairs, npairs, s);
+          L.adj = left && P.box_adj ? P.box_adj : d->d_adj;
+          L.img_off = left <= 1 ? img_off : nullptr;
+          L.img = left <= 1 ? img : nullptr;
           if (e == hipSuccess) e = launch_sweep(L, d->plan, s);
-          fresh = img_off != nullptr;
+          fresh = L.img_off != nullptr;
         }
         if (e != hipSuccess) return e;
       }

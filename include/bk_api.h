@@ -307,12 +307,13 @@ int bk_plan_build_host(const uint32_t *h_adj, uint32_t nbricks,
  * ghost brick that a pair makes its copy -- BK_ERR_UNSUPPORTED otherwise, and
  * the plan stays as it was.  A sequence of sweeps over such a quad plan that
  * refreshes with these pairs (bk_sweeps, bk_sweeps_fused called with npairs
- * pairs) may take several sweeps per pass over the field.  Both fields' box
+ * pairs) then reads the periodic images themselves, refreshes only what its
+ * last sweep leaves, and may take several sweeps per pass.  Both fields' box
  * bricks then hold what single sweeps leave in them, bit for bit, and so do
  * the ghost bricks of the input field of the last sweep (of both fields, for
  * bk_sweeps_fused); the ghost bricks of a bk_sweeps result are not refreshed
  * and hold older values.  No counterpart in the reference.  Allocates device
- * memory. */
+ * memory: the ids and, with pairs, an adjacency of its own. */
 int bk_plan_set_box(bk_plan plan, const uint32_t *h_adj, const long nb[3],
                     const uint32_t *h_ids, const uint32_t *h_pairs, uint32_t npairs);
 int bk_plan_query(bk_plan plan, uint32_t *nunits, uint32_t *kcol, int *shape,
