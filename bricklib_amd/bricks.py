@@ -11,13 +11,14 @@ operation goes through the C-ABI; nothing here computes on the CPU.
 from __future__ import annotations
 
 import ctypes as C
+import struct
 from dataclasses import dataclass, field
 
 import numpy as np
 
 from . import _lib
 from ._lib import (BK_BF16, BK_F32, BK_F64, bk_sweep_desc, check, load, longs)
-from .stencils import Stencil, stencil_id
+from .stencils import NCOEFF, Stencil, stencil_id
 
 DTYPE_NP = {BK_F64: np.float64, BK_F32: np.float32, BK_BF16: np.uint16}
 DTYPE_SIZE = {BK_F64: 8, BK_F32: 4, BK_BF16: 2}
@@ -633,44 +634,48 @@ def _resolve_plan(plan, st: Stencil, grid: PeriodicGrid, dtype: int = BK_F64):
     return plan
 
 
+# bk_sweep_desc's fields in order, padded to its size
+_DESC = struct.Struct("@iiPPIPNPNPdiPiii0P")
+assert _DESC.size == C.sizeof(bk_sweep_desc)
+
+
+def _address(a: np.ndarray) -> int:
+    """The address of a contiguous array's data (a.ctypes.data takes 1 us)."""
+    if a.size and a.flags.writeable:
+        return C.addressof(C.c_char.from_buffer(a))
+    return a.ctypes.data
+
+
 def _desc(st: Stencil, out: Brick, inp: Brick, grid: PeriodicGrid, coeff_keep: list,
           blist: DeviceBuffer | None = None, nlist: int | None = None,
           plan=None, wg_bricks=None, lane_shift=None) -> bk_sweep_desc:
     if out.dtype != inp.dtype:
         raise ValueError("input and output fields must share a dtype")
+    kind, dtype = st.kind, inp.dtype
     coeff = np.ascontiguousarray(st.coeff, dtype=np.float64)
-    if coeff.size != _lib.load().bk_stencil_ncoeff(st.kind):
-        raise ValueError(f"stencil {st.kind} takes {_lib.load().bk_stencil_ncoeff(st.kind)} "
+    if coeff.size != NCOEFF.get(kind, 0):
+        raise ValueError(f"stencil {kind} takes {NCOEFF.get(kind, 0)} "
                          f"coefficients, got {coeff.size}")
     coeff_keep.append(coeff)
-    d = bk_sweep_desc()
-    d.stencil = st.kind
-    d.dtype = inp.dtype
-    d.d_adj = grid.info.dptr
-    d.d_list = (blist or grid.d_sweep_list).ptr
-    d.nlist = grid.interior.size if nlist is None else nlist
-    d.d_in = inp.ptr
-    d.in_step = inp.step
-    d.d_out = out.ptr
-    d.out_step = out.step
-    d.h_coeff = coeff.ctypes.data_as(_lib.dblp)
-    d.theta = float(st.theta)
-    d.cond_mode = int(st.cond_mode)
-    pl = _resolve_plan(plan, st, grid, inp.dtype)
-    d.plan = pl.handle if pl is not None else None
+    pl = _resolve_plan(plan, st, grid, dtype)
     coeff_keep.append(pl)
-    d.layout = getattr(grid, "brick_layout", 0)
     if wg_bricks is None:
-        wg_bricks = (grid.auto_wg_bricks(st.kind)
+        wg_bricks = (grid.auto_wg_bricks(kind)
                      if plan == "auto" and hasattr(grid, "auto_wg_bricks") else 0)
-    d.wg_bricks = 0 if pl is not None else int(wg_bricks)
     if lane_shift is None:
         # automatic: only where the kernels have it (quad plans of the stars)
-        quad_star = pl is not None and pl.shape == "quad" and st.kind != _lib.BK_CUBE125
-        lane_shift = (grid.auto_lane_shift(st.kind, inp.dtype)
+        quad_star = pl is not None and pl.shape == "quad" and kind != _lib.BK_CUBE125
+        lane_shift = (grid.auto_lane_shift(kind, dtype)
                       if quad_star and hasattr(grid, "auto_lane_shift") else 0)
-    d.lane_shift = int(lane_shift)
-    return d
+    # packed at once: field by field, with numpy's data_as for the
+    # coefficients, the record took 4.0 us of a small sweep's 7.4, now 2.3 of
+    # 6.0
+    return bk_sweep_desc.from_buffer_copy(_DESC.pack(
+        kind, dtype, grid.info.dptr, (blist or grid.d_sweep_list).ptr or 0,
+        grid.interior.size if nlist is None else nlist, inp.ptr or 0, inp.step, out.ptr or 0,
+        out.step, _address(coeff), float(st.theta), int(st.cond_mode),
+        pl.handle or 0 if pl is not None else 0, getattr(grid, "brick_layout", 0),
+        0 if pl is not None else int(wg_bricks), int(lane_shift)))
 
 
 def sweep(st: Stencil, out: Brick, inp: Brick, grid: PeriodicGrid, stream=None,
@@ -682,7 +687,7 @@ def sweep(st: Stencil, out: Brick, inp: Brick, grid: PeriodicGrid, stream=None,
     DPP lane shifts in the quad star kernels (None: tuned or default)."""
     keep: list = []
     d = _desc(st, out, inp, grid, keep, plan=plan, wg_bricks=wg_bricks, lane_shift=lane_shift)
-    check(load().bk_sweep(C.byref(d), _vp(_stream_of(stream))))
+    check(load().bk_sweep(C.byref(d), _stream_of(stream)))
 
 
 def sweeps(st: Stencil, a: Brick, b: Brick, grid: PeriodicGrid, nsweeps: int,
