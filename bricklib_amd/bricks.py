@@ -379,7 +379,7 @@ DEFAULT_PLANS = {
     (3, BK_F64): ("quad", 6), (3, BK_F32): ("quad", 6), (3, BK_BF16): ("quad", 6),
 }
 # Stencils whose sequences may take several sweeps per pass (bk_plan_set_box).
-STEP_STENCILS = (_lib.BK_STAR7, _lib.BK_COND7)
+STEP_STENCILS = (_lib.BK_STAR7, _lib.BK_COND7, _lib.BK_STAR13)
 # lane_shift of the quad star kernels per (stencil, dtype); absent = 0 (the
 # i-taps from the LDS tile).
 DEFAULT_LANE_SHIFT: dict = {}

@@ -1,5 +1,5 @@
-// bk_steps.hip -- several sweeps of a radius-1 stencil (7-point star, cond)
-// per pass over the field, for periodic boxes of 8x8x8 bricks on gfx950.
+// bk_steps.hip -- several sweeps of a short-armed stencil (7- and 13-point star,
+// cond) per pass over the field, for periodic boxes of 8x8x8 bricks on gfx950.
 //
 // bk_sweeps runs a loop of sweeps (weak/main.hip.cpp:274-279) whose every
 // step reads and writes the whole field: past the caches' size each sweep
@@ -7,14 +7,13 @@
 // one pass reads the field once, applies TS sweeps in registers and writes
 // the result; the sweeps in between never reach memory.
 //
-// One wave owns a strip of J rows (j) of up to 7 bricks (V = 1; 15 for V = 2)
-// along i and marches along k.  Lane l holds V adjacent cells of every row.
-// The 64 V cells of a row are the strip's and kHalo halo cells a side, laid
-// round the wave as a ring -- strip first, right halo, left halo -- so the
-// i-taps are one-lane wave rotations (DPP) and groups of lanes fall on whole
-// brick rows.  For each sweep s of the pass the wave keeps two planes of the
-// field after s sweeps in registers (rows s .. NR-s-1 of the NR = J + 2 TS
-// input rows).  When a new input plane arrives, each row goes through all TS
+// One wave owns a strip of J rows (j) of up to 7 bricks along i and marches
+// along k.  Lane l holds one cell of every row (V = 1).  The 64 cells of a row
+// are the strip's and kHalo halo cells a side, laid round the wave as a ring --
+// strip first, right halo, left halo -- so the i-taps are one-lane wave
+// rotations (DPP) and groups of lanes fall on whole brick rows.  For each sweep
+// s of the pass the wave keeps two planes of the field after s sweeps in
+// registers (rows s .. NR-s-1 of the NR = J + 2 TS input rows).  When a new input plane arrives, each row goes through all TS
 // sweeps at once:
 //   n_{s+1}[r] = stencil of plane s around row r: centre row and rows r +- 1
 //                from the newer kept plane, k+1 from n_s[r] just computed,
@@ -42,7 +41,6 @@
 // first five taps of the next row among the last ones of this row, two rows
 // per scheduling group, or loads two planes ahead no faster.
 #include <algorithm>
-#include <atomic>
 #include <type_traits>
 
 #include "bk_device.h"
@@ -58,7 +56,8 @@ constexpr int kHalo = 4;  // halo cells at either end of a row (TS <= 4)
 // planes save the clamps of four taps in five; the select of the reference
 // form needs no kept value, and with a threshold theta >= 0 a value exceeds
 // theta exactly where its clamped one does.
-enum Form { kStar = 0, kCondRaw = 1, kCondPos = 2 };
+enum Form { kStar = 0, kCondRaw = 1, kCondPos = 2, kStar13 = 3 };
+constexpr int radius_of(int form) { return form == kStar13 ? 2 : 1; }
 
 template <class T>
 struct StepArgs {
@@ -75,7 +74,7 @@ struct StepArgs {
   uint32_t ksegs;          // marches along k
   int cond_mode;
   A theta;
-  A c[7];
+  A c[13];
 };
 
 // V adjacent cells of a lane
@@ -100,19 +99,19 @@ __device__ __forceinline__ double wave_turn(double x) {
   return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
-// The value of the next (UP) or previous lane of a 16-lane row.
-template <bool UP>
+// The value of the lane D above (UP) or below in its row of 16.
+template <bool UP, int D>
 __device__ __forceinline__ uint32_t row_next32(uint32_t x) {
-  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, UP ? 0x101 : 0x111, 0xf, 0xf, true);
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, (UP ? 0x100 : 0x110) + D, 0xf, 0xf, true);
 }
-template <bool UP>
+template <bool UP, int D>
 __device__ __forceinline__ float row_next(float x) {
-  return __builtin_bit_cast(float, row_next32<UP>(__builtin_bit_cast(uint32_t, x)));
+  return __builtin_bit_cast(float, row_next32<UP, D>(__builtin_bit_cast(uint32_t, x)));
 }
-template <bool UP>
+template <bool UP, int D>
 __device__ __forceinline__ double row_next(double x) {
   const uint64_t u = __builtin_bit_cast(uint64_t, x);
-  const uint32_t lo = row_next32<UP>((uint32_t)u), hi = row_next32<UP>((uint32_t)(u >> 32));
+  const uint32_t lo = row_next32<UP, D>((uint32_t)u), hi = row_next32<UP, D>((uint32_t)(u >> 32));
   return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
@@ -406,6 +405,177 @@ void star_steps(const StepArgs<T> a) {
   }
 }
 
+// The 13-point star (radius 2), two sweeps per pass: the same strips, halos and
+// marches, so eight input planes for a first output.  A wave keeps in registers
+// three planes of the input (the centre, the one above and the one arriving)
+// and three of the field after one sweep; of both, what lies below the centre
+// that still is needed is in LDS (two planes and one, each lane its own cells).
+// The planes change roles from step to step, with a period of three.  Bound by
+// memory and VALU about equally (210 registers in FP64: two waves per SIMD; 120
+// in FP32).  us a sweep, one by one / so: FP64 256^3 60 / 39, 384^3 188 / 121,
+// 512^3 434 / 289; FP32 256^3 36 / 27, 384^3 102 / 72, 512^3 228 / 167.  With E's
+// rows loaded again wherever the scheduler liked, each row took two registers:
+// 67 of FP64's spilled.
+template <class T>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(2)))
+void star13_steps(const StepArgs<T> a) {
+  using A = typename acc_of<T>::type;
+  constexpr int R = 2, J = 8, H = 2 * R;
+  constexpr int NR = J + 2 * H;   // rows of the input planes
+  constexpr int N1 = J + 2 * R;   // rows after one sweep: R .. NR-R-1
+  static_assert(H <= kHalo, "the halo cells of a row");
+  const int lane = threadIdx.x & 63;
+  __shared__ A older_all[4 * (2 * N1 + J) * 64];
+  A *older = older_all + (threadIdx.x >> 6) * ((2 * N1 + J) * 64) + lane;
+  A *older1 = older + 2 * N1 * 64;  // after one sweep, two planes below the centre
+  int o1 = 0, o2 = N1 * 64;         // the input, one and two planes below
+
+  // as in star_steps
+  uint32_t w = xcd_remap(blockIdx.x, gridDim.x);
+  const uint32_t ch = w % a.nchunk;
+  w /= a.nchunk;
+  const uint32_t jg = (w % a.njw) * 4u + uniform(threadIdx.x >> 6);
+  const uint32_t seg = w / a.njw;
+  if (jg >= a.njg) return;  // wave-uniform; nothing below synchronises waves
+  const uint32_t c0 = a.nb0 * ch / a.nchunk, c1 = a.nb0 * (ch + 1) / a.nchunk;
+  const uint32_t n0 = a.nb0 * 8, n1 = a.nb1 * 8, n2 = a.nb2 * 8;
+  const int off = lane < 64 - kHalo ? lane : lane - 64;
+  const uint32_t cell = (uint32_t)((int)(c0 * 8 + n0) + off) % n0;
+  const uint32_t bi = cell >> 3, io = cell & 7;
+  const bool mine = (uint32_t)lane < (c1 - c0) * 8;
+  const uint32_t j0 = jg * J;
+  const uint32_t jl = (j0 + n1 - 1) % n1, jh = (j0 + J) % n1;
+  const uint32_t bj = j0 >> 3, bl = jl >> 3, bh = jh >> 3;
+  const uint32_t k0 = (uint32_t)((uint64_t)n2 * seg / a.ksegs),
+                 k1 = (uint32_t)((uint64_t)n2 * (seg + 1) / a.ksegs);
+  const int total = (int)(k1 - k0) + 2 * H;
+  const int ol = ((int)(jl & 7) + 1) * 8 + (int)io, oc = (int)(j0 & 7) * 8 + (int)io,
+            oh = ((int)(jh & 7) - J) * 8 + (int)io;
+  auto id_of = [&](uint32_t lv, uint32_t b) { return a.ids[(lv * a.nb1 + b) * a.nb0 + bi]; };
+  const uint32_t kf = (k0 + n2 - H) % n2;
+  uint32_t lv = kf >> 3, kq = kf & 7;
+  const T *pl, *pc, *ph;
+  auto set_rows = [&](uint32_t il, uint32_t ic, uint32_t ih, int kofs) {
+    pl = a.in + (size_t)il * a.in_step + (ol + kofs);
+    pc = a.in + (size_t)ic * a.in_step + (oc + kofs);
+    ph = a.in + (size_t)ih * a.in_step + (oh + kofs);
+  };
+  set_rows(id_of(lv, bl), id_of(lv, bj), id_of(lv, bh), (int)kq * 64);
+  lv = lv + 1 == a.nb2 ? 0 : lv + 1;
+  uint32_t nl = id_of(lv, bl), nc = id_of(lv, bj), nh = id_of(lv, bh);
+
+  A e0[NR], e1[NR], e2[NR];  // planes of the input
+  A m0[NR], m1[NR], m2[NR];  // planes of the field after one sweep
+  auto load_row = [&](int r, A(&e)[NR]) {
+    const T *p = r < H ? pl : (r < H + J ? pc : ph);
+    e[r] = widen(p[(r - H) * 8]);
+  };
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    e0[r] = e1[r] = m0[r] = m1[r] = m2[r] = A(0);
+    load_row(r, e2);
+  }
+  uint32_t ko = k0;  // next output plane
+  T *po = a.out + (size_t)id_of(k0 >> 3, bj) * a.out_step + ((int)(k0 & 7) * 64 + oc);
+
+  // one sweep at row r of plane e; planes k + 1, k + 2, k - 1, k - 2
+  auto point = [&](const A(&e)[NR], int r, A kp1, A kp2, A km1, A km2) {
+    const A t = e[r];
+    const A n1 = wave_turn<true>(t), p1 = wave_turn<false>(t);
+    A acc = a.c[0] * t;
+    acc = fmadd(a.c[1], n1, acc);
+    acc = fmadd(a.c[2], p1, acc);
+    acc = fmadd(a.c[3], e[r + 1], acc);
+    acc = fmadd(a.c[4], e[r - 1], acc);
+    acc = fmadd(a.c[5], kp1, acc);
+    acc = fmadd(a.c[6], km1, acc);
+    acc = fmadd(a.c[7], wave_turn<true>(n1), acc);
+    acc = fmadd(a.c[8], wave_turn<false>(p1), acc);
+    acc = fmadd(a.c[9], e[r + 2], acc);
+    acc = fmadd(a.c[10], e[r - 2], acc);
+    acc = fmadd(a.c[11], kp2, acc);
+    return fmadd(a.c[12], km2, acc);
+  };
+  // one input plane F arrived, P the one before it, E the centre of the first
+  // sweep; of the second, p the plane above the centre c and m the one below
+  auto step = [&](A(&E)[NR], A(&P)[NR], A(&F)[NR], A(&c)[NR], A(&p)[NR], A(&m)[NR], int it) {
+    if (++kq == 8) {
+      kq = 0;
+      set_rows(nl, nc, nh, 0);
+      lv = lv + 1 == a.nb2 ? 0 : lv + 1;
+      nl = id_of(lv, bl);
+      nc = id_of(lv, bj);
+      nh = id_of(lv, bh);
+    } else {
+      pl += 64;
+      pc += 64;
+      ph += 64;
+    }
+    const bool emit = it >= 2 * H, st = emit && mine;
+    asm volatile("" ::: "memory");  // keeps the LDS planes in LDS
+    RowStore<T> rs;
+    A km1 = older[o1], km2 = older[o2], kn2 = older1[0];
+    // row q of E is done with: it takes the place of the plane two below, the
+    // next plane's row comes in its place
+    auto release = [&](int q) {
+      if (q >= R && q < NR - R) older[o2 + (q - R) * 64] = E[q];
+      load_row(q, E);
+    };
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      if (r >= R && r < NR - R) {
+        const A a1 = km1, a2 = km2;
+        if (r + 1 < NR - R) {
+          km1 = older[o1 + (r + 1 - R) * 64];
+          km2 = older[o2 + (r + 1 - R) * 64];
+        }
+        A x = point(E, r, P[r], F[r], a1, a2);
+        // loaded again only after x: the old and the new row share a register
+        asm volatile("" : "+v"(E[r - R]) : "v"(x));
+        release(r - R);
+        if (r >= H && r < NR - H) {
+          const A b2 = kn2;
+          if (r + 1 < NR - H) kn2 = older1[(r + 1 - H) * 64];
+          A y = point(c, r, p[r], x, m[r], b2);
+          older1[(r - H) * 64] = m[r];
+          constexpr int G = RowStore<T>::G;
+          const int q = r - H;
+          rs.put(q % G, y);
+          m[r] = x;
+          asm volatile("" : "+v"(m[r]) : "v"(y));
+          if (q % G == G - 1) rs.store(po + (q - (G - 1)) * 8, lane, st);
+        } else {
+          m[r] = x;
+        }
+      } else if (r >= NR - R) {
+        release(r - R);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    release(NR - 2);
+    release(NR - 1);
+    const int o = o1;
+    o1 = o2;
+    o2 = o;
+    if (emit) {
+      ++ko;
+      if ((ko & 7) == 0 && it + 1 < total)
+        po = a.out + (size_t)id_of(ko >> 3, bj) * a.out_step + oc;
+      else
+        po += 64;
+    }
+  };
+  for (int it = 0;; it += 3) {
+    step(e0, e1, e2, m0, m1, m2, it);
+    if (it + 1 >= total) break;
+    step(e1, e2, e0, m1, m2, m0, it + 1);
+    if (it + 2 >= total) break;
+    step(e2, e0, e1, m2, m0, m1, it + 2);
+    if (it + 3 >= total) break;
+  }
+}
+
 // Small boxes: one workgroup per brick (BK = 8) or half brick (BK = 4 planes)
 // and pass, so that a few hundred bricks reach every CU.  The workgroup's 256
 // threads are the 16 x 16 columns of the brick's plane and its 4 halo cells a
@@ -416,12 +586,13 @@ void star_steps(const StepArgs<T> a) {
 template <class T, int TS, int BK, int FORM>
 __global__ __launch_bounds__(256) void star_steps_block(const StepArgs<T> a) {
   using A = typename acc_of<T>::type;
-  constexpr int NP = BK + 2 * TS;  // planes of the input
-  static_assert(TS >= 1 && TS <= kHalo && TS <= BK && (BK == 4 || BK == 8),
+  constexpr int R = radius_of(FORM), H = TS * R;  // radius, halo planes a side
+  constexpr int NP = BK + 2 * H;                  // planes of the input
+  static_assert(TS >= 1 && H <= kHalo && H <= BK && (BK == 4 || BK == 8),
                 "the halo planes of a side lie in one level");
-  // buffer s & 1 of sweep s + 1: planes s+1 .. NP-s-2 of the field after s
-  // sweeps, from plane 1 (even s) or 2 (odd s)
-  __shared__ A lds[((NP - 2) + (NP - 4)) * 256];
+  // buffer s & 1 of sweep s + 1: planes (s+1) R .. NP-(s+1)R-1 of the field
+  // after s sweeps, from plane R (even s) or 2 R (odd s)
+  __shared__ A lds[((NP - 2 * R) + (NP - 4 * R)) * 256];
   const int t = threadIdx.x, x = t & 15, y = t >> 4;
   uint32_t w = xcd_remap(blockIdx.x, gridDim.x);
   const uint32_t bi = w % a.nb0;
@@ -441,86 +612,201 @@ __global__ __launch_bounds__(256) void star_steps_block(const StepArgs<T> a) {
   A c[NP];
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
-    const T *q = p < TS ? pl : (p < TS + BK ? pc : ph);
-    c[p] = widen(q[(p - TS) * 64]);
+    const T *q = p < H ? pl : (p < H + BK ? pc : ph);
+    c[p] = widen(q[(p - H) * 64]);
   }
+  constexpr bool kCond = FORM == kCondRaw || FORM == kCondPos;
   auto tap = [](A v) -> A {
-    if constexpr (FORM != kStar) return relu_ref(v);
+    if constexpr (kCond) return relu_ref(v);
     else return v;
   };
-  const int yp = (y < 15 ? t + 16 : t), ym = (y > 0 ? t - 16 : t);
+  int yp[R], ym[R];  // the columns at j + 1 .. j + R and j - 1 .. (of halo rows: any)
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    yp[r] = y + r < 15 ? t + (r + 1) * 16 : t;
+    ym[r] = y > r ? t - (r + 1) * 16 : t;
+  }
 #pragma unroll
   for (int s = 0; s < TS; ++s) {
-    A *buf = lds + (s & 1 ? (NP - 2) * 256 : 0);
-    const int p0 = (s & 1) + 1;
+    A *buf = lds + (s & 1 ? (NP - 2 * R) * 256 : 0);
+    const int p0 = ((s & 1) + 1) * R, lo = (s + 1) * R, hi = NP - (s + 1) * R;
 #pragma unroll
-    for (int p = s + 1; p < NP - s - 1; ++p) buf[(p - p0) * 256 + t] = tap(c[p]);
+    for (int p = lo; p < hi; ++p) buf[(p - p0) * 256 + t] = tap(c[p]);
     __syncthreads();
-    A below = tap(c[s]);
+    A below[R];  // planes p - 1 .. p - R before this sweep
 #pragma unroll
-    for (int p = s + 1; p < NP - s - 1; ++p) {
+    for (int r = 0; r < R; ++r) below[r] = tap(c[lo - 1 - r]);
+#pragma unroll
+    for (int p = lo; p < hi; ++p) {
       const A m = tap(c[p]);
+      const A *row = buf + (p - p0) * 256;
       A acc = a.c[0] * m;
-      acc = fmadd(a.c[1], row_next<true>(m), acc);
-      acc = fmadd(a.c[2], row_next<false>(m), acc);
-      acc = fmadd(a.c[3], buf[(p - p0) * 256 + yp], acc);
-      acc = fmadd(a.c[4], buf[(p - p0) * 256 + ym], acc);
+      acc = fmadd(a.c[1], row_next<true, 1>(m), acc);
+      acc = fmadd(a.c[2], row_next<false, 1>(m), acc);
+      acc = fmadd(a.c[3], row[yp[0]], acc);
+      acc = fmadd(a.c[4], row[ym[0]], acc);
       acc = fmadd(a.c[5], tap(c[p + 1]), acc);
-      acc = fmadd(a.c[6], below, acc);
-      if constexpr (FORM != kStar) {
+      acc = fmadd(a.c[6], below[0], acc);
+      if constexpr (R == 2) {
+        acc = fmadd(a.c[7], row_next<true, 2>(m), acc);
+        acc = fmadd(a.c[8], row_next<false, 2>(m), acc);
+        acc = fmadd(a.c[9], row[yp[R - 1]], acc);
+        acc = fmadd(a.c[10], row[ym[R - 1]], acc);
+        acc = fmadd(a.c[11], c[p + R], acc);
+        acc = fmadd(a.c[12], below[R - 1], acc);
+      }
+      if constexpr (kCond) {
         const bool sel = a.cond_mode == 0 ? (acc > A(0)) : (c[p] > a.theta);
         acc = sel ? acc : -acc;
       }
       Cells<A, 1> o;
       o.v[0] = acc;
       round_cells<T>(o);
-      below = m;
+      if constexpr (R == 2) below[R - 1] = below[0];
+      below[0] = m;
       c[p] = o.v[0];
     }
   }
   if (x >= kHalo && x < kHalo + 8 && y >= kHalo && y < kHalo + 8) {
     T *po = a.out + (size_t)ic * a.out_step + (e + (int)(k0 & 7) * 64);
 #pragma unroll
-    for (int p = TS; p < TS + BK; ++p) narrow(po[(p - TS) * 64], c[p]);
+    for (int p = H; p < H + BK; ++p) narrow(po[(p - H) * 64], c[p]);
   }
 }
 
-// Workgroups (four strips each) the device holds at once.
-template <class T, int TS, int J, int FORM>
-uint32_t steps_slots() {
-  static std::atomic<uint32_t> known{0};
-  uint32_t n = known.load(std::memory_order_relaxed);
-  if (n == 0) {
-    int dev = 0, cus = 256, per = 0;
-    (void)hipGetDevice(&dev);
-    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &per, reinterpret_cast<const void *>(&star_steps<T, TS, J, FORM>), 256, 0);
-    n = (uint32_t)(cus * std::max(1, per));
-    known.store(n, std::memory_order_relaxed);
-  }
-  return n;
+template <class T, int TS, int FORM>
+auto strip_kernel() {
+  if constexpr (FORM == kStar13) return &star13_steps<T>;
+  else return &star_steps<T, TS, 8, FORM>;
 }
 
-// Whether a box goes by blocks (one workgroup per brick) or by strips.  The
-// strips' long serial marches need a few thousand of them to fill the device;
-// the blocks compute 2.9 times the points a pass keeps.  Equal at (us a sweep,
-// blocks / strips): FP64 7-point 128^3 6.9 / 7.1, 160^3 12.4 / 10.4; cond
-// 160^3 16.5 / 17.6, 192^3 27.0 / 19.7; FP32 7-point 160^3 7.3 / 8.5, 192^3
-// 11.2 / 11.2; BF16 160^3 8.4 / 9.9, 192^3 12.9 / 12.8.
-bool steps_by_block(const SweepLaunch &L, const PlanView &P) {
-  const uint32_t most = L.dtype != BK_F64 ? 12000 : L.stencil == BK_COND7 ? 8000 : 5000;
-  return P.ncovered <= most;
-}
+// How a box is cut into strips of 8 rows and marches along k.  Two workgroups
+// (of four strips) per CU; more, shorter marches fill the device better and
+// compute more halo planes.  us a sweep with one, two, three, four workgroups
+// per CU: 7-point FP64 192^3 12.7, 12.5, 14.2, 16.0, FP32 10.6, 10.0, 10.6,
+// 12.2, BF16 256^3 21.0, 17.4, 17.5, 19.1, 13-point FP32 192^3 19.3, 17.9, 18.6,
+// 20.7.  In large boxes marches of at most 64 planes for four sweeps (512^3
+// FP32 97.8 with 171, 93.9 with 64), 171 for fewer sweeps, which are bound by
+// memory (three sweeps 107 against 117, 13-point FP32 167 against 181).
+struct Strips {
+  uint32_t nchunk, njg, njw, ksegs;
+  Strips(const PlanView &P, int ts) {
+    const uint32_t most = (64 - 2 * kHalo) / 8;  // bricks of a strip along i
+    nchunk = (P.box_nb[0] + most - 1) / most;
+    njg = P.box_nb[1];
+    njw = (njg + 3) / 4;
+    const uint64_t per = (uint64_t)nchunk * njw;  // workgroups of a march
+    const uint32_t least = ts == 4 ? P.box_nb[2] / 8 : P.box_nb[2] / 21;
+    uint64_t segs = std::min<uint64_t>(std::max<uint64_t>(512 / per, least), P.box_nb[2]);
+    segs = std::max<uint64_t>(segs, 1);
+    // a little more than the device takes at once (FP64) would wait for a
+    // second turn of a few
+    if (per * segs > 512 && per * segs < 768 && per <= 512) segs = 512 / per;
+    // one a CU where the second would add less than it costs (18^3 bricks: 270
+    // workgroups of 16 planes, a few CUs with two, against 255 of 17)
+    const uint64_t one = 256 / per, n2 = (uint64_t)P.box_nb[2] * 8;
+    if (one >= std::max<uint32_t>(least, 1) && one < segs &&
+        2 * (n2 / one + 2 * kHalo) <= 3 * (n2 / segs + 2 * kHalo))
+      segs = one;
+    ksegs = (uint32_t)segs;
+  }
+  // of workgroups per CU: the fullest CU's while the device takes all at once
+  float load() const {
+    const uint64_t wgs = (uint64_t)nchunk * njw * ksegs;
+    return wgs <= 512 ? (float)((wgs + 255) / 256) : (float)wgs / 256.0f;
+  }
+};
 
 bool clamped_form(const SweepLaunch &L) {
   return L.cond_mode == BK_COND_REFERENCE || L.theta >= 0.0;
+}
+
+// What a pass takes, in us.  A single sweep and a pass by blocks are linear in
+// the bricks (in thousands).  By strips a wave takes `alone` per plane where it
+// has its SIMD to itself, the device `each` per plane and workgroup of a CU,
+// and the memory `brick` per thousand bricks.  Fitted over 28 boxes of 8 to
+// 262144 bricks, one to 80 an axis (errors up to 12 %, single sweeps of a few
+// thousand bricks 25 %).  The form that the model takes is the fastest one or
+// within 5 % of it in all but a few of the 28 boxes and 12 kinds.  Some of both
+// sides, us a sweep (single / blocks / strips): 7-point FP64 8^3 bricks 4.7 /
+// 2.7 / 6.6, 20^3 15.6 / 12.9 / 10.5, 64^3 411 / 376 / 155, 1x140x140 39 / 32 /
+// 62; BF16 64^3 116 / 227 / 97; 13-point FP64 8^3 5.5 / 4.6 / 13, 16^3 11.0 / 14
+// / 14, 64^3 434 / 900 / 289, FP32 8^3 6.0 / 4.1 / 10, 64^3 228 / 370 / 166.
+struct Line {
+  float at0, per_k;
+};
+struct Strip {
+  float at0, alone, each, brick;  // at0 < 0: not built
+};
+struct PassModel {
+  Line single;
+  Line block[2];   // passes of 3 and 4 sweeps; radius 2: of 2
+  Strip strip[2];
+};
+constexpr Strip kNoStrip = {-1.0f, 0.0f, 0.0f, 0.0f};
+constexpr Line kNoLine = {-1.0f, 0.0f};
+const PassModel kModel[4][3] = {
+    // 7-point: FP64, FP32, BF16
+    {{{4.38f, 1.56f}, {{7.52f, 4.53f}, {7.88f, 5.7f}},
+      {{3.27f, 1.38f, 0.96f, 2.07f}, {1.85f, 1.76f, 1.29f, 2.33f}}},
+     {{4.65f, 0.84f}, {{7.47f, 2.21f}, {7.63f, 3.01f}},
+      {{4.5f, 1.12f, 0.74f, 1.14f}, {5.68f, 1.31f, 0.93f, 1.32f}}},
+     {{6.34f, 0.44f}, {{7.56f, 2.59f}, {7.47f, 3.47f}},
+      {{5.38f, 1.26f, 0.83f, 1.04f}, {7.5f, 1.48f, 1.06f, 1.45f}}}},
+    // cond, values: FP64, FP32, BF16
+    {{{5.1f, 1.54f}, {{7.65f, 5.72f}, {8.36f, 7.41f}},
+      {{0.75f, 2.77f, 1.89f, 2.41f}, kNoStrip}},
+     {{5.83f, 0.82f}, {{7.55f, 3.22f}, {7.89f, 4.89f}},
+      {{3.72f, 2.24f, 1.37f, 1.81f}, {1.86f, 3.07f, 1.93f, 2.49f}}},
+     {{7.61f, 0.5f}, {{7.92f, 3.78f}, {8.12f, 5.4f}},
+      {{4.84f, 2.28f, 1.47f, 1.85f}, {20.0f, 0.44f, 1.93f, 2.56f}}}},
+    // cond, clamped values: FP64, FP32, BF16
+    {{{5.09f, 1.55f}, {{7.65f, 5.72f}, {8.08f, 7.43f}},
+      {{0.0f, 2.43f, 1.65f, 2.23f}, {19.45f, 1.47f, 1.9f, 2.59f}}},
+     {{5.74f, 0.82f}, {{7.86f, 3.16f}, {7.83f, 4.87f}},
+      {{4.25f, 1.88f, 1.21f, 1.61f}, {9.89f, 2.21f, 1.57f, 2.04f}}},
+     {{7.61f, 0.49f}, {{7.86f, 3.76f}, {8.15f, 5.37f}},
+      {{4.88f, 2.15f, 1.36f, 1.72f}, {10.72f, 2.41f, 1.75f, 2.23f}}}},
+    // 13-point: FP64, FP32, BF16
+    {{{4.92f, 1.64f}, {{7.41f, 5.92f}, kNoLine},
+      {{1.72f, 1.68f, 1.12f, 2.22f}, kNoStrip}},
+     {{5.4f, 0.86f}, {{7.14f, 2.56f}, kNoLine},
+      {{4.13f, 1.33f, 0.86f, 1.24f}, kNoStrip}},
+     {{6.88f, 0.46f}, {{7.19f, 3.26f}, kNoLine},
+      {kNoStrip, kNoStrip}}},
+};
+
+constexpr float kNever = 1e9f;
+
+// The time of a pass of ts sweeps and whether it goes by blocks.
+float pass_time(const SweepLaunch &L, const PlanView &P, int ts, bool &block) {
+  const int form = L.stencil == BK_STAR13 ? kStar13 : L.stencil == BK_STAR7 ? kStar
+                   : clamped_form(L) ? kCondPos : kCondRaw;
+  const int dt = L.dtype == BK_F64 ? 0 : L.dtype == BK_F32 ? 1 : 2;
+  const PassModel &m = kModel[form][dt];
+  const float k = (float)P.ncovered * 1e-3f;
+  block = false;
+  if (ts == 1) return m.single.at0 + m.single.per_k * k;
+  if ((ts == 2) != (form == kStar13)) return kNever;  // not built
+  const int q = ts == 4;
+  const float b = m.block[q].at0 + m.block[q].per_k * k;
+  float s = kNever;
+  if (m.strip[q].at0 >= 0.0f) {
+    const Strips st(P, ts);
+    const float planes = (float)P.box_nb[2] * 8.0f / (float)st.ksegs +
+                         2.0f * (float)(ts * radius_of(form));
+    s = m.strip[q].at0 + std::max(planes * std::max(m.strip[q].alone, m.strip[q].each * st.load()),
+                                  m.strip[q].brick * k);
+  }
+  block = b <= s;
+  return std::min(b, s);
 }
 
 // Strips of four FP64 sweeps with unclamped cond planes spill (0.75 ms a
 // sweep against 0.22 with three): not built.
 template <class T, int TS, int FORM>
 constexpr bool strip_built() {
+  if (FORM == kStar13) return !std::is_same<T, bf16>::value;
   return !(std::is_same<T, double>::value && TS == 4 && FORM == kCondRaw);
 }
 
@@ -538,9 +824,11 @@ hipError_t launch_steps_t(const SweepLaunch &L, const PlanView &P, hipStream_t s
   a.nb2 = P.box_nb[2];
   a.cond_mode = L.cond_mode;
   a.theta = (A)L.theta;
-  for (int q = 0; q < 7; ++q) a.c[q] = (A)L.coeff[q];
+  for (int q = 0; q < 13; ++q) a.c[q] = (A)L.coeff[q];
   a.nchunk = a.njg = a.njw = a.ksegs = 0;
-  if (steps_by_block(L, P)) {
+  bool block;
+  (void)pass_time(L, P, TS, block);
+  if (block) {
     // half bricks while whole ones would leave half of the 256 CUs without a
     // workgroup (64 bricks: 1.43 us a sweep against 1.58; 216: 1.72 / 1.70)
     if (P.ncovered <= 128)
@@ -551,25 +839,18 @@ hipError_t launch_steps_t(const SweepLaunch &L, const PlanView &P, hipStream_t s
                          a);
     return hipGetLastError();
   }
-  if constexpr (!strip_built<T, TS, FORM>()) {
-    return hipErrorInvalidValue;
-  } else {
-  constexpr int J = 8;
-  const uint32_t most = (64 - 2 * kHalo) / 8;  // bricks of a strip along i
-  a.nchunk = (a.nb0 + most - 1) / most;
-  a.njg = a.nb1 * 8 / J;
-  a.njw = (a.njg + 3) / 4;
-  const uint64_t per = (uint64_t)a.nchunk * a.njw;  // workgroups of a march
-  // marches: enough to fill the device once, of at most 64 planes (shorter
-  // ones read and compute more halo planes; 512^3 FP64, TS = 4: 0.563 ms a
-  // pass with 64 planes, 0.579 with 171, 0.604 with 32) and at least 8
-  const uint64_t segs = std::max<uint64_t>(steps_slots<T, TS, J, FORM>() / per, a.nb2 / 8);
-  a.ksegs = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(segs, a.nb2));
-  const uint64_t nblk = per * a.ksegs;
-  if (nblk > 0x7fffffffull) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((star_steps<T, TS, J, FORM>), dim3((uint32_t)nblk), dim3(256), 0, s, a);
-  return hipGetLastError();
+  if constexpr (strip_built<T, TS, FORM>()) {
+    const Strips st(P, TS);
+    a.nchunk = st.nchunk;
+    a.njg = st.njg;
+    a.njw = st.njw;
+    a.ksegs = st.ksegs;
+    const uint64_t nblk = (uint64_t)st.nchunk * st.njw * st.ksegs;
+    if (nblk > 0x7fffffffull) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((strip_kernel<T, TS, FORM>()), dim3((uint32_t)nblk), dim3(256), 0, s, a);
+    return hipGetLastError();
   }
+  return hipErrorInvalidValue;
 }
 
 template <class T, int FORM>
@@ -584,6 +865,8 @@ hipError_t launch_steps_dt(const SweepLaunch &L, const PlanView &P, int ts, hipS
 template <class T>
 hipError_t launch_steps_st(const SweepLaunch &L, const PlanView &P, int ts, hipStream_t s) {
   if (L.stencil == BK_STAR7) return launch_steps_dt<T, kStar>(L, P, ts, s);
+  if (L.stencil == BK_STAR13)
+    return ts == 2 ? launch_steps_t<T, 2, kStar13>(L, P, s) : hipErrorInvalidValue;
   if (L.stencil == BK_COND7)
     return clamped_form(L) ? launch_steps_dt<T, kCondPos>(L, P, ts, s)
                            : launch_steps_dt<T, kCondRaw>(L, P, ts, s);
@@ -593,7 +876,8 @@ hipError_t launch_steps_st(const SweepLaunch &L, const PlanView &P, int ts, hipS
 }  // namespace
 
 bool steps_fit(const SweepLaunch &L, const PlanView &P) {
-  if (!P.box_ids || (L.stencil != BK_STAR7 && L.stencil != BK_COND7)) return false;
+  if (!P.box_ids || (L.stencil != BK_STAR7 && L.stencil != BK_COND7 && L.stencil != BK_STAR13))
+    return false;
   // both fields take 16-byte stores (single ones in BF16)
   const size_t es = L.dtype == BK_F64 ? 8 : L.dtype == BK_F32 ? 4 : 2;
   const uintptr_t bits = reinterpret_cast<uintptr_t>(L.in) | reinterpret_cast<uintptr_t>(L.out) |
@@ -601,24 +885,12 @@ bool steps_fit(const SweepLaunch &L, const PlanView &P) {
   return es == 2 || bits % 16 == 0;
 }
 
-// The cost of a pass of 1, 3 and 4 sweeps (passes of two are never needed:
-// see SweepSplit) in units of one sweep by itself, refresh included.  By
-// strips, 512^3, ms a pass: FP64 7-point 0.42 / 0.53 / 0.57, FP32 0.235 /
-// 0.318 / 0.353, BF16 0.130 / 0.310 / 0.359; cond with clamped planes FP64
-// 0.42 / 0.59 / 0.74, FP32 0.235 / 0.38 / 0.51, BF16 0.145 / 0.40 / 0.57,
-// unclamped 0.66, 0.42, 0.44 for three.  By blocks, 32^3: 3.3 us / 5.5 us.
+// Several sweeps per pass have to be 6 % faster than the model of single ones.
 void steps_costs(const SweepLaunch &L, const PlanView &P, float cost[5]) {
-  static const float star[3][2] = {{1.25f, 1.35f}, {1.35f, 1.5f}, {2.4f, 2.8f}};
-  static const float pos[3][2] = {{1.4f, 1.76f}, {1.6f, 2.2f}, {2.7f, 4.0f}};
-  static const float raw[3][2] = {{1.56f, 9.0f}, {1.8f, 2.9f}, {3.1f, 5.0f}};
-  const int dt = L.dtype == BK_F64 ? 0 : L.dtype == BK_F32 ? 1 : 2;
-  const float(*t)[2] = L.stencil == BK_STAR7 ? star : clamped_form(L) ? pos : raw;
-  const bool block = steps_by_block(L, P);
+  bool block;
   cost[0] = 0.0f;
-  cost[1] = 1.0f;
-  cost[2] = 9.0f;
-  cost[3] = block ? 1.4f : t[dt][0];
-  cost[4] = block ? 1.6f : t[dt][1];
+  for (int ts = 1; ts <= 4; ++ts) cost[ts] = pass_time(L, P, ts, block);
+  cost[1] *= 0.94f;
 }
 
 hipError_t launch_star_steps(const SweepLaunch &L, const PlanView &P, int ts, hipStream_t s) {
