@@ -385,6 +385,28 @@ STEP_STENCILS = (_lib.BK_STAR7, _lib.BK_COND7, _lib.BK_STAR13)
 DEFAULT_LANE_SHIFT: dict = {}
 
 
+def star_levels(kind: int, dtype: int, n: int, most: int) -> int:
+    """Levels a star's quad unit marches on a grid of n bricks.  More levels
+    read fewer k-halos, fewer units leave a small device idle.  us a sweep,
+    fewer levels / DEFAULT_PLANS': 25-point BF16 20^3 bricks 9.8 (2) / 18.8,
+    45x27x33 35.1 (2) / 39.9, 48^3 82.0 (4) / 81.3, FP32 20^3 12.4 (1) / 13.9,
+    32^3 35.6 (1) / 38.9, 48^3 103.9 (2) / 104.7, FP64 20^3 20.6 (1) / 21.4,
+    45x27x33 83.2 (1) / 81.9; 13-point BF16 20^3 8.0 (1) / 9.7, 45x27x33 25.7
+    (2) / 27.6; 7-point FP32 20^3 10.0 (1) / 10.4, 45x27x33 37.1 (1) / 39.0,
+    48^3 91.0 (1) / 92.6, 64^3 203.9 (1) / 200.7."""
+    wide = kind == _lib.BK_STAR25
+    if dtype == BK_F64:
+        few = 1 if n <= 12000 else most
+    elif dtype == BK_F32:
+        few = (1 if n <= 60000 else 2 if n <= 150000 else most) if wide else (
+            1 if n <= 120000 else most)
+    elif wide:
+        few = 2 if n <= 60000 else 4 if n <= 100000 else most
+    else:
+        few = 1 if n <= 12000 else 2 if n <= 60000 else most
+    return min(few, most)
+
+
 class PeriodicGrid:
     """n = 8*nb interior cells per axis with periodic boundaries, in one of
     two layouts, all tables in HBM:
@@ -523,6 +545,7 @@ class PeriodicGrid:
         choice = DEFAULT_PLANS.get((int(stencil_kind), int(dtype)))
         if choice is None:
             return None
+        n = self.interior.size
         if int(stencil_kind) == _lib.BK_CUBE125:
             # levels per unit by size: one wave marches a unit, so small grids
             # need short units to fill the device (up to 2000 to 14000 bricks
@@ -532,10 +555,11 @@ class PeriodicGrid:
             # 4 levels 329, 6 levels 346; FP32 256^3 84 / 86 / 137, 384^3 3
             # levels 239, 6 levels 272.  1024^3 FP64: 4, 5, 6, 8 and 12 levels
             # within 1.5 % on one host, 8 never the slower.
-            n = self.interior.size
             wide = 4 if dtype == BK_F64 else 3
             choice = ("quad", 8 if n > (1 << 20) else 6 if n > 200000 else wide if n > 80000
                       else 2 if n > 9000 else 1)
+        else:
+            choice = ("quad", star_levels(int(stencil_kind), int(dtype), n, choice[1]))
         return self.plan(*choice)
 
     def auto_wg_bricks(self, stencil_kind: int) -> int:

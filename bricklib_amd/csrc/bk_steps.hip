@@ -747,32 +747,32 @@ constexpr Strip kNoStrip = {-1.0f, 0.0f, 0.0f, 0.0f};
 constexpr Line kNoLine = {-1.0f, 0.0f};
 const PassModel kModel[4][3] = {
     // 7-point: FP64, FP32, BF16
-    {{{4.38f, 1.56f}, {{7.52f, 4.53f}, {7.88f, 5.7f}},
-      {{3.27f, 1.38f, 0.96f, 2.07f}, {1.85f, 1.76f, 1.29f, 2.33f}}},
-     {{4.65f, 0.84f}, {{7.47f, 2.21f}, {7.63f, 3.01f}},
-      {{4.5f, 1.12f, 0.74f, 1.14f}, {5.68f, 1.31f, 0.93f, 1.32f}}},
-     {{6.34f, 0.44f}, {{7.56f, 2.59f}, {7.47f, 3.47f}},
-      {{5.38f, 1.26f, 0.83f, 1.04f}, {7.5f, 1.48f, 1.06f, 1.45f}}}},
+    {{{4.07f, 1.56f}, {{6.32f, 4.6f}, {6.8f, 5.77f}},
+      {{5.64f, 1.2f, 0.89f, 2.03f}, {5.6f, 1.52f, 1.17f, 2.31f}}},
+     {{3.81f, 0.81f}, {{6.37f, 2.25f}, {6.68f, 3.06f}},
+      {{5.93f, 1.0f, 0.71f, 1.11f}, {7.03f, 1.21f, 0.89f, 1.31f}}},
+     {{4.08f, 0.48f}, {{6.45f, 2.61f}, {6.73f, 3.46f}},
+      {{5.85f, 1.2f, 0.81f, 1.05f}, {8.01f, 1.41f, 1.04f, 1.41f}}}},
     // cond, values: FP64, FP32, BF16
-    {{{5.1f, 1.54f}, {{7.65f, 5.72f}, {8.36f, 7.41f}},
-      {{0.75f, 2.77f, 1.89f, 2.41f}, kNoStrip}},
-     {{5.83f, 0.82f}, {{7.55f, 3.22f}, {7.89f, 4.89f}},
-      {{3.72f, 2.24f, 1.37f, 1.81f}, {1.86f, 3.07f, 1.93f, 2.49f}}},
-     {{7.61f, 0.5f}, {{7.92f, 3.78f}, {8.12f, 5.4f}},
-      {{4.84f, 2.28f, 1.47f, 1.85f}, {20.0f, 0.44f, 1.93f, 2.56f}}}},
+    {{{4.96f, 1.53f}, {{6.7f, 5.73f}, {7.44f, 7.45f}},
+      {{5.02f, 2.46f, 1.77f, 2.46f}, kNoStrip}},
+     {{4.4f, 0.8f}, {{6.7f, 3.23f}, {7.07f, 4.91f}},
+      {{6.08f, 2.05f, 1.3f, 1.83f}, {5.07f, 2.83f, 1.84f, 2.48f}}},
+     {{4.57f, 0.54f}, {{6.8f, 3.81f}, {7.54f, 5.39f}},
+      {{6.32f, 2.15f, 1.42f, 1.85f}, {6.08f, 3.05f, 2.02f, 2.65f}}}},
     // cond, clamped values: FP64, FP32, BF16
-    {{{5.09f, 1.55f}, {{7.65f, 5.72f}, {8.08f, 7.43f}},
-      {{0.0f, 2.43f, 1.65f, 2.23f}, {19.45f, 1.47f, 1.9f, 2.59f}}},
-     {{5.74f, 0.82f}, {{7.86f, 3.16f}, {7.83f, 4.87f}},
-      {{4.25f, 1.88f, 1.21f, 1.61f}, {9.89f, 2.21f, 1.57f, 2.04f}}},
-     {{7.61f, 0.49f}, {{7.86f, 3.76f}, {8.15f, 5.37f}},
-      {{4.88f, 2.15f, 1.36f, 1.72f}, {10.72f, 2.41f, 1.75f, 2.23f}}}},
+    {{{4.95f, 1.54f}, {{6.71f, 5.74f}, {7.42f, 7.45f}},
+      {{4.02f, 2.14f, 1.54f, 2.19f}, {20.0f, 1.68f, 1.84f, 2.75f}}},
+     {{4.38f, 0.81f}, {{6.68f, 3.21f}, {7.06f, 4.89f}},
+      {{6.06f, 1.74f, 1.17f, 1.62f}, {10.79f, 2.13f, 1.53f, 2.04f}}},
+     {{4.54f, 0.54f}, {{6.74f, 3.8f}, {7.51f, 5.39f}},
+      {{6.19f, 2.03f, 1.32f, 1.72f}, {11.74f, 2.3f, 1.71f, 2.23f}}}},
     // 13-point: FP64, FP32, BF16
-    {{{4.92f, 1.64f}, {{7.41f, 5.92f}, kNoLine},
-      {{1.72f, 1.68f, 1.12f, 2.22f}, kNoStrip}},
-     {{5.4f, 0.86f}, {{7.14f, 2.56f}, kNoLine},
-      {{4.13f, 1.33f, 0.86f, 1.24f}, kNoStrip}},
-     {{6.88f, 0.46f}, {{7.19f, 3.26f}, kNoLine},
+    {{{4.73f, 1.64f}, {{6.24f, 5.98f}, kNoLine},
+      {{5.79f, 1.42f, 1.02f, 2.19f}, kNoStrip}},
+     {{4.28f, 0.84f}, {{6.53f, 2.56f}, kNoLine},
+      {{5.44f, 1.23f, 0.82f, 1.22f}, kNoStrip}},
+     {{4.36f, 0.5f}, {{6.18f, 3.29f}, kNoLine},
       {kNoStrip, kNoStrip}}},
 };
 
