@@ -1,7 +1,5 @@
 // bk_shape.hip -- per-brick sweeps for bricks of other shapes and vector
-// folds: Brick<Dim<4,8,16>,Dim<4,16>> and Brick<Dim<4,8,16>,Dim<8,8>>,
-// plus the 8x8x8 brick through the same code (a candidate the tuner times
-// against the dedicated 8x8x8 kernels).
+// folds: Brick<Dim<4,8,16>,Dim<4,16>> and Brick<Dim<4,8,16>,Dim<8,8>>.
 //
 // Element (k, j, i) of a (BK, BJ, BI) brick in fold (FJ, FI) sits at
 //   vec * 64 + (j % FJ) * FI + i % FI,
@@ -17,7 +15,8 @@
 //     k-plane) or of the k-1 / k+1 neighbour's planes, all in registers;
 //   - i/j taps: an LDS tile [BK][BJ+2R][BI+2R] per wave holding the brick
 //     and the R-deep faces of its four in-plane neighbours;
-//   - the cube: an LDS box [BK+4][BJ+4][BI+4] with all 26 neighbours' cells.
+//   - the cube: an LDS box [BK+4][BJ+4][BI+4] with all 26 neighbours' cells,
+//     lanes by pairs of rows (at the kernel).
 // Each point is evaluated in the same fixed order as the 8x8x8 kernels
 // (stars: centre, then i+r, i-r, j+r, j-r, k+r, k-r for r = 1..R; cube:
 // (dk, dj, di) lexicographic), so a cell's value does not depend on the
@@ -29,9 +28,6 @@ namespace bk {
 namespace {
 
 template <int LAY> struct Shape;
-template <> struct Shape<BK_LAYOUT_8x8x8> {
-  static constexpr int BK = 8, BJ = 8, BI = 8, FJ = 8, FI = 8;
-};
 template <> struct Shape<BK_LAYOUT_4x8x16> {
   static constexpr int BK = 4, BJ = 8, BI = 16, FJ = 4, FI = 16;
 };
@@ -168,61 +164,112 @@ __global__ __launch_bounds__(64 * WPB) void star_sweep_shape(const ShapeArgs<T, 
 }
 
 // ---------------------------------------------------------------------------
-// the 125-point cube: the whole 5x5x5 neighbourhood from an LDS box
+// the 125-point cube on 4x8x16 bricks: the 5x5x5 neighbourhoods from an LDS box
 // ---------------------------------------------------------------------------
+// A wave a brick, lane (jj, i) the columns of rows 2 jj and 2 jj + 1: eight
+// points.  Every cell that a lane reads from the box serves all of its points
+// that have it as a tap -- 30 reads per plane of the box, 240 for 1000
+// multiply-adds, where a read per tap bound the kernel by LDS bandwidth.  The
+// box's rows come 16 lanes a row, four rows at once, from bricks that a select
+// between two gives (a division per cell took as long as the taps).  256^3, us
+// before / now: FP64 782 / 142, FP32 347 / 82, BF16 239 / 79 (fold 4x16), 918 /
+// 139, 354 / 79, 238 / 75 (fold 8x8); bound by the VALU, 53 for the taps alone.
+// With fences for the scheduler per plane (81 registers instead of 154 in FP64)
+// 172, 89, 86.
 template <class T, int LAY, int WPB>
 __global__ __launch_bounds__(64 * WPB) void cube_sweep_shape(const ShapeArgs<T, 125> a) {
   using A = typename acc_of<T>::type;
   using F = Fold<LAY>;
   constexpr int R = 2;
   constexpr int BK = F::BK, BJ = F::BJ, BI = F::BI;
-  constexpr int PJ = BJ + 2 * R, PI = BI + 2 * R, PK = BK + 2 * R, PL = PJ * PI;
+  static_assert(BK == 4 && BJ == 8 && BI == 16, "lane (jj, i), rows in groups of four");
+  constexpr int PK = BK + 2 * R, PJ = BJ + 2 * R;
+  constexpr int PI = 24;  // BI + 2 R cells and four unused: rows 2 jj in different banks
+  constexpr int PL = PJ * PI;
   __shared__ A boxes[WPB][PK * PL];
   __shared__ uint32_t nbr[WPB][27];
 
   const int w = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
+  const int jj = lane >> 4, i = lane & 15;
   const uint32_t slot = xcd_remap(blockIdx.x, gridDim.x) * WPB + (uint32_t)w;
   const bool active = slot < a.nlist;
   A *box = boxes[w];
   uint32_t b = 0;
   if (active) {
     b = uniform(a.list[slot]);
-    if (lane < 27) nbr[w][lane] = a.adj[(size_t)b * 27 + lane];
-    const T *pc = a.in + (size_t)b * a.in_step;
+    const uint32_t *ab = a.adj + (size_t)b * 27;
+    if (lane < 27) nbr[w][lane] = ab[lane];
+    // the rows' middle 16 cells; group g: rows 4 g .. 4 g + 3 of a plane
+    A v[PK][3];
 #pragma unroll
-    for (int n = 0; n < 8; ++n)
-      box[(R + F::kof(n)) * PL + (R + F::jof(n, lane)) * PI + R + F::iof(n, lane)] =
-          widen(pc[n * 64 + lane]);
+    for (int g = 0; g < 3; ++g) {
+      const int y = 4 * g + jj, jr = (y + BJ - R) % BJ;
+#pragma unroll
+      for (int kd = 0; kd < 3; ++kd) {
+        const uint32_t lo = uniform(ab[kd * 9 + (g == 2 ? 1 : g) * 3 + 1]),
+                       hi = uniform(ab[kd * 9 + (g == 0 ? 1 : g) * 3 + 1]);
+        const T *p = a.in + (size_t)(jj < 2 ? lo : hi) * a.in_step;
+#pragma unroll
+        for (int z = 0; z < PK; ++z)
+          if ((z + BK - R) / BK == kd) v[z][g] = widen(p[F::off((z + BK - R) % BK, jr, i)]);
+      }
+    }
+#pragma unroll
+    for (int z = 0; z < PK; ++z)
+#pragma unroll
+      for (int g = 0; g < 3; ++g) box[z * PL + (4 * g + jj) * PI + R + i] = v[z][g];
   }
   __syncthreads();
   if (active) {
-    // the cells of the box outside the brick, each from its neighbour
-    for (int q = lane; q < PK * PL; q += 64) {
-      const int x = q % PI, y = (q / PI) % PJ, z = q / PL;
-      const int k = z - R, j = y - R, i = x - R;
-      const int kd = (k + BK) / BK, jd = (j + BJ) / BJ, id = (i + BI) / BI;
-      if (kd == 1 && jd == 1 && id == 1) continue;
-      const uint32_t nb = nbr[w][kd * 9 + jd * 3 + id];
-      box[q] = widen(a.in[(size_t)nb * a.in_step +
-                          F::off((k + BK) % BK, (j + BJ) % BJ, (i + BI) % BI)]);
+    // the two cells at either end of the rows, four lanes a row
+    const int c = lane & 3;
+#pragma unroll
+    for (int q = 0; q < PK * PJ / 16; ++q) {
+      const int row = q * 16 + (lane >> 2), z = row / PJ, y = row % PJ;
+      const int k = z + BK - R, j = y + BJ - R;
+      const uint32_t nb = nbr[w][(k / BK) * 9 + (j / BJ) * 3 + (c < R ? 0 : 2)];
+      box[row * PI + (c < R ? c : BI + c)] = widen(
+          a.in[(size_t)nb * a.in_step + F::off(k % BK, j % BJ, c < R ? BI - R + c : c - R)]);
     }
   }
   __syncthreads();
   if (!active) return;
-  T *__restrict__ po = a.out + (size_t)b * a.out_step;
-#pragma unroll 1
-  for (int n = 0; n < 8; ++n) {
-    const int k = F::kof(n), j = F::jof(n, lane), i = F::iof(n, lane);
-    const A *t = box + k * PL + j * PI + i;  // the (-2, -2, -2) corner
-    A acc = a.c[0] * t[0];
+  const A *t = box + 2 * jj * PI + i;  // the (-2, -2, -2) corner of row 2 jj
+  A acc[BK][2];
 #pragma unroll
-    for (int q = 1; q < 125; ++q) {
-      const int dk = q / 25, dj = (q / 5) % 5, di = q % 5;
-      acc = fmadd(a.c[q], t[dk * PL + dj * PI + di], acc);
+  for (int z = 0; z < PK; ++z) {
+#pragma unroll
+    for (int y = 0; y < 2 + 2 * R; ++y) {
+      A x[5];
+#pragma unroll
+      for (int d = 0; d < 5; ++d) x[d] = t[z * PL + y * PI + d];
+#pragma unroll
+      for (int k = 0; k < BK; ++k) {
+        const int dk = z - k;
+        if (dk < 0 || dk > 4) continue;
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+          const int dj = y - r;
+          if (dj < 0 || dj > 4) continue;
+#pragma unroll
+          for (int d = 0; d < 5; ++d) {
+            const A cc = a.c[dk * 25 + dj * 5 + d];
+            acc[k][r] = dk + dj + d == 0 ? cc * x[d] : fmadd(cc, x[d], acc[k][r]);
+          }
+        }
+      }
     }
-    store_nt(&po[n * 64 + lane], acc);
   }
+  // complete before the stores: the BF16 rounding branches, and the sums would
+  // move into its branches one by one (245 registers)
+#pragma unroll
+  for (int k = 0; k < BK; ++k) asm volatile("" : "+v"(acc[k][0]), "+v"(acc[k][1]));
+  T *__restrict__ po = a.out + (size_t)b * a.out_step;
+#pragma unroll
+  for (int k = 0; k < BK; ++k)
+#pragma unroll
+    for (int r = 0; r < 2; ++r) store_nt(&po[F::off(k, 2 * jj + r, i)], acc[k][r]);
 }
 
 template <class T, int NC>
@@ -285,7 +332,6 @@ hipError_t launch_lay(const SweepLaunch &L, hipStream_t s) {
 template <class T>
 hipError_t launch_dt(const SweepLaunch &L, hipStream_t s) {
   switch (L.layout) {
-    case BK_LAYOUT_8x8x8: return launch_lay<T, BK_LAYOUT_8x8x8>(L, s);
     case BK_LAYOUT_4x8x16: return launch_lay<T, BK_LAYOUT_4x8x16>(L, s);
     case BK_LAYOUT_4x8x16_F88: return launch_lay<T, BK_LAYOUT_4x8x16_F88>(L, s);
     default: return hipErrorInvalidValue;
