@@ -548,13 +548,13 @@ class PeriodicGrid:
         n = self.interior.size
         if int(stencil_kind) == _lib.BK_CUBE125:
             # levels per unit by size: one wave marches a unit, so small grids
-            # need short units to fill the device (up to 2000 to 14000 bricks
-            # the library takes a workgroup per level).  us a sweep: FP64
-            # 160^3 1 level 30, 2 levels 37, 6 levels 91; 256^3 2 levels 98, 1
-            # level 103, 6 levels 136; 320^3 2 levels 197, 6 levels 205; 384^3
-            # 4 levels 329, 6 levels 346; FP32 256^3 84 / 86 / 137, 384^3 3
-            # levels 239, 6 levels 272.  1024^3 FP64: 4, 5, 6, 8 and 12 levels
-            # within 1.5 % on one host, 8 never the slower.
+            # need short units to fill the device (up to 4500 bricks in FP64 and
+            # 130000 in the narrower types the library takes other forms, with
+            # any plan).  us a sweep: FP64 160^3 1 level 30, 2 levels 37, 6
+            # levels 91; 256^3 2 levels 98, 1 level 103, 6 levels 136; 320^3 2
+            # levels 197, 6 levels 205; 384^3 4 levels 329, 6 levels 346.
+            # 1024^3 FP64: 4, 5, 6, 8 and 12 levels within 1.5 % on one host, 8
+            # never the slower.
             wide = 4 if dtype == BK_F64 else 3
             choice = ("quad", 8 if n > (1 << 20) else 6 if n > 200000 else wide if n > 80000
                       else 2 if n > 9000 else 1)

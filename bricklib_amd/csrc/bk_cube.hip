@@ -4,14 +4,11 @@
 // Replaces the codegen brick kernel of weak/main.hip.cpp:32-40 built from
 // stencils/mpi125pt.py:12-162 (here one coefficient per offset).
 //
-// One wave64 per brick, four bricks per workgroup.  The wave gathers the
-// brick's 12x12x12 neighbourhood (its own 512 points plus the 2-deep shell
-// from all 26 neighbours, found through the adjacency table) into LDS, then
-// lane L = j*8 + i accumulates the eight outputs of column (j, i): for each
-// input plane kk it reads the 5x5 window once and feeds it to every output
-// plane within reach, so each LDS value serves up to five FMAs.  Per point
+// Three forms: a wave a brick over any list (below), a wave marching a 2x2
+// block of brick columns, and a workgroup a level of such a block.  Per point
 // the taps accumulate in (dk, dj, di) lexicographic order, starting with a
-// multiply -- the coefficient order of the API.
+// multiply -- the coefficient order of the API -- so the bits do not depend on
+// the form.
 #include <cstddef>
 
 #include "bk_device.h"
@@ -39,65 +36,123 @@ struct CubeArgs {
   A c[125];
 };
 
-template <class T>
-__global__ __launch_bounds__(256) void cube_sweep_lds(const CubeArgs<T> a) {
+// One wave64 per brick.  The wave brings the brick's 12x12x12 neighbourhood (its
+// own 512 points and the 2-deep shell from all 26 neighbours, found through the
+// adjacency table) into LDS; lane (kh, jj, i) accumulates the eight points of
+// planes 4 kh .. 4 kh + 3 and rows 2 jj, 2 jj + 1 of column i, and each cell it
+// reads serves all of them that have it as a tap (240 reads for 1000 multiply-
+// adds).  The box comes in rows of the bricks: 12 loads of whole planes, 6 of
+// the rows before and after, 9 of row ends.  Bound by the VALU (256^3: 53 us for
+// the taps alone): FP32 73 us, BF16 74, FP64 (two and a half waves a SIMD by LDS)
+// 128; with one column of eight planes a lane and the box cell by cell 99, 231
+// (the sums had moved into the stores' branches) and 262.
+//
+// The box of a wave: 12 x 12 rows of 12 cells, planes 8 cells apart: the lanes of
+// a read (two plane halves, four row pairs, eight columns) fall on different
+// banks.
+constexpr int kBoxRow = 12, kBoxPlane = 12 * kBoxRow + 8;
+
+template <class T, int WPB>
+__global__ __launch_bounds__(64 * WPB) void cube_sweep_lds(const CubeArgs<T> a) {
   using A = typename acc_of<T>::type;
-  constexpr int R = 2, P = 8 + 2 * R;  // 12
-  __shared__ A box[4][P][P][P];
-  __shared__ uint32_t sadj[4][32];
+  constexpr int R = 2;
+  __shared__ A boxes[WPB][12 * kBoxPlane];
+  __shared__ uint32_t nbr[WPB][32];
 
   const int w = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
-  const int j = lane >> 3, i = lane & 7;
-  const uint32_t slot = xcd_remap(blockIdx.x, gridDim.x) * 4u + (uint32_t)w;
+  const uint32_t slot = xcd_remap(blockIdx.x, gridDim.x) * WPB + (uint32_t)w;
   const bool active = slot < a.nlist;
-
+  A *box = boxes[w];
   uint32_t b = 0;
   if (active) {
     b = uniform(a.list[slot]);
-    if (lane < 27) sadj[w][lane] = a.adj[(size_t)b * 27 + lane];
+    const uint32_t *ab = a.adj + (size_t)b * 27;
+    if (lane < 27) nbr[w][lane] = ab[lane];
+    // the planes' own columns: a load a plane; and the rows before and after
+    // them, two planes a load
+    A v[12], e[6];
+    const int r4 = (lane >> 3) & 3, hp = lane >> 5;  // halo row, plane of the two
+#pragma unroll
+    for (int kd = 0; kd < 3; ++kd) {
+      const T *pc = a.in + (size_t)uniform(ab[kd * 9 + 4]) * a.in_step;
+      const uint32_t jm = uniform(ab[kd * 9 + 1]), jp = uniform(ab[kd * 9 + 7]);
+      const T *pj = a.in + (size_t)(r4 < R ? jm : jp) * a.in_step +
+                    (r4 < R ? 8 - R + r4 : r4 - R) * 8 + (lane & 7);
+#pragma unroll
+      for (int z = 0; z < 12; ++z) {
+        if ((z + 8 - R) / 8 != kd) continue;
+        const int k = (z + 8 - R) % 8;
+        v[z] = widen(pc[k * 64 + lane]);
+        if (z % 2 == 0) e[z / 2] = widen(pj[(k + hp) * 64]);
+      }
+    }
+    const int own = (R + (lane >> 3)) * kBoxRow + R + (lane & 7);
+    const int rim = hp * kBoxPlane + (r4 < R ? r4 : 8 + r4) * kBoxRow + R + (lane & 7);
+#pragma unroll
+    for (int z = 0; z < 12; ++z) {
+      box[z * kBoxPlane + own] = v[z];
+      if (z % 2 == 0) box[z * kBoxPlane + rim] = e[z / 2];
+    }
   }
   __syncthreads();
   if (active) {
-    const size_t st = a.in_step;
+    // the two cells at either end of the rows, four lanes a row
+    const int c = lane & 3;
+    A x[9];
 #pragma unroll
-    for (int t = 0; t < 27; ++t) {  // 27 * 64 == 12^3
-      const int q = t * 64 + lane;
-      const int kk = q / (P * P), rem = q - kk * P * P;
-      const int jj = rem / P, ii = rem - jj * P;
-      const int k = kk - R + 8, jn = jj - R + 8, in_ = ii - R + 8;  // shifted by +8
-      const int s = (k >> 3) * 9 + (jn >> 3) * 3 + (in_ >> 3);
-      const int e = (k & 7) * 64 + (jn & 7) * 8 + (in_ & 7);
-      box[w][kk][jj][ii] = widen(a.in[(size_t)sadj[w][s] * st + e]);
+    for (int q = 0; q < 9; ++q) {
+      const int row = q * 16 + (lane >> 2), k = row / 12 + 8 - R, j = row % 12 + 8 - R;
+      const uint32_t nb = nbr[w][(k >> 3) * 9 + (j >> 3) * 3 + (c < R ? 0 : 2)];
+      x[q] = widen(a.in[(size_t)nb * a.in_step +
+                        ((k & 7) * 64 + (j & 7) * 8 + (c < R ? 8 - R + c : c - R))]);
+    }
+#pragma unroll
+    for (int q = 0; q < 9; ++q) {
+      const int row = q * 16 + (lane >> 2);
+      box[(row / 12) * kBoxPlane + (row % 12) * kBoxRow + (c < R ? c : 8 + c)] = x[q];
     }
   }
   __syncthreads();
   if (!active) return;
 
-  A acc[8];
+  // planes 4 kh .. 4 kh + 3, rows 2 jj and 2 jj + 1 of column i
+  const int i = lane & 7, jj = (lane >> 3) & 3, kh = lane >> 5;
+  const A *t = box + 4 * kh * kBoxPlane + 2 * jj * kBoxRow + i;
+  A acc[4][2];
 #pragma unroll
-  for (int kk = 0; kk < P; ++kk) {
+  for (int z = 0; z < 8; ++z) {
 #pragma unroll
-    for (int dj = 0; dj < 5; ++dj) {
+    for (int y = 0; y < 6; ++y) {
+      A x[5];
 #pragma unroll
-      for (int di = 0; di < 5; ++di) {
-        const A x = box[w][kk][j + dj][i + di];
+      for (int d = 0; d < 5; ++d) x[d] = t[z * kBoxPlane + y * kBoxRow + d];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          const int dk = kk - k;  // 0..4 when plane kk reaches output k
-          if (dk < 0 || dk > 4) continue;
-          const A c = a.c[dk * 25 + dj * 5 + di];
-          if (dk == 0 && dj == 0 && di == 0) acc[k] = c * x;
-          else acc[k] = fmadd(c, x, acc[k]);
+      for (int k = 0; k < 4; ++k) {
+        const int dk = z - k;  // 0..4 when the plane reaches output k
+        if (dk < 0 || dk > 4) continue;
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+          const int dj = y - r;
+          if (dj < 0 || dj > 4) continue;
+#pragma unroll
+          for (int d = 0; d < 5; ++d) {
+            const A cc = a.c[dk * 25 + dj * 5 + d];
+            acc[k][r] = dk + dj + d == 0 ? cc * x[d] : fmadd(cc, x[d], acc[k][r]);
+          }
         }
       }
     }
   }
-  T *po = a.out + (size_t)b * a.out_step;
+  // complete before the stores, whose BF16 rounding branches
 #pragma unroll
-  for (int k = 0; k < 8; ++k) narrow(po[k * 64 + lane], acc[k]);
+  for (int k = 0; k < 4; ++k) asm volatile("" : "+v"(acc[k][0]), "+v"(acc[k][1]));
+  T *po = a.out + (size_t)b * a.out_step + kh * 256 + jj * 16 + i;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+#pragma unroll
+    for (int r = 0; r < 2; ++r) narrow(po[k * 64 + r * 8], acc[k][r]);
 }
-
 
 // Plane-streaming variant over 2x2 column quads (plan shape BK_PLAN_QUAD).
 //
@@ -625,13 +680,13 @@ __device__ __forceinline__ void cube_quad_unit_dma(
 // KO = 1 more), so past the sizes where waves are scarce the marching form is
 // the faster one.  Per point the taps go (dk, dj, di) lexicographic.
 //
-// us a sweep, block KO = 1 / KO = 2 / best marching plan / one brick a wave
-// (the six-level plans of large grids took 85 to 137 us at these sizes):
-//   FP64  64^3 7.9 / 8.6 / 18.0 / 10.1, 128^3 22.2 / 20.1 / 21.7 / 36.5,
-//         160^3 36 / 32 / 30, 256^3 138 / 121 / 98
-//   FP32  64^3 6.7 / 8.3 / 23.1 / 7.9, 128^3 15.4 / 15.6 / 27.3 / 18.1,
-//         192^3 41.3 / 40.6 / 48.4 / 52, 256^3 88.0 / 84.6 / 83.7
-//   BF16 as FP32.
+// us a sweep, block KO = 1 / KO = 2 / best marching plan (the six-level plans of
+// large grids took 85 to 137 us at these sizes):
+//   FP64  64^3 7.9 / 8.6 / 18.0, 128^3 22.2 / 20.1 / 21.7, 160^3 36 / 32 / 30,
+//         256^3 138 / 121 / 98
+//   FP32  64^3 6.7 / 8.3 / 23.1, 128^3 15.4 / 15.6 / 27.3, 192^3 41.3 / 40.6 /
+//         48.4, 256^3 88.0 / 84.6 / 83.7
+//   BF16 as FP32.  (Single grids of these types: see by_brick.)
 // A row stride of 20 cells (four instead of three FP64 workgroups a CU) and
 // touching the coefficients' lines ahead of the loads were no faster.
 template <class T, int KO>
@@ -892,9 +947,25 @@ int block_planes(size_t es, uint64_t bricks) {
   return bricks <= (es == 8 ? 4500u : 14000u) ? 2 : 0;
 }
 
+// Whether a plan's bricks go one by one: 4- and 2-byte types between the block
+// form and the marching one, us a sweep, block or marching / bricks: FP32 10^3
+// bricks 7.35 / 7.54, 12^3 9.5 / 9.1, 18^3 20.0 / 18.4, 28^3 67 / 53, 32^3 82 / 73,
+// 45x27x33 110 / 90, 50^3 278 / 274, 56^3 371 / 382; BF16 10^3 7.8 / 7.6, 32^3 89 /
+// 74, 50^3 291 / 273, 64^3 535 / 562.  FP64 loses by it: 32^3 104 / 128.
+bool by_brick(size_t es, uint64_t bricks) { return es < 8 && bricks > 1200 && bricks <= 130000; }
+
+template <class T>
+hipError_t launch_t(const SweepLaunch &L, hipStream_t s);
+
 template <class T>
 hipError_t launch_quads_t(const SweepLaunch &L, const PlanView &P, hipStream_t s) {
   using A = typename acc_of<T>::type;
+  if (!P.march && by_brick(sizeof(T), P.ncovered)) {
+    SweepLaunch F = L;
+    F.list = P.flat;
+    F.nlist = P.ncovered;
+    return launch_t<T>(F, s);
+  }
   CubeArgs<T> a;
   a.adj = L.adj;
   a.list = nullptr;
@@ -914,10 +985,10 @@ hipError_t launch_quads_t(const SweepLaunch &L, const PlanView &P, hipStream_t s
   const int ko = P.march || levels > 0x7fffffffull ? 0 : block_planes(sizeof(T), P.ncovered);
   if (ko == 1)
     hipLaunchKernelGGL((cube_sweep_block<T, 1>), dim3((uint32_t)levels), dim3(512), 0, s, a);
-  else if (ko == 2)
-    hipLaunchKernelGGL((cube_sweep_block<T, 2>), dim3((uint32_t)levels), dim3(256), 0, s, a);
-  else
+  else if (ko == 0)
     hipLaunchKernelGGL((cube_sweep_quads<T>), dim3(P.nunits), dim3(64), 0, s, a);
+  else if constexpr (sizeof(T) == 8)  // (narrower types went by bricks)
+    hipLaunchKernelGGL((cube_sweep_block<T, 2>), dim3((uint32_t)levels), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
@@ -935,8 +1006,9 @@ hipError_t launch_t(const SweepLaunch &L, hipStream_t s) {
   a.anchor = a.len = a.mask = nullptr;
   a.nunits = a.kcol = 0;
   for (int q = 0; q < 125; ++q) a.c[q] = (A)L.coeff[q];
-  const uint32_t nwg = (L.nlist + 3u) / 4u;
-  hipLaunchKernelGGL((cube_sweep_lds<T>), dim3(nwg), dim3(256), 0, s, a);
+  constexpr int WPB = sizeof(T) == 8 ? 2 : 4;
+  const uint32_t nwg = (L.nlist + WPB - 1) / WPB;
+  hipLaunchKernelGGL((cube_sweep_lds<T, WPB>), dim3(nwg), dim3(64 * WPB), 0, s, a);
   return hipGetLastError();
 }
 
