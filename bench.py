@@ -4,15 +4,15 @@ Workload (the headline): 7-point star, FP64, 512^3 interior cells plus an
 8-cell ghost zone (66^3 bricks of 8x8x8), inputs U[-1,1], per-axis
 symmetric coefficients U(0,1) normalised to sum 1, periodic ghost-brick
 refresh every sweep, ping-pong sweeps.  One "step" is one sweep over all
-262144 interior bricks whose stores also refresh the periodic ghost bricks
-of its output (the fused form: the input's ghosts are refreshed once before
-the first step; the separate-refresh form is reported in by_stencil); the
-reported value is
-interior cells per second of the timed steps (GStencil/s), timed with HIP
-events recorded on the stream the kernels run on.
+262144 interior bricks (bk_sweeps_fused over a plan declared a periodic box:
+the library takes up to four sweeps per pass over the field and leaves both
+fields, ghost bricks included, bit for bit as single sweeps with a refresh
+each do; the separate-refresh form is reported in by_stencil); the reported
+value is interior cells per second of the timed steps (GStencil/s), timed
+with HIP events recorded on the stream the kernels run on.
 
 The same JSON line also carries:
-  roofline     -- the sweep kernel alone (no refresh): algorithmic bytes
+  roofline     -- the single-sweep kernel alone (no refresh): algorithmic bytes
                   (16 B/point: one FP64 read + one write) / its mean launch
                   time, against the 8 TB/s HBM3E peak; `measured_copy_gbs`
                   is a plain device copy kernel on the same box;
@@ -445,17 +445,17 @@ def main():
     print(f"[bench] setup {time.perf_counter() - t_setup:.1f}s, {g.nbricks} bricks, "
           f"{g.npairs} ghost bricks", file=sys.stderr, flush=True)
 
-    # headline: K timed steps, each a sweep whose stores also refresh the
-    # periodic ghost bricks of its output (the input's ghosts are refreshed
-    # once first): bk_sweeps_fused, the same bits as a separate refresh
-    # before every sweep (that form is by_stencil's 7pt_f64_separate_refresh)
+    # headline: K timed steps by bk_sweeps_fused: both fields and their ghost
+    # bricks end as K sweeps leave them whose stores also refresh the ghost
+    # bricks, the same bits as a separate refresh before every sweep (that
+    # form is by_stencil's 7pt_f64_separate_refresh)
     pl7 = g.auto_plan(st7.kind, bk.BK_F64)
     sched7 = ("one brick per wave" if pl7 is None else
               f"2x2 brick blocks ({pl7.shape} plan, {pl7.kcol} level(s) per unit), one "
-              f"workgroup of four waves per block")
+              f"workgroup of four waves per block; up to four sweeps per pass by strips")
     ms_step = time_sweeps(bk, st7, a, b, g, stream, args.steps, args.warmup, fused=True,
                           warm_s=args.warm_s)
-    # the dominant kernel alone, for the roofline
+    # the single-sweep kernel alone, for the roofline
     ms_kernel = time_sweeps(bk, st7, a, b, g, stream, args.steps, 2, refresh=False)
     peak_copy, copies = copy_peak(bk, stream)
     alg_bytes = 16 * pts

@@ -191,12 +191,11 @@ hipError_t enqueue_chain(bk_batch_s *b, const Chain &c, uint32_t t, hipStream_t 
 
 // The launches of a run on stream s.  `fork`: chains that need nothing of each
 // other (a group, or all groups of a type that refreshes ghosts) take all
-// their ticks side by side, on kSide streams and s, one per hardware queue, and
-// join once at the run's end.  A launch of a small group fills a fraction of
+// their ticks side by side, on kSide streams and s, and join once at the run's
+// end.  A launch of a small group fills a fraction of
 // the chip, and behind one another every tick pays every group's start and
 // drain: 24 mixed requests (up to 32^3 bricks, 16 ticks, 10 groups) 1882 ->
-// 1240 us side by side; with one side stream 1465 us, with seven 1831 (more
-// streams than queues).
+// 1240 us side by side; with one side stream 1465 us, with seven 1831.
 hipError_t enqueue_run(bk_batch_s *b, uint32_t nticks, bool fork, hipStream_t s) {
   Chain chain[kGroups];
   int nchains = 0;
