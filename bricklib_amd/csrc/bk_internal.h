@@ -49,6 +49,8 @@ struct PlanView {
   // periodic box (bk_plan_set_box): its brick ids in grid order, or null
   const uint32_t *box_ids;
   const uint32_t *box_adj;  // with ghost bricks: an adjacency that wraps, or null
+  bool box_affine;  // the ids are box_base + i, j, k times box_stride (mod 2^32)
+  uint32_t box_base, box_stride[3];
   uint32_t box_nb[3];
   uint32_t box_npairs;  // ghost pairs that refresh its ghost bricks
   bool march;           // cube: march the units at every size (plan_march)

@@ -48,6 +48,8 @@ struct bk_plan_s {
   // periodic box (bk_plan_set_box): brick ids in grid order, in HBM
   uint32_t *d_box = nullptr;
   uint32_t *d_box_adj = nullptr;  // its wrapped adjacency, behind d_box
+  bool box_affine = false;
+  uint32_t box_base = 0, box_stride[3] = {0, 0, 0};
   uint32_t box_nb[3] = {0, 0, 0};
   uint32_t box_npairs = 0;
   bool march = false;  // the cube marches the units at every size
@@ -74,7 +76,12 @@ const PlanView plan_view(const bk_plan_s *p) {
   v.id = p->id;
   v.box_ids = p->d_box;
   v.box_adj = p->d_box_adj;
-  for (int a = 0; a < 3; ++a) v.box_nb[a] = p->box_nb[a];
+  v.box_affine = p->box_affine;
+  v.box_base = p->box_base;
+  for (int a = 0; a < 3; ++a) {
+    v.box_nb[a] = p->box_nb[a];
+    v.box_stride[a] = p->box_stride[a];
+  }
   v.box_npairs = p->box_npairs;
   v.march = p->march;
   return v;
@@ -452,6 +459,19 @@ int bk_plan_set_box(bk_plan p, const uint32_t *h_adj, const long nb[3], const ui
   p->d_box_adj = nadj ? d + at : nullptr;
   for (int a = 0; a < 3; ++a) p->box_nb[a] = (uint32_t)nb[a];
   p->box_npairs = npairs;
+  // ids that follow a rule (init_grid's numbering): steps from the first brick
+  const size_t step[3] = {1, (size_t)nb[0], (size_t)plane};
+  p->box_base = h_ids[0];
+  for (int a = 0; a < 3; ++a) p->box_stride[a] = nb[a] > 1 ? h_ids[step[a]] - h_ids[0] : 0;
+  p->box_affine = true;
+  q = 0;
+  for (uint32_t k = 0; k < p->box_nb[2] && p->box_affine; ++k)
+    for (uint32_t j = 0; j < p->box_nb[1] && p->box_affine; ++j) {
+      const uint32_t row = p->box_base + j * p->box_stride[1] + k * p->box_stride[2];
+      bool same = true;
+      for (uint32_t i = 0; i < p->box_nb[0]; ++i) same &= h_ids[q++] == row + i * p->box_stride[0];
+      p->box_affine = same;
+    }
   return BK_OK;
 }
 

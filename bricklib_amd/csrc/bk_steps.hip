@@ -68,6 +68,7 @@ struct StepArgs {
   uint64_t in_step;
   uint64_t out_step;
   uint32_t nb0, nb1, nb2;  // bricks of the box along i, j, k
+  uint32_t affine, base, stride[3];  // affine: ids[...] = base + i, j, k by stride
   uint32_t nchunk;         // strips along i
   uint32_t njg;            // strips along j (nb1 * 8 / J)
   uint32_t njw;            // workgroups along j (four strips each)
@@ -600,11 +601,23 @@ __global__ __launch_bounds__(256) void star_steps_block(const StepArgs<T> a) {
   const uint32_t bj = w % a.nb1;
   const uint32_t k0 = w / a.nb1 * BK;  // first output plane
   const uint32_t n0 = a.nb0 * 8, n1 = a.nb1 * 8, n2 = a.nb2 * 8;
-  const uint32_t ci = (bi * 8 + n0 - kHalo + x) % n0, cj = (bj * 8 + n1 - kHalo + y) % n1;
-  const uint32_t kl = (k0 + n2 - 1) % n2, kh = (k0 + BK) % n2;  // planes next to the block
-  const uint32_t row = (cj >> 3) * a.nb0 + (ci >> 3), per = a.nb0 * a.nb1;
-  const uint32_t il = a.ids[(kl >> 3) * per + row], ic = a.ids[(k0 >> 3) * per + row],
-                 ih = a.ids[(kh >> 3) * per + row];
+  // (kHalo before the box to kHalo + 7 past it: at most one box away)
+  auto wrap = [](uint32_t v, uint32_t n) { return v < n ? v : (int)v < 0 ? v + n : v - n; };
+  const uint32_t ci = wrap(bi * 8 - kHalo + x, n0), cj = wrap(bj * 8 - kHalo + y, n1);
+  const uint32_t kl = k0 ? k0 - 1 : n2 - 1, kh = k0 + BK < n2 ? k0 + BK : 0;  // planes next to the block
+  // computed where the ids follow a rule: the table is a load ahead of the loads
+  uint32_t il, ic, ih;
+  if (a.affine) {
+    const uint32_t row = a.base + (cj >> 3) * a.stride[1] + (ci >> 3) * a.stride[0];
+    il = row + (kl >> 3) * a.stride[2];
+    ic = row + (k0 >> 3) * a.stride[2];
+    ih = row + (kh >> 3) * a.stride[2];
+  } else {
+    const uint32_t row = (cj >> 3) * a.nb0 + (ci >> 3), per = a.nb0 * a.nb1;
+    il = a.ids[(kl >> 3) * per + row];
+    ic = a.ids[(k0 >> 3) * per + row];
+    ih = a.ids[(kh >> 3) * per + row];
+  }
   const int e = (int)((cj & 7) * 8 + (ci & 7));
   const T *pl = a.in + (size_t)il * a.in_step + (e + ((int)(kl & 7) + 1) * 64);
   const T *pc = a.in + (size_t)ic * a.in_step + (e + (int)(k0 & 7) * 64);
@@ -815,6 +828,9 @@ hipError_t launch_steps_t(const SweepLaunch &L, const PlanView &P, hipStream_t s
   using A = typename acc_of<T>::type;
   StepArgs<T> a;
   a.ids = P.box_ids;
+  a.affine = P.box_affine;
+  a.base = P.box_base;
+  for (int q = 0; q < 3; ++q) a.stride[q] = P.box_stride[q];
   a.in = static_cast<const T *>(L.in);
   a.out = static_cast<T *>(L.out);
   a.in_step = L.in_step;
