@@ -550,14 +550,14 @@ class PeriodicGrid:
             # levels per unit by size: one wave marches a unit, so small grids
             # need short units to fill the device (up to 4500 bricks in FP64 and
             # 130000 in the narrower types the library takes other forms, with
-            # any plan).  us a sweep: FP64 160^3 1 level 30, 2 levels 37, 6
-            # levels 91; 256^3 2 levels 98, 1 level 103, 6 levels 136; 320^3 2
-            # levels 197, 6 levels 205; 384^3 4 levels 329, 6 levels 346.
-            # 1024^3 FP64: 4, 5, 6, 8 and 12 levels within 1.5 % on one host, 8
-            # never the slower.
-            wide = 4 if dtype == BK_F64 else 3
-            choice = ("quad", 8 if n > (1 << 20) else 6 if n > 200000 else wide if n > 80000
-                      else 2 if n > 9000 else 1)
+            # any plan).  us a sweep, FP64: 160^3 1 level 32, 2 levels 37, 6
+            # levels 91; 176^3 1 level 40, 2 levels 48; 192^3 50 / 49; 256^3 2
+            # levels 90, 1 level 99, 4 levels 95, 6 levels 134; 320^3 2 levels
+            # 177, 6 levels 189; 384^3 3 levels 283, 4 levels 292, 2 levels
+            # 296, 6 levels 310.  1024^3: 4, 5, 6, 8 and 12 levels within
+            # 1.5 % on one host, 8 never the slower.
+            choice = ("quad", 8 if n > (1 << 20) else 6 if n > 200000 else 3 if n > 80000
+                      else 2 if n > 12500 else 1)
         else:
             choice = ("quad", star_levels(int(stencil_kind), int(dtype), n, choice[1]))
         return self.plan(*choice)
