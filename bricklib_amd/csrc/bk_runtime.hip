@@ -107,9 +107,9 @@ int get_scratch(ReduceScratch **p) {
 
 // Partials of bk_field_stats_noalloc: a file-scope device array, one copy per
 // GPU at its own address, held until the process ends (6 KiB).  Its size does
-// not depend on the input: a fixed kReduceBlocks blocks each write their own
-// three partials and the last one reads all of them, so every slot is
-// rewritten by every call.  Behind them the count of blocks done: 0 when the
+// not depend on the input: at most kReduceBlocks blocks each write their own
+// three partials and the last one reads all of theirs, so every slot that a
+// call reads is rewritten by it.  Behind them the count of blocks done: 0 when the
 // library is loaded, and again after every call.  Calls that overlap on one
 // GPU share the array and race.
 constexpr size_t kStaticScratchDoubles = (size_t)bk::kReduceBlocks * 3 + 1;
