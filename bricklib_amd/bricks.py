@@ -320,7 +320,8 @@ class Plan:
         self.nunits = nu.value
         self.ncovered = nc.value
 
-    def set_box(self, info: BrickInfo, nb, ids: np.ndarray, pairs: np.ndarray) -> None:
+    def set_box(self, info: BrickInfo, nb, ids: np.ndarray, pairs: np.ndarray,
+                stream=None) -> None:
         """Declare the plan's bricks a periodic box (bk_plan_set_box): ``ids``
         its nb[0] x nb[1] x nb[2] bricks in grid order (k slowest), ``pairs``
         the (dst, src) ghost pairs, flat.  Sequences of sweeps that refresh
@@ -330,7 +331,8 @@ class Plan:
         pairs = np.ascontiguousarray(pairs, np.uint32)
         check(load().bk_plan_set_box(_vp(self.handle), info.adj.ctypes.data_as(_lib.u32p),
                                      longs(nb), ids.ctypes.data_as(_lib.u32p),
-                                     pairs.ctypes.data_as(_lib.u32p), pairs.size // 2))
+                                     pairs.ctypes.data_as(_lib.u32p), pairs.size // 2,
+                                     _stream_of(stream)))
         self.boxed = True
 
     def __del__(self):
@@ -499,13 +501,13 @@ class PeriodicGrid:
             self._plans[key] = Plan(self.info, blist, shape, kcol)
         return self._plans[key]
 
-    def _declare_box(self, plan) -> None:
+    def _declare_box(self, plan, stream=None) -> None:
         """Declare one of this grid's own quad plans a periodic box, once,
         ahead of a sequence of sweeps that refresh it."""
         if plan.shape != "quad" or plan.boxed or not any(plan is p for p in self._plans.values()):
             return
         try:
-            plan.set_box(self.info, self.nb, self.interior, self.pairs)
+            plan.set_box(self.info, self.nb, self.interior, self.pairs, stream)
         except _lib.BrickError:  # not a periodic box (changed tables): one sweep per pass
             plan.boxed = True
 
@@ -733,7 +735,7 @@ def sweeps(st: Stencil, a: Brick, b: Brick, grid: PeriodicGrid, nsweeps: int,
     npairs = grid.npairs if refresh else 0
     if (nsweeps > 3 and keep[-1] is not None and ghost_iters == 1
             and (npairs or st.kind in STEP_STENCILS)):
-        grid._declare_box(keep[-1])
+        grid._declare_box(keep[-1], stream)
     if fused:
         if ghost_iters != 1:
             raise ValueError("the fused refresh refreshes every sweep (ghost_iters = 1)")

@@ -19,6 +19,8 @@
 #include <atomic>
 #include <cstring>
 #include <new>
+#include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -46,7 +48,9 @@ struct bk_plan_s {
   uint64_t id = 0;               // unique per plan for the process's lifetime (never 0)
   std::vector<bool> covered;     // [nbricks] the covered bricks
   // periodic box (bk_plan_set_box): brick ids in grid order, in HBM
-  uint32_t *d_box = nullptr;
+  // (published last: a sequence of another thread may be reading the plan)
+  std::atomic<uint32_t *> d_box{nullptr};
+  std::mutex box_mu;  // one declaration at a time
   uint32_t *d_box_adj = nullptr;  // its wrapped adjacency, behind d_box
   bool box_affine = false;
   uint32_t box_base = 0, box_stride[3] = {0, 0, 0};
@@ -74,7 +78,7 @@ const PlanView plan_view(const bk_plan_s *p) {
   v.start = p->d_start;
   v.nbricks = p->nbricks;
   v.id = p->id;
-  v.box_ids = p->d_box;
+  v.box_ids = p->d_box.load(std::memory_order_acquire);  // before what goes with it
   v.box_adj = p->d_box_adj;
   v.box_affine = p->box_affine;
   v.box_base = p->box_base;
@@ -372,16 +376,46 @@ int bk_plan_destroy(bk_plan p) {
   // cached graphs captured the plan's device arrays: drop them first
   bk::graphs_forget_plan(p->id);
   (void)hipFree(p->d_arrays);
-  (void)hipFree(p->d_box);
+  (void)hipFree(p->d_box.load());
   delete p;
   return BK_OK;
 }
 
+namespace {
+// Allocations and copies of this thread while one of its streams is capturing:
+// they are not part of the capture.
+struct OutsideCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  OutsideCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~OutsideCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+// The stream for them: the caller's, or while that is capturing one of our own
+// per device, kept until the process ends (creating one takes 4 ms).
+hipError_t setup_stream(hipStream_t &s) {
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &capturing) != hipSuccess) (void)hipGetLastError();
+  if (capturing == hipStreamCaptureStatusNone) return hipSuccess;
+  static std::mutex mu;
+  static std::map<int, hipStream_t> streams;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  std::lock_guard<std::mutex> lock(mu);
+  hipStream_t &kept = streams[dev];
+  if (!kept) e = hipStreamCreateWithFlags(&kept, hipStreamNonBlocking);
+  s = kept;
+  return e;
+}
+}  // namespace
+
 int bk_plan_set_box(bk_plan p, const uint32_t *h_adj, const long nb[3], const uint32_t *h_ids,
-                    const uint32_t *h_pairs, uint32_t npairs) {
+                    const uint32_t *h_pairs, uint32_t npairs, bk_stream stream) {
   if (!p || !h_adj || !nb || !h_ids || (npairs && !h_pairs))
     return bk::plan_fail(BK_ERR_ARG, "bk_plan_set_box: null pointer");
-  if (p->d_box) return bk::plan_fail(BK_ERR_ARG, "bk_plan_set_box: the plan has a box already");
+  std::lock_guard<std::mutex> lock(p->box_mu);
+  if (p->d_box.load())
+    return bk::plan_fail(BK_ERR_ARG, "bk_plan_set_box: the plan has a box already");
   for (int a = 0; a < 3; ++a)
     if (nb[a] <= 0 || nb[a] > (long)p->nbricks)
       return bk::plan_fail(BK_ERR_ARG, "bk_plan_set_box: bricks per axis out of range");
@@ -435,27 +469,31 @@ int bk_plan_set_box(bk_plan p, const uint32_t *h_adj, const long nb[3], const ui
           }
       }
     }
-  // a box with ghost bricks gets an adjacency without them
+  // a box with ghost bricks gets an adjacency without them (a sequence that is
+  // being captured may be the first over the plan)
+  const OutsideCapture outside;
   const size_t at = (n + 63) & ~(size_t)63, nadj = npairs ? (size_t)p->nbricks * 27 : 0;
   uint32_t *d = nullptr;
+  hipStream_t own = static_cast<hipStream_t>(stream);
   hipError_t e = hipMalloc(&d, (at + nadj) * sizeof(uint32_t));
-  if (e == hipSuccess) e = hipMemcpy(d, h_ids, n * sizeof(uint32_t), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = setup_stream(own);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(d, h_ids, n * sizeof(uint32_t), hipMemcpyHostToDevice, own);
   if (e == hipSuccess && nadj) {
-    e = hipMemsetAsync(d + at, 0, nadj * sizeof(uint32_t), nullptr);  // ghost bricks' rows: unused
+    e = hipMemsetAsync(d + at, 0, nadj * sizeof(uint32_t), own);  // ghost bricks' rows: unused
     if (e == hipSuccess) {
-      hipLaunchKernelGGL(wrap_adjacency, dim3((uint32_t)((n + 255) / 256), 27), dim3(256), 0,
-                         nullptr, d, (uint32_t)n, (uint32_t)nb[0], (uint32_t)nb[1],
-                         (uint32_t)nb[2], d + at);
+      hipLaunchKernelGGL(wrap_adjacency, dim3((uint32_t)((n + 255) / 256), 27), dim3(256), 0, own,
+                         d, (uint32_t)n, (uint32_t)nb[0], (uint32_t)nb[1], (uint32_t)nb[2],
+                         d + at);
       e = hipGetLastError();
     }
-    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
   }
+  if (e == hipSuccess) e = hipStreamSynchronize(own);
   if (e != hipSuccess) {
     (void)hipFree(d);
     std::string m = std::string("bk_plan_set_box: ") + hipGetErrorString(e);
     return bk::plan_fail(e == hipErrorOutOfMemory ? BK_ERR_NOMEM : BK_ERR_HIP, m.c_str());
   }
-  p->d_box = d;
   p->d_box_adj = nadj ? d + at : nullptr;
   for (int a = 0; a < 3; ++a) p->box_nb[a] = (uint32_t)nb[a];
   p->box_npairs = npairs;
@@ -472,6 +510,7 @@ int bk_plan_set_box(bk_plan p, const uint32_t *h_adj, const long nb[3], const ui
       for (uint32_t i = 0; i < p->box_nb[0]; ++i) same &= h_ids[q++] == row + i * p->box_stride[0];
       p->box_affine = same;
     }
+  p->d_box.store(d, std::memory_order_release);
   return BK_OK;
 }
 

@@ -313,9 +313,11 @@ int bk_plan_build_host(const uint32_t *h_adj, uint32_t nbricks,
  * the ghost bricks of the input field of the last sweep (of both fields, for
  * bk_sweeps_fused); the ghost bricks of a bk_sweeps result are not refreshed
  * and hold older values.  No counterpart in the reference.  Allocates device
- * memory: the ids and, with pairs, an adjacency of its own. */
+ * memory (the ids and, with pairs, an adjacency of its own), filled on s when
+ * the call returns; a capture of s is left as it is. */
 int bk_plan_set_box(bk_plan plan, const uint32_t *h_adj, const long nb[3],
-                    const uint32_t *h_ids, const uint32_t *h_pairs, uint32_t npairs);
+                    const uint32_t *h_ids, const uint32_t *h_pairs, uint32_t npairs,
+                    bk_stream s);
 int bk_plan_query(bk_plan plan, uint32_t *nunits, uint32_t *kcol, int *shape,
                   uint32_t *ncovered);
 /* Copy the plan's arrays to the host (any pointer may be NULL):
