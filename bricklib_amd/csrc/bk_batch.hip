@@ -189,6 +189,18 @@ hipError_t enqueue_chain(bk_batch_s *b, const Chain &c, uint32_t t, hipStream_t 
   return e;
 }
 
+// The streams and events of forked runs, made for the first of them.
+hipError_t make_sides(bk_batch_s *b) {
+  hipError_t e = hipSuccess;
+  if (!b->forked) e = hipEventCreateWithFlags(&b->forked, hipEventDisableTiming);
+  for (int l = 0; l < kSide && e == hipSuccess; ++l) {
+    if (!b->side[l]) e = hipStreamCreateWithFlags(&b->side[l], hipStreamNonBlocking);
+    if (e == hipSuccess && !b->joined[l])
+      e = hipEventCreateWithFlags(&b->joined[l], hipEventDisableTiming);
+  }
+  return e;
+}
+
 // The launches of a run on stream s.  `fork`: chains that need nothing of each
 // other (a group, or all groups of a type that refreshes ghosts) take all
 // their ticks side by side, on kSide streams and s, and join once at the run's
@@ -282,11 +294,6 @@ int bk_batch_create(uint32_t max_reqs, bk_batch *out) {
   if (hipEventCreateWithFlags(&b->staged, hipEventDisableTiming) != hipSuccess ||
       hipStreamCreateWithFlags(&b->capture, hipStreamNonBlocking) != hipSuccess)
     return cleanup(fail(BK_ERR_HIP, "bk_batch_create: event/stream creation failed"));
-  bool made = hipEventCreateWithFlags(&b->forked, hipEventDisableTiming) == hipSuccess;
-  for (int l = 0; l < kSide; ++l)
-    made = made && hipStreamCreateWithFlags(&b->side[l], hipStreamNonBlocking) == hipSuccess &&
-           hipEventCreateWithFlags(&b->joined[l], hipEventDisableTiming) == hipSuccess;
-  if (!made) return cleanup(fail(BK_ERR_HIP, "bk_batch_create: event/stream creation failed"));
   *out = b;
   return BK_OK;
 }
@@ -446,6 +453,7 @@ int bk_batch_run(bk_batch b, uint32_t nticks, int use_graph, bk_stream stream) {
   const std::tuple<uint32_t, uint64_t, uint32_t> key{
       nticks, b->sweep_mask, b->ref_mask | (fork ? 1u << kDtypes : 0u)};
   if (!b->graphs.find(key)) {
+    if (fork) BKB_HIP(make_sides(b));
     BKB_HIP(hipStreamBeginCapture(b->capture, hipStreamCaptureModeThreadLocal));
     hipError_t e = enqueue_run(b, nticks, fork, b->capture);
     hipGraph_t g = nullptr;
