@@ -79,7 +79,7 @@ hipError_t launch_star_quads(const SweepLaunch &L, const PlanView &P, hipStream_
 hipError_t launch_cube_quads(const SweepLaunch &L, const PlanView &P, hipStream_t s);
 // Several sweeps per pass over a periodic box (bk_steps.hip): whether the
 // kernels take the sweep (plan, stencil, alignment), the passes' costs, and
-// one pass of ts sweeps, 3 or 4, from L.in to L.out.
+// one pass of ts sweeps (3 or 4; radius 2: 2) from L.in to L.out.
 bool steps_fit(const SweepLaunch &L, const PlanView &P);
 void steps_costs(const SweepLaunch &L, const PlanView &P, float cost[5]);
 hipError_t launch_star_steps(const SweepLaunch &L, const PlanView &P, int ts, hipStream_t s);
