@@ -734,7 +734,7 @@ def sweeps(st: Stencil, a: Brick, b: Brick, grid: PeriodicGrid, nsweeps: int,
     pairs = grid.d_pairs.ptr if (refresh and grid.d_pairs is not None) else None
     npairs = grid.npairs if refresh else 0
     if (nsweeps > 3 and keep[-1] is not None and ghost_iters == 1
-            and (npairs or st.kind in STEP_STENCILS)):
+            and (npairs or st.kind in STEP_STENCILS) and hasattr(grid, "_declare_box")):
         grid._declare_box(keep[-1], stream)
     if fused:
         if ghost_iters != 1:
