@@ -250,6 +250,8 @@ SIGNATURES = {
                                  C.POINTER(vp)]),
     "bk_plan_destroy": (C.c_int, [vp]),
     "bk_plan_set_box": (C.c_int, [vp, u32p, longp, u32p, u32p, C.c_uint32, vp]),
+    "bk_plan_bind_box": (C.c_int, [vp, vp, vp, C.c_uint32, vp, vp, vp]),
+    "bk_plan_unbind_box": (C.c_int, [vp]),
     "bk_plan_query": (C.c_int, [vp, u32p, u32p, C.POINTER(C.c_int), u32p]),
     "bk_plan_download": (C.c_int, [vp, u32p, u32p, u32p, u32p]),
     "bk_plan_build_host": (C.c_int, [u32p, C.c_uint32, u32p, C.c_uint32, C.c_int, C.c_uint32,

@@ -315,6 +315,7 @@ class Plan:
         self.shape = shape
         self.kcol = int(kcol)
         self.boxed = False  # set_box ran
+        self.tables: set = set()  # device tables that sequences came with (_declare_box)
         nu, nc = C.c_uint32(), C.c_uint32()
         check(load().bk_plan_query(_vp(self.handle), C.byref(nu), None, None, C.byref(nc)))
         self.nunits = nu.value
@@ -324,9 +325,9 @@ class Plan:
                 stream=None) -> None:
         """Declare the plan's bricks a periodic box (bk_plan_set_box): ``ids``
         its nb[0] x nb[1] x nb[2] bricks in grid order (k slowest), ``pairs``
-        the (dst, src) ghost pairs, flat.  Sequences of sweeps that refresh
-        with those pairs then read the images themselves and may take
-        several sweeps per pass."""
+        the (dst, src) ghost pairs, flat.  Sequences of sweeps whose device
+        tables are bound to the box (bind_box; ``sweeps`` does it) then read
+        the images themselves and may take several sweeps per pass."""
         ids = np.ascontiguousarray(ids, np.uint32)
         pairs = np.ascontiguousarray(pairs, np.uint32)
         check(load().bk_plan_set_box(_vp(self.handle), info.adj.ctypes.data_as(_lib.u32p),
@@ -334,6 +335,19 @@ class Plan:
                                      pairs.ctypes.data_as(_lib.u32p), pairs.size // 2,
                                      _stream_of(stream)))
         self.boxed = True
+
+    def bind_box(self, d_adj: int, d_pairs: int = 0, npairs: int = 0, d_img_off: int = 0,
+                 d_img: int = 0, stream=None) -> None:
+        """Check these device tables against the declared box and let
+        sequences that come with them use it (bk_plan_bind_box), until one of
+        them is written through the library or freed."""
+        check(load().bk_plan_bind_box(_vp(self.handle), _vp(d_adj), _vp(d_pairs), int(npairs),
+                                      _vp(d_img_off), _vp(d_img), _stream_of(stream)))
+
+    def unbind_box(self) -> None:
+        """End every binding of the plan (bk_plan_unbind_box): sequences
+        refresh with their own tables before every sweep again."""
+        check(load().bk_plan_unbind_box(_vp(self.handle)))
 
     def __del__(self):
         try:
@@ -501,15 +515,24 @@ class PeriodicGrid:
             self._plans[key] = Plan(self.info, blist, shape, kcol)
         return self._plans[key]
 
-    def _declare_box(self, plan, stream=None) -> None:
-        """Declare one of this grid's own quad plans a periodic box, once,
-        ahead of a sequence of sweeps that refresh it."""
-        if plan.shape != "quad" or plan.boxed or not any(plan is p for p in self._plans.values()):
+    def _declare_box(self, plan, stream=None, fused: bool = False) -> None:
+        """Ahead of a sequence of sweeps that refresh this grid: declare one
+        of its own quad plans a periodic box, once, and bind the tables that
+        the sequence comes with."""
+        images = tuple(t.ptr for t in self.ghost_images) if fused else (0, 0)
+        tables = (self.info.dptr, self.d_pairs.ptr if self.d_pairs is not None else 0,
+                  self.npairs, *images)
+        if tables in plan.tables or plan.shape != "quad":
             return
+        if not plan.boxed and not any(plan is p for p in self._plans.values()):
+            return
+        plan.tables.add(tables)
         try:
-            plan.set_box(self.info, self.nb, self.interior, self.pairs, stream)
+            if not plan.boxed:
+                plan.set_box(self.info, self.nb, self.interior, self.pairs, stream)
+            plan.bind_box(*tables, stream=stream)
         except _lib.BrickError:  # not a periodic box (changed tables): one sweep per pass
-            plan.boxed = True
+            pass
 
     @property
     def ghost_images(self):
@@ -735,7 +758,7 @@ def sweeps(st: Stencil, a: Brick, b: Brick, grid: PeriodicGrid, nsweeps: int,
     npairs = grid.npairs if refresh else 0
     if (nsweeps > 3 and keep[-1] is not None and ghost_iters == 1
             and (npairs or st.kind in STEP_STENCILS) and hasattr(grid, "_declare_box")):
-        grid._declare_box(keep[-1], stream)
+        grid._declare_box(keep[-1], stream, fused)
     if fused:
         if ghost_iters != 1:
             raise ValueError("the fused refresh refreshes every sweep (ghost_iters = 1)")

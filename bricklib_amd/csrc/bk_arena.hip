@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "bk_api.h"
+#include "bk_internal.h"
 
 namespace bk {
 int plan_fail(int code, const char *msg);
@@ -91,7 +92,10 @@ int bk_arena_create(size_t slab_bytes, size_t capacity, bk_arena *out) {
 
 int bk_arena_destroy(bk_arena a) {
   if (!a) return BK_OK;
-  for (auto &s : a->slabs) (void)hipFree(s.base);
+  for (auto &s : a->slabs) {
+    bk::device_freed(s.base);
+    (void)hipFree(s.base);
+  }
   delete a;
   return BK_OK;
 }

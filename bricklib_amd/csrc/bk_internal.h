@@ -56,6 +56,14 @@ struct PlanView {
   bool march;           // cube: march the units at every size (plan_march)
 };
 const PlanView plan_view(const bk_plan_s *p);
+// Whether these device tables are bound to the plan's box (bk_plan_bind_box);
+// img_off null: a sequence without the fused refresh.
+bool box_bound(const PlanView &P, const uint32_t *adj, const uint32_t *pairs,
+               const uint32_t *img_off, const uint32_t *img);
+// The library writes these bytes, or frees the allocation at p: tables in them
+// are no longer bound.
+void device_written(const void *p, size_t bytes);
+void device_freed(void *p);
 // Keep cube sweeps over the plan to the marching form, the one the batched
 // kernel runs (the tuner times it for them).
 void plan_march(bk_plan_s *p);

@@ -52,6 +52,10 @@ struct bk_plan_s {
   std::atomic<uint32_t *> d_box{nullptr};
   std::mutex box_mu;  // one declaration at a time
   uint32_t *d_box_adj = nullptr;  // its wrapped adjacency, behind d_box
+  uint32_t *d_box_holds = nullptr;  // [nbricks] the box brick each holds the values of, or kNone
+  uint32_t *d_box_seen = nullptr;   // [nbricks] stamps of bk_plan_bind_box, then its two results
+  uint32_t box_stamp = 0;
+  uint32_t box_ghosts = 0;  // ghost bricks the pairs refresh
   bool box_affine = false;
   uint32_t box_base = 0, box_stride[3] = {0, 0, 0};
   uint32_t box_nb[3] = {0, 0, 0};
@@ -92,6 +96,93 @@ const PlanView plan_view(const bk_plan_s *p) {
 }
 
 void plan_march(bk_plan_s *p) { p->march = true; }
+
+namespace {
+// The device tables bound to the plans' boxes (bk_plan_bind_box): a sequence
+// takes what the box stands for in place of its own tables only if they are
+// among these, so what the library writes or frees in them ends the binding.
+struct BoxTables {
+  const uint32_t *adj, *pairs, *img_off, *img;  // pairs: null without ghost bricks
+  std::array<std::pair<uintptr_t, uintptr_t>, 4> span;  // their bytes
+};
+constexpr size_t kMaxBound = 4;  // per plan; the oldest makes way
+struct BoundTables {
+  std::mutex mu;
+  std::map<uint64_t, std::vector<BoxTables>> of;  // by plan id
+  std::atomic<size_t> plans{0};                   // = of.size()
+};
+BoundTables &bound_tables() {
+  static BoundTables *b = new BoundTables;  // frees at exit may still come
+  return *b;
+}
+}  // namespace
+
+bool box_bound(const PlanView &P, const uint32_t *adj, const uint32_t *pairs,
+               const uint32_t *img_off, const uint32_t *img) {
+  BoundTables &B = bound_tables();
+  std::lock_guard<std::mutex> lock(B.mu);
+  const auto it = B.of.find(P.id);
+  if (it == B.of.end()) return false;
+  for (const BoxTables &t : it->second)
+    if (t.adj == adj && (!P.box_npairs || t.pairs == pairs) &&
+        (!img_off || (t.img_off == img_off && t.img == img)))
+      return true;
+  return false;
+}
+
+void device_written(const void *p, size_t bytes) {
+  BoundTables &B = bound_tables();
+  if (!B.plans.load(std::memory_order_acquire)) return;
+  const uintptr_t lo = reinterpret_cast<uintptr_t>(p), hi = lo + bytes;
+  std::lock_guard<std::mutex> lock(B.mu);
+  for (auto &entry : B.of) {
+    auto &v = entry.second;
+    v.erase(std::remove_if(v.begin(), v.end(),
+                           [&](const BoxTables &t) {
+                             return std::any_of(t.span.begin(), t.span.end(), [&](const auto &s) {
+                               return s.first < hi && lo < s.second;
+                             });
+                           }),
+            v.end());
+  }
+}
+
+void device_freed(void *p) {
+  if (!bound_tables().plans.load(std::memory_order_acquire)) return;
+  hipDeviceptr_t base = p;
+  size_t bytes = 1;
+  if (hipMemGetAddressRange(&base, &bytes, p) != hipSuccess) {
+    (void)hipGetLastError();
+    base = p;
+    bytes = 1;
+  }
+  device_written(base, bytes);
+}
+
+namespace {
+void unbind_box(uint64_t plan) {
+  BoundTables &B = bound_tables();
+  std::lock_guard<std::mutex> lock(B.mu);
+  B.of.erase(plan);
+  B.plans.store(B.of.size(), std::memory_order_release);
+}
+
+// in place of older ones at the same addresses
+void bind_box(uint64_t plan, const BoxTables &t) {
+  BoundTables &B = bound_tables();
+  std::lock_guard<std::mutex> lock(B.mu);
+  auto &v = B.of[plan];
+  B.plans.store(B.of.size(), std::memory_order_release);
+  v.erase(std::remove_if(v.begin(), v.end(),
+                         [&](const BoxTables &o) {
+                           return o.adj == t.adj && o.pairs == t.pairs &&
+                                  (!o.img_off || (o.img_off == t.img_off && o.img == t.img));
+                         }),
+          v.end());
+  if (v.size() == kMaxBound) v.erase(v.begin());
+  v.push_back(t);
+}
+}  // namespace
 
 }  // namespace bk
 
@@ -198,6 +289,62 @@ __global__ __launch_bounds__(256) void wrap_adjacency(const uint32_t *__restrict
   const uint32_t ii = (i + nb0 + e % 3 - 1) % nb0, jj = (j + nb1 + e / 3 % 3 - 1) % nb1,
                  kk = (k + nb2 + e / 9 - 1) % nb2;
   adj[(size_t)ids[q] * 27 + e] = ids[(kk * nb1 + jj) * nb0 + ii];
+}
+
+// Whether device tables are those of a declared box, by what each brick holds
+// after a refresh (bk_plan_set_box): result[0] counts entries that are not,
+// result[1] the ghost bricks found, each once (stamped in seen).
+struct BoxCheck {
+  const uint32_t *__restrict__ ids;    // [n]
+  const uint32_t *__restrict__ holds;  // [nbricks]
+  uint32_t *seen;                      // [nbricks]
+  uint32_t *result;
+  uint32_t n, nbricks, nb0, nb1, nb2, npairs, stamp;
+
+  // ghost brick dst takes src's values
+  __device__ __forceinline__ void ghost(uint32_t dst, uint32_t src) const {
+    if (dst >= nbricks || dst == src || holds[dst] != src)
+      atomicAdd(&result[0], 1u);
+    else if (atomicExch(&seen[dst], stamp) != stamp)
+      atomicAdd(&result[1], 1u);
+  }
+};
+
+// thread (q, e): neighbour e of the box's q-th brick
+__global__ __launch_bounds__(256) void check_adjacency(const BoxCheck c,
+                                                       const uint32_t *__restrict__ adj) {
+  const uint32_t q = blockIdx.x * 256 + threadIdx.x, e = blockIdx.y;
+  if (q >= c.n) return;
+  const uint32_t i = q % c.nb0, j = q / c.nb0 % c.nb1, k = q / c.nb0 / c.nb1;
+  const uint32_t ii = (i + c.nb0 + e % 3 - 1) % c.nb0, jj = (j + c.nb1 + e / 3 % 3 - 1) % c.nb1,
+                 kk = (k + c.nb2 + e / 9 - 1) % c.nb2;
+  const uint32_t b = adj[(size_t)c.ids[q] * 27 + e];
+  if (b >= c.nbricks || c.holds[b] != c.ids[(kk * c.nb1 + jj) * c.nb0 + ii])
+    atomicAdd(&c.result[0], 1u);
+}
+
+__global__ __launch_bounds__(256) void check_pairs(const BoxCheck c,
+                                                   const uint32_t *__restrict__ pairs) {
+  const uint32_t q = blockIdx.x * 256 + threadIdx.x;
+  if (q < c.npairs) c.ghost(pairs[2 * (size_t)q], pairs[2 * (size_t)q + 1]);
+}
+
+// off rises from 0 to npairs, so that check_images stays in a table of as many
+__global__ __launch_bounds__(256) void check_offsets(const BoxCheck c,
+                                                     const uint32_t *__restrict__ off) {
+  const uint32_t b = blockIdx.x * 256 + threadIdx.x;
+  if (b >= c.nbricks) return;
+  if (off[b] > off[b + 1] || (b == 0 && (off[0] != 0 || off[c.nbricks] != c.npairs)))
+    atomicAdd(&c.result[0], 1u);
+}
+
+__global__ __launch_bounds__(256) void check_images(const BoxCheck c,
+                                                    const uint32_t *__restrict__ off,
+                                                    const uint32_t *__restrict__ img) {
+  const uint32_t q = blockIdx.x * 256 + threadIdx.x;
+  if (q >= c.n) return;
+  const uint32_t b = c.ids[q];
+  for (uint32_t t = off[b]; t < off[b + 1]; ++t) c.ghost(img[t], b);
 }
 
 // A plan's arrays on the host.
@@ -375,6 +522,7 @@ int bk_plan_destroy(bk_plan p) {
   if (!p) return BK_OK;
   // cached graphs captured the plan's device arrays: drop them first
   bk::graphs_forget_plan(p->id);
+  bk::unbind_box(p->id);
   (void)hipFree(p->d_arrays);
   (void)hipFree(p->d_box.load());
   delete p;
@@ -473,9 +621,10 @@ int bk_plan_set_box(bk_plan p, const uint32_t *h_adj, const long nb[3], const ui
   // being captured may be the first over the plan)
   const OutsideCapture outside;
   const size_t at = (n + 63) & ~(size_t)63, nadj = npairs ? (size_t)p->nbricks * 27 : 0;
-  uint32_t *d = nullptr;
+  const size_t nbr = p->nbricks, total = at + nadj + 2 * nbr + 2;
+  uint32_t *d = nullptr, *d_holds = nullptr;
   hipStream_t own = static_cast<hipStream_t>(stream);
-  hipError_t e = hipMalloc(&d, (at + nadj) * sizeof(uint32_t));
+  hipError_t e = hipMalloc(&d, total * sizeof(uint32_t));
   if (e == hipSuccess) e = setup_stream(own);
   if (e == hipSuccess)
     e = hipMemcpyAsync(d, h_ids, n * sizeof(uint32_t), hipMemcpyHostToDevice, own);
@@ -488,6 +637,11 @@ int bk_plan_set_box(bk_plan p, const uint32_t *h_adj, const long nb[3], const ui
       e = hipGetLastError();
     }
   }
+  if (e == hipSuccess) {
+    d_holds = d + at + nadj;
+    e = hipMemcpyAsync(d_holds, holds.data(), nbr * sizeof(uint32_t), hipMemcpyHostToDevice, own);
+  }
+  if (e == hipSuccess) e = hipMemsetAsync(d_holds + nbr, 0, nbr * sizeof(uint32_t), own);
   if (e == hipSuccess) e = hipStreamSynchronize(own);
   if (e != hipSuccess) {
     (void)hipFree(d);
@@ -495,6 +649,11 @@ int bk_plan_set_box(bk_plan p, const uint32_t *h_adj, const long nb[3], const ui
     return bk::plan_fail(e == hipErrorOutOfMemory ? BK_ERR_NOMEM : BK_ERR_HIP, m.c_str());
   }
   p->d_box_adj = nadj ? d + at : nullptr;
+  p->d_box_holds = d_holds;
+  p->d_box_seen = d_holds + nbr;
+  p->box_ghosts = (uint32_t)(std::count_if(holds.begin(), holds.end(),
+                                           [](uint32_t b) { return b != kNone; }) -
+                             (ptrdiff_t)n);
   for (int a = 0; a < 3; ++a) p->box_nb[a] = (uint32_t)nb[a];
   p->box_npairs = npairs;
   // ids that follow a rule (init_grid's numbering): steps from the first brick
@@ -511,6 +670,75 @@ int bk_plan_set_box(bk_plan p, const uint32_t *h_adj, const long nb[3], const ui
       p->box_affine = same;
     }
   p->d_box.store(d, std::memory_order_release);
+  return BK_OK;
+}
+
+int bk_plan_bind_box(bk_plan p, const uint32_t *d_adj, const uint32_t *d_pairs,
+                     uint32_t npairs, const uint32_t *d_img_off, const uint32_t *d_img,
+                     bk_stream stream) {
+  if (!p || !d_adj || (npairs && !d_pairs) || !d_img_off != !d_img)
+    return bk::plan_fail(BK_ERR_ARG, "bk_plan_bind_box: null pointer");
+  std::lock_guard<std::mutex> lock(p->box_mu);
+  const uint32_t *ids = p->d_box.load();
+  if (!ids) return bk::plan_fail(BK_ERR_ARG, "bk_plan_bind_box: the plan has no box");
+  if (npairs != p->box_npairs)
+    return bk::plan_fail(BK_ERR_UNSUPPORTED, "bk_plan_bind_box: not as many pairs as the box has");
+  const OutsideCapture outside;
+  hipStream_t own = static_cast<hipStream_t>(stream);
+  hipError_t e = setup_stream(own);
+  uint32_t result[2] = {0, 0};
+  const uint32_t n = p->ncovered, nbricks = p->nbricks;
+  const auto blocks = [](uint32_t m) { return dim3((m + 255) / 256); };
+  BoxCheck c{ids,     p->d_box_holds, p->d_box_seen, p->d_box_seen + nbricks, n,
+             nbricks, p->box_nb[0],   p->box_nb[1],  p->box_nb[2],            npairs,   0};
+  // the launches of one check, each ghost brick found once by it; then its results
+  auto check = [&](auto launches, uint32_t ghosts) {
+    if (e == hipSuccess) e = hipMemsetAsync(c.result, 0, sizeof result, own);
+    if (e != hipSuccess) return false;
+    c.stamp = ++p->box_stamp;
+    launches();
+    e = hipGetLastError();
+    if (e == hipSuccess)
+      e = hipMemcpyAsync(result, c.result, sizeof result, hipMemcpyDeviceToHost, own);
+    if (e == hipSuccess) e = hipStreamSynchronize(own);
+    return e == hipSuccess && result[0] == 0 && result[1] == ghosts;
+  };
+  bool same = check(
+      [&] {
+        hipLaunchKernelGGL(check_adjacency, dim3((n + 255) / 256, 27), dim3(256), 0, own, c, d_adj);
+        if (c.npairs)
+          hipLaunchKernelGGL(check_pairs, blocks(c.npairs), dim3(256), 0, own, c, d_pairs);
+        if (d_img_off)
+          hipLaunchKernelGGL(check_offsets, blocks(nbricks), dim3(256), 0, own, c, d_img_off);
+      },
+      p->box_ghosts);
+  if (same && d_img_off && c.npairs)
+    same = check(
+        [&] {
+          hipLaunchKernelGGL(check_images, blocks(n), dim3(256), 0, own, c, d_img_off, d_img);
+        },
+        p->box_ghosts);
+  if (e != hipSuccess) {
+    std::string m = std::string("bk_plan_bind_box: ") + hipGetErrorString(e);
+    return bk::plan_fail(BK_ERR_HIP, m.c_str());
+  }
+  if (!same)
+    return bk::plan_fail(BK_ERR_UNSUPPORTED,
+                         "bk_plan_bind_box: the tables are not those of the plan's box");
+  const auto span = [](const uint32_t *t, size_t words) {
+    const uintptr_t lo = reinterpret_cast<uintptr_t>(t);
+    return std::make_pair(lo, t ? lo + 4 * words : lo);
+  };
+  const uint32_t *pairs = c.npairs ? d_pairs : nullptr;
+  bk::bind_box(p->id, {d_adj, pairs, d_img_off, d_img,
+                       {span(d_adj, (size_t)nbricks * 27), span(pairs, 2 * (size_t)c.npairs),
+                        span(d_img_off, (size_t)nbricks + 1), span(d_img, c.npairs)}});
+  return BK_OK;
+}
+
+int bk_plan_unbind_box(bk_plan p) {
+  if (!p) return bk::plan_fail(BK_ERR_ARG, "bk_plan_unbind_box: null plan");
+  bk::unbind_box(p->id);
   return BK_OK;
 }
 

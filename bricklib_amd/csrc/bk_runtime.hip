@@ -303,16 +303,26 @@ class SweepSplit {
   }
 };
 
+// Whether a sequence sweeps a declared box whose tables it uses are bound to it.
+bool box_path(const bk_sweep_desc *d, const uint32_t *pairs, uint32_t npairs, int nsweeps,
+              int ghost_iters, const uint32_t *img_off, const uint32_t *img) {
+  if (nsweeps <= 2 || ghost_iters != 1 || !d->plan || d->layout != BK_LAYOUT_8x8x8) return false;
+  const bk::PlanView P = bk::plan_view(d->plan);
+  return P.shape == BK_PLAN_QUAD && P.box_ids && P.box_npairs == npairs &&
+         bk::box_bound(P, d->d_adj, pairs, img_off, img);
+}
+
 // Enqueue the ping-pong sequence of bk_sweeps on stream s.
 // The ping-pong sequence: before sweep t the ghost bricks of its input are
 // refreshed when t % ghost_iters == 0; sweep t covers the desc's brick list
 // (or plan) when it is the last of its refresh group or of the sequence,
 // and the `all` list (or plan) -- every brick of the padded grid, ghosts
 // included -- otherwise.  ghost_iters == 1 is the refresh-every-sweep loop.
+// boxed: box_path() of the same arguments.
 hipError_t enqueue_sweeps(const bk_sweep_desc *d, const uint32_t *pairs, uint32_t npairs,
                           int nsweeps, int ghost_iters, const uint32_t *all, uint32_t nall,
                           bk_plan all_plan, const uint32_t *img_off, const uint32_t *img,
-                          hipStream_t s) {
+                          bool boxed, hipStream_t s) {
   bk::SweepLaunch L;
   to_launch(d, L);
   // fused refresh: the input's ghosts once, then every sweep also writes
@@ -328,38 +338,36 @@ hipError_t enqueue_sweeps(const bk_sweep_desc *d, const uint32_t *pairs, uint32_
   // point FP64 160^3 37.0 (25.5) / 21.6 (20.7), 125-point FP64 160^3 48.9 /
   // 34.1, 13-point FP32 of 9x7x8 bricks 16.1 (10.7) / 7.0 (6.7).  Stencils of radius 1 take
   // several sweeps per pass besides; the last sweep runs by itself.
-  if (nsweeps > 2 && ghost_iters == 1 && d->plan && d->layout == BK_LAYOUT_8x8x8) {
+  if (boxed) {
     const bk::PlanView P = bk::plan_view(d->plan);
-    if (P.shape == BK_PLAN_QUAD && P.box_ids && P.box_npairs == npairs) {
-      const bool many = bk::steps_fit(L, P);
-      float cost[5] = {};
-      if (many) bk::steps_costs(L, P, cost);
-      SweepSplit split(nsweeps - 1, cost);
-      bool fwd = true, fresh = false;  // fresh: the input's ghost bricks are up to date
-      for (int left = nsweeps; left; fwd = !fwd) {
-        const int ts = left == 1 || !many ? 1 : split.next();
-        left -= ts;
-        L.in = fwd ? d->d_in : d->d_out;
-        L.in_step = fwd ? d->in_step : d->out_step;
-        L.out = fwd ? d->d_out : const_cast<void *>(d->d_in);
-        L.out_step = fwd ? d->out_step : d->in_step;
-        hipError_t e = hipSuccess;
-        if (ts > 1) {
-          e = bk::launch_star_steps(L, P, ts, s);
-        } else {
-          if (left == 0 && npairs && !fresh)
-            e = bk::launch_ghost_refresh(const_cast<void *>(L.in), L.in_step * es, 512 * es,
-                                         pairs, npairs, s);
-          L.adj = left && P.box_adj ? P.box_adj : d->d_adj;
-          L.img_off = left <= 1 ? img_off : nullptr;
-          L.img = left <= 1 ? img : nullptr;
-          if (e == hipSuccess) e = launch_sweep(L, d->plan, s);
-          fresh = L.img_off != nullptr;
-        }
-        if (e != hipSuccess) return e;
+    const bool many = bk::steps_fit(L, P);
+    float cost[5] = {};
+    if (many) bk::steps_costs(L, P, cost);
+    SweepSplit split(nsweeps - 1, cost);
+    bool fwd = true, fresh = false;  // fresh: the input's ghost bricks are up to date
+    for (int left = nsweeps; left; fwd = !fwd) {
+      const int ts = left == 1 || !many ? 1 : split.next();
+      left -= ts;
+      L.in = fwd ? d->d_in : d->d_out;
+      L.in_step = fwd ? d->in_step : d->out_step;
+      L.out = fwd ? d->d_out : const_cast<void *>(d->d_in);
+      L.out_step = fwd ? d->out_step : d->in_step;
+      hipError_t e = hipSuccess;
+      if (ts > 1) {
+        e = bk::launch_star_steps(L, P, ts, s);
+      } else {
+        if (left == 0 && npairs && !fresh)
+          e = bk::launch_ghost_refresh(const_cast<void *>(L.in), L.in_step * es, 512 * es,
+                                       pairs, npairs, s);
+        L.adj = left && P.box_adj ? P.box_adj : d->d_adj;
+        L.img_off = left <= 1 ? img_off : nullptr;
+        L.img = left <= 1 ? img : nullptr;
+        if (e == hipSuccess) e = launch_sweep(L, d->plan, s);
+        fresh = L.img_off != nullptr;
       }
-      return hipSuccess;
+      if (e != hipSuccess) return e;
     }
+    return hipSuccess;
   }
   for (int t = 0; t < nsweeps; ++t) {
     const bool fwd = (t % 2) == 0;
@@ -537,12 +545,14 @@ int bk_alloc_async(size_t bytes, void **d_ptr, bk_stream s) {
 
 int bk_free_async(void *d_ptr, bk_stream s) {
   if (!d_ptr) return BK_OK;
+  bk::device_freed(d_ptr);
   BK_HIP(hipFreeAsync(d_ptr, S(s)));
   return BK_OK;
 }
 
 int bk_free(void *d_ptr) {
   if (!d_ptr) return BK_OK;
+  bk::device_freed(d_ptr);
   BK_HIP(hipFree(d_ptr));
   return BK_OK;
 }
@@ -550,6 +560,7 @@ int bk_free(void *d_ptr) {
 int bk_memcpy_h2d(void *d_dst, const void *h_src, size_t bytes, bk_stream s) {
   if (bytes == 0) return BK_OK;
   if (!d_dst || !h_src) return fail(BK_ERR_ARG, "bk_memcpy_h2d: null pointer");
+  bk::device_written(d_dst, bytes);
   BK_HIP(hipMemcpyAsync(d_dst, h_src, bytes, hipMemcpyHostToDevice, S(s)));
   BK_HIP(hipStreamSynchronize(S(s)));
   return BK_OK;
@@ -566,6 +577,7 @@ int bk_memcpy_d2h(void *h_dst, const void *d_src, size_t bytes, bk_stream s) {
 int bk_memcpy_d2d(void *d_dst, const void *d_src, size_t bytes, bk_stream s) {
   if (bytes == 0) return BK_OK;
   if (!d_dst || !d_src) return fail(BK_ERR_ARG, "bk_memcpy_d2d: null pointer");
+  bk::device_written(d_dst, bytes);
   BK_HIP(hipMemcpyAsync(d_dst, d_src, bytes, hipMemcpyDeviceToDevice, S(s)));
   return BK_OK;
 }
@@ -578,6 +590,7 @@ int bk_stream_copy(void *d_dst, const void *d_src, size_t bytes, bk_stream s) {
   const char *a = static_cast<const char *>(d_src);
   const char *b = static_cast<const char *>(d_dst);
   if (a < b + bytes && b < a + bytes) return fail(BK_ERR_ARG, "bk_stream_copy: ranges overlap");
+  bk::device_written(d_dst, bytes);
   BK_HIP(bk::launch_stream_copy(d_dst, d_src, bytes, S(s)));
   return BK_OK;
 }
@@ -608,6 +621,7 @@ int bk_valu_probe(int dtype, int chains, int waves_per_simd, uint32_t iters, voi
 int bk_zero(void *d_dst, size_t bytes, bk_stream s) {
   if (bytes == 0) return BK_OK;
   if (!d_dst) return fail(BK_ERR_ARG, "bk_zero: null pointer");
+  bk::device_written(d_dst, bytes);
   BK_HIP(bk::launch_zero(d_dst, bytes, S(s)));
   return BK_OK;
 }
@@ -797,9 +811,10 @@ int sweeps_impl(const bk_sweep_desc *d, const uint32_t *d_pairs, uint32_t npairs
                 int ghost_iters, const uint32_t *d_all, uint32_t nall, bk_plan all_plan,
                 const uint32_t *img_off, const uint32_t *img, int use_graph, hipStream_t s) {
   if (nsweeps == 0 || desc_empty(d)) return BK_OK;
+  const bool boxed = box_path(d, d_pairs, npairs, nsweeps, ghost_iters, img_off, img);
   if (!use_graph) {
     BK_HIP(enqueue_sweeps(d, d_pairs, npairs, nsweeps, ghost_iters, d_all, nall, all_plan,
-                          img_off, img, s));
+                          img_off, img, boxed, s));
     return BK_OK;
   }
   // key: every argument that shapes the captured launches
@@ -834,6 +849,7 @@ int sweeps_impl(const bk_sweep_desc *d, const uint32_t *d_pairs, uint32_t npairs
   put(&apid, sizeof(apid));
   put(&img_off, sizeof(img_off));
   put(&img, sizeof(img));
+  put(&boxed, sizeof(boxed));
   auto &gc = graphs();
   std::lock_guard<std::mutex> lock(gc.mu);
   if (!gc.exec.find(key)) {
@@ -847,7 +863,7 @@ int sweeps_impl(const bk_sweep_desc *d, const uint32_t *d_pairs, uint32_t npairs
     }
     BK_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
     hipError_t e = enqueue_sweeps(d, d_pairs, npairs, nsweeps, ghost_iters, d_all, nall,
-                                  all_plan, img_off, img, cs);
+                                  all_plan, img_off, img, boxed, cs);
     hipGraph_t g = nullptr;
     hipError_t e2 = hipStreamEndCapture(cs, &g);
     if (e != hipSuccess) {

@@ -305,19 +305,37 @@ int bk_plan_build_host(const uint32_t *h_adj, uint32_t nbricks,
  * Checked against h_adj, the adjacency the plan was built on: every
  * neighbour of every box brick must be the brick of the wrapped box, or a
  * ghost brick that a pair makes its copy -- BK_ERR_UNSUPPORTED otherwise, and
- * the plan stays as it was.  A sequence of sweeps over such a quad plan that
- * refreshes with these pairs (bk_sweeps, bk_sweeps_fused called with npairs
- * pairs) then reads the periodic images themselves, refreshes only what its
- * last sweep leaves, and may take several sweeps per pass.  Both fields' box
- * bricks then hold what single sweeps leave in them, bit for bit, and so do
- * the ghost bricks of the input field of the last sweep (of both fields, for
- * bk_sweeps_fused); the ghost bricks of a bk_sweeps result are not refreshed
- * and hold older values.  No counterpart in the reference.  Allocates device
- * memory (the ids and, with pairs, an adjacency of its own), filled on s when
- * the call returns; a capture of s is left as it is. */
+ * the plan stays as it was.  No counterpart in the reference.  Allocates
+ * device memory (the ids, two words a brick and, with pairs, an adjacency of
+ * its own), filled on s when the call returns; a capture of s is left as it
+ * is.  Sequences use the box only with device tables bound to it:
+ *
+ * bk_plan_bind_box compares device tables with the declared box (on s, which
+ * it waits for): d_adj, the npairs pairs of d_pairs, and with d_img_off and
+ * d_img (both or neither NULL) the ghost-image tables of bk_sweeps_fused.
+ * BK_ERR_UNSUPPORTED where they do not say the same.  A
+ * sequence of sweeps over such a quad plan called with tables bound to it
+ * (bk_sweeps, bk_sweeps_fused) then reads the periodic
+ * images themselves, refreshes only what its last sweep leaves, and may take
+ * several sweeps per pass.  Both fields' box bricks then hold what single
+ * sweeps leave in them, bit for bit, and so do the ghost bricks of the input
+ * field of the last sweep (of both fields, for bk_sweeps_fused); the ghost
+ * bricks of a bk_sweeps result are not refreshed and hold older values.
+ * Sequences with any other table refresh with that table before every sweep.
+ * Up to four sets of tables per plan; the oldest makes way.
+ *
+ * A binding lasts until the library writes into one of its tables
+ * (bk_memcpy_h2d, bk_memcpy_d2d, bk_stream_copy, bk_zero), frees one, or
+ * bk_plan_unbind_box ends all of the plan's: call it before tables are
+ * written by other means.  A capture of the caller's keeps the form that its
+ * sequences had when they were captured. */
 int bk_plan_set_box(bk_plan plan, const uint32_t *h_adj, const long nb[3],
                     const uint32_t *h_ids, const uint32_t *h_pairs, uint32_t npairs,
                     bk_stream s);
+int bk_plan_bind_box(bk_plan plan, const uint32_t *d_adj, const uint32_t *d_pairs,
+                     uint32_t npairs, const uint32_t *d_img_off, const uint32_t *d_img,
+                     bk_stream s);
+int bk_plan_unbind_box(bk_plan plan);
 int bk_plan_query(bk_plan plan, uint32_t *nunits, uint32_t *kcol, int *shape,
                   uint32_t *ncovered);
 /* Copy the plan's arrays to the host (any pointer may be NULL):
