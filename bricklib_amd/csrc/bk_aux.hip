@@ -293,13 +293,15 @@ __device__ __forceinline__ void block_reduce(double (&v)[NV], const bool (&is_ma
 }
 
 // A block's partials to part[block][NV]; the last block combines them all into
-// out[0 .. NV).  *count holds the blocks that are done; it wraps back to 0
-// with the last one.
+// out[0 .. NV).  *count rises by kReduceBlocks per launch, whatever its grid:
+// by one a block and by what is left over with block 0, and the block that
+// completes a multiple is the last.  Launches that overlap on one count spoil
+// each other's results, but leave a multiple for those after them.
 template <int NV>
 __device__ __forceinline__ void finish(double (&v)[NV], const bool (&is_max)[NV], double *part,
                                        uint32_t *count, double *out) {
   __shared__ double sh[NV][kReduceThreads / 64];
-  __shared__ uint32_t last;
+  __shared__ bool last;
   block_reduce<NV>(v, is_max, sh);
   if (threadIdx.x == 0) {
 #pragma unroll
@@ -309,10 +311,11 @@ __device__ __forceinline__ void finish(double (&v)[NV], const bool (&is_max)[NV]
     // the partials, written through to memory every XCD reads, are there
     // before the count says so (a fence would write all of L2 back)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    last = atomicInc(count, gridDim.x - 1);
+    const uint32_t by = blockIdx.x ? 1u : kReduceBlocks + 1u - gridDim.x;
+    last = (atomicAdd(count, by) + by) % kReduceBlocks == 0;
   }
   __syncthreads();
-  if (last != gridDim.x - 1) return;
+  if (!last) return;
 #pragma unroll
   for (int q = 0; q < NV; ++q) v[q] = 0.0;
   for (uint32_t t = threadIdx.x; t < gridDim.x; t += kReduceThreads) {

@@ -155,7 +155,7 @@ hipError_t launch_fill_uniform(int layout, int dtype, void *dat, size_t step,
                                const long nb[3], int ghost, uint64_t seed,
                                double lo, double hi, hipStream_t s);
 // Deterministic FP64 reductions; `scratch` holds kReduceBlocks*nout doubles
-// (the blocks' partials), *count is 0 and returns to 0.  Results land in
+// (the blocks' partials), *count starts at 0 and belongs to them.  Results land in
 // out[0 .. nout) (device memory, or pinned host memory).
 constexpr int kReduceBlocks = 256;
 hipError_t launch_field_stats(int dtype, const void *dat, size_t step,

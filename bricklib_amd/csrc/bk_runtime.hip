@@ -64,7 +64,7 @@ int dt_size(int dt) { return dt == BK_F64 ? 8 : dt == BK_F32 ? 4 : dt == BK_BF16
 // results go straight to pinned host memory: no copy after the kernel.
 struct ReduceScratch {
   double *part = nullptr;     // the blocks' partials
-  uint32_t *count = nullptr;  // blocks done, 0 between calls
+  uint32_t *count = nullptr;  // blocks done, a multiple of kReduceBlocks between calls
   double *host = nullptr;     // results, pinned
 };
 struct Scratch {
@@ -109,9 +109,9 @@ int get_scratch(ReduceScratch **p) {
 // GPU at its own address, held until the process ends (6 KiB).  Its size does
 // not depend on the input: at most kReduceBlocks blocks each write their own
 // three partials and the last one reads all of theirs, so every slot that a
-// call reads is rewritten by it.  Behind them the count of blocks done: 0 when the
-// library is loaded, and again after every call.  Calls that overlap on one
-// GPU share the array and race.
+// call reads is rewritten by it.  Behind them the count of blocks done, 0 when
+// the library is loaded.  Calls that overlap on one GPU share the array and
+// spoil each other's results, not those of later calls.
 constexpr size_t kStaticScratchDoubles = (size_t)bk::kReduceBlocks * 3 + 1;
 static __device__ __align__(256) double scratch[kStaticScratchDoubles];
 

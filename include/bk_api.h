@@ -661,8 +661,9 @@ int bk_field_stats(int dtype, const void *d_dat, size_t step,
  * the blocks' partials live in a static 6 KiB device array of the library
  * (one per GPU, whatever the input size) and the three results are written
  * to device memory d_out[3], stream-ordered on s with no host wait.  Calls
- * that overlap on one GPU share that array and race: order them on one
- * stream (or wait between them). */
+ * that overlap on one GPU share that array and spoil each other's results
+ * (not those of later calls): order them on one stream (or wait between
+ * them). */
 int bk_field_stats_noalloc(int dtype, const void *d_dat, size_t step,
                            const uint32_t *d_list, uint32_t nlist,
                            size_t brick_elems, double *d_out, bk_stream s);
