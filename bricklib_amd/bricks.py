@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import ctypes as C
 import struct
+import threading
 from dataclasses import dataclass, field
 
 import numpy as np
@@ -315,6 +316,7 @@ class Plan:
         self.shape = shape
         self.kcol = int(kcol)
         self.boxed = False  # set_box ran
+        self.lock = threading.Lock()  # one declaration at a time
         self.tables: set = set()  # device tables that sequences came with (_declare_box)
         nu, nc = C.c_uint32(), C.c_uint32()
         check(load().bk_plan_query(_vp(self.handle), C.byref(nu), None, None, C.byref(nc)))
@@ -526,13 +528,20 @@ class PeriodicGrid:
             return
         if not plan.boxed and not any(plan is p for p in self._plans.values()):
             return
-        plan.tables.add(tables)
-        try:
-            if not plan.boxed:
-                plan.set_box(self.info, self.nb, self.interior, self.pairs, stream)
-            plan.bind_box(*tables, stream=stream)
-        except _lib.BrickError:  # not a periodic box (changed tables): one sweep per pass
-            pass
+        with plan.lock:
+            if tables in plan.tables:
+                return
+            try:
+                if not plan.boxed:
+                    plan.set_box(self.info, self.nb, self.interior, self.pairs, stream)
+                plan.bind_box(*tables, stream=stream)
+            except _lib.BrickError as e:
+                if e.code == _lib.BK_ERR_NOMEM:
+                    return  # one sweep per pass now; the next sequence tries again
+                if e.code != _lib.BK_ERR_UNSUPPORTED:
+                    raise
+                # not a periodic box (changed tables): one sweep per pass with them
+            plan.tables.add(tables)
 
     @property
     def ghost_images(self):

@@ -645,6 +645,7 @@ int bk_plan_set_box(bk_plan p, const uint32_t *h_adj, const long nb[3], const ui
   if (e == hipSuccess) e = hipStreamSynchronize(own);
   if (e != hipSuccess) {
     (void)hipFree(d);
+    (void)hipGetLastError();  // the next launch is not to report it
     std::string m = std::string("bk_plan_set_box: ") + hipGetErrorString(e);
     return bk::plan_fail(e == hipErrorOutOfMemory ? BK_ERR_NOMEM : BK_ERR_HIP, m.c_str());
   }

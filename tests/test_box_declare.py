@@ -1,0 +1,81 @@
+"""The declaration ahead of a sequence of sweeps: what each status of the
+library makes of it (host logic, no device)."""
+import threading
+from types import SimpleNamespace
+
+import numpy as np
+import pytest
+
+from bricklib_amd import _lib
+from bricklib_amd.bricks import Plan, PeriodicGrid
+
+
+class FakePlan:
+    """A Plan whose library calls end with the given statuses in turn."""
+
+    def __init__(self, *codes):
+        self.shape, self.boxed, self.handle = "quad", False, None
+        self.lock, self.tables = threading.Lock(), set()
+        self.codes, self.calls = list(codes), 0
+
+    def _end(self):
+        self.calls += 1
+        code = self.codes.pop(0) if self.codes else 0
+        if code:
+            raise _lib.BrickError(code, "planted")
+
+    def set_box(self, *args, **kw):
+        self._end()
+        self.boxed = True
+
+    def bind_box(self, *args, **kw):
+        self._end()
+
+
+def _grid(plan):
+    g = PeriodicGrid.__new__(PeriodicGrid)
+    g.info, g.d_pairs = SimpleNamespace(dptr=4096), None
+    g.pairs = np.empty(0, np.uint32)
+    g.interior, g.nb, g._plans = np.arange(8, dtype=np.uint32), (2, 2, 2), {"p": plan}
+    return g
+
+
+def test_declared_once():
+    p = FakePlan()
+    g = _grid(p)
+    for _ in range(3):
+        g._declare_box(p)
+    assert p.boxed and p.calls == 2
+
+
+@pytest.mark.parametrize("at", [0, 1])
+def test_not_a_box_is_remembered(at):
+    p = FakePlan(*[0] * at, _lib.BK_ERR_UNSUPPORTED)
+    g = _grid(p)
+    for _ in range(3):
+        g._declare_box(p)
+    assert p.calls == at + 1
+
+
+@pytest.mark.parametrize("at", [0, 1])
+def test_out_of_memory_is_tried_again(at):
+    p = FakePlan(*[0] * at, _lib.BK_ERR_NOMEM)
+    g = _grid(p)
+    g._declare_box(p)  # the sequence goes on by single sweeps
+    assert p.boxed == bool(at)
+    g._declare_box(p)
+    assert p.boxed and p.calls == 3
+    g._declare_box(p)
+    assert p.calls == 3
+
+
+@pytest.mark.parametrize("code", [_lib.BK_ERR_HIP, _lib.BK_ERR_ARG])
+def test_other_errors_are_raised(code):
+    p = FakePlan(code)
+    with pytest.raises(_lib.BrickError) as e:
+        _grid(p)._declare_box(p)
+    assert e.value.code == code
+
+
+def test_plan_has_what_the_declaration_uses():
+    assert {"set_box", "bind_box", "unbind_box"} <= set(dir(Plan))
