@@ -526,7 +526,7 @@ class PeriodicGrid:
                   self.npairs, *images)
         if tables in plan.tables or plan.shape != "quad":
             return
-        if not plan.boxed and not any(plan is p for p in self._plans.values()):
+        if not plan.boxed and not any(plan is p for p in list(self._plans.values())):
             return
         with plan.lock:
             if tables in plan.tables:

@@ -1,5 +1,6 @@
 """The declaration ahead of a sequence of sweeps: what each status of the
 library makes of it (host logic, no device)."""
+import sys
 import threading
 from types import SimpleNamespace
 
@@ -75,6 +76,39 @@ def test_other_errors_are_raised(code):
     with pytest.raises(_lib.BrickError) as e:
         _grid(p)._declare_box(p)
     assert e.value.code == code
+
+
+def test_while_another_thread_adds_plans():
+    """grid.plan() of another thread grows the table that is searched."""
+    p = FakePlan()
+    g = _grid(p)
+    g._plans = {("other", q): object() for q in range(500)}
+    stop, errors = threading.Event(), []
+
+    def add():
+        q = 0
+        while not stop.is_set():
+            g._plans[("more", q % 4000)] = object()
+            q += 1
+            if q % 4000 == 0:
+                for r in range(4000):
+                    del g._plans[("more", r)]
+
+    was = sys.getswitchinterval()
+    sys.setswitchinterval(1e-6)
+    t = threading.Thread(target=add)
+    t.start()
+    try:
+        for _ in range(300):
+            try:
+                g._declare_box(p)
+            except RuntimeError as e:
+                errors.append(e)
+    finally:
+        stop.set()
+        t.join()
+        sys.setswitchinterval(was)
+    assert not errors and p.calls == 0
 
 
 def test_plan_has_what_the_declaration_uses():
