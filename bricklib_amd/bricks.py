@@ -766,7 +766,8 @@ def sweeps(st: Stencil, a: Brick, b: Brick, grid: PeriodicGrid, nsweeps: int,
     pairs = grid.d_pairs.ptr if (refresh and grid.d_pairs is not None) else None
     npairs = grid.npairs if refresh else 0
     if (nsweeps > 3 and keep[-1] is not None and ghost_iters == 1
-            and (npairs or st.kind in STEP_STENCILS) and hasattr(grid, "_declare_box")):
+            and (npairs or st.kind in STEP_STENCILS) and hasattr(grid, "_declare_box")
+            and npairs == grid.npairs):  # (ghost bricks left alone are boundary values)
         grid._declare_box(keep[-1], stream, fused)
     if fused:
         if ghost_iters != 1:

@@ -113,3 +113,25 @@ def test_while_another_thread_adds_plans():
 
 def test_plan_has_what_the_declaration_uses():
     assert {"set_box", "bind_box", "unbind_box"} <= set(dir(Plan))
+
+
+@pytest.mark.parametrize("name", ["7pt", "25pt"])
+@pytest.mark.parametrize("ghosts,refresh,n,want", [
+    (True, False, 9, False),  # ghost bricks as boundary values: no periodic box
+    (True, True, 9, True), (True, True, 3, False), (False, True, 9, None), (False, False, 9, None)])
+def test_which_sequences_declare(monkeypatch, name, ghosts, refresh, n, want):
+    """Only sequences that may use the box pay for its declaration."""
+    from bricklib_amd import bricks
+    from bricklib_amd.stencils import Stencil
+    p = FakePlan()
+    g = _grid(p)
+    asked = []
+    g._declare_box = lambda *a, **k: asked.append(a)
+    if ghosts:
+        g.d_pairs, g.pairs = SimpleNamespace(ptr=8192), np.zeros(2, np.uint32)
+    monkeypatch.setattr(bricks, "_desc", lambda *a, **k: a[4].append(p) or _lib.bk_sweep_desc())
+    monkeypatch.setattr(bricks, "load", lambda: SimpleNamespace(bk_sweeps=lambda *a: 0))
+    f = SimpleNamespace(dtype=0)
+    bricks.sweeps(Stencil.make(name, seed=1), f, f, g, n, refresh=refresh)
+    # a wrapped box has nothing to refresh: only what takes several sweeps per pass
+    assert bool(asked) == (name == "7pt" if want is None else want)
