@@ -16,6 +16,7 @@
 #include <cstdio>
 #include <map>
 #include <mutex>
+#include <set>
 #include <vector>
 
 #include "bk_api.h"
@@ -74,7 +75,41 @@ namespace {
 
 int fail(int code, const char *msg) { return bk::plan_fail(code, msg); }
 
+// The arenas there are, for block_end().
+struct Arenas {
+  std::mutex mu;
+  std::set<bk_arena_s *> all;
+};
+Arenas &arenas() {
+  static Arenas *a = new Arenas;  // arenas may be destroyed at exit
+  return *a;
+}
+
 }  // namespace
+
+namespace bk {
+uintptr_t block_end(const void *p) {
+  char *at = static_cast<char *>(const_cast<void *>(p));
+  {
+    std::lock_guard<std::mutex> lock(arenas().mu);
+    for (bk_arena_s *a : arenas().all) {
+      std::lock_guard<std::mutex> own(a->mu);
+      auto it = a->live.upper_bound(at);
+      if (it == a->live.begin()) continue;
+      --it;
+      if (at < it->first + it->second.size)
+        return reinterpret_cast<uintptr_t>(it->first + it->second.size);
+    }
+  }
+  hipDeviceptr_t base = nullptr;
+  size_t bytes = 0;
+  if (hipMemGetAddressRange(&base, &bytes, const_cast<void *>(p)) != hipSuccess) {
+    (void)hipGetLastError();
+    return UINTPTR_MAX;
+  }
+  return reinterpret_cast<uintptr_t>(base) + bytes;
+}
+}  // namespace bk
 
 extern "C" {
 
@@ -86,12 +121,20 @@ int bk_arena_create(size_t slab_bytes, size_t capacity, bk_arena *out) {
   (void)hipGetDevice(&a->device);
   a->slab_bytes = round_up(slab_bytes);
   a->capacity = capacity;
+  {
+    std::lock_guard<std::mutex> lock(arenas().mu);
+    arenas().all.insert(a);
+  }
   *out = a;
   return BK_OK;
 }
 
 int bk_arena_destroy(bk_arena a) {
   if (!a) return BK_OK;
+  {
+    std::lock_guard<std::mutex> lock(arenas().mu);
+    arenas().all.erase(a);
+  }
   for (auto &s : a->slabs) {
     bk::device_freed(s.base);
     (void)hipFree(s.base);

@@ -123,22 +123,25 @@ int hipfail(hipError_t e, const char *what) {
     if (e_ != hipSuccess) return hipfail(e_, #call);  \
   } while (0)
 
-// No two requests' fields overlap, as far as the host can tell: a field spans
-// the bricks of its plan's adjacency, or as many as its list and pairs have.
+// No two requests' fields overlap: a field spans the bricks of its plan's
+// adjacency; without a plan, whose list may hold any ids, all up to the end of
+// its arena block or allocation (24 requests: 48 looked up in 6 us).
 bool fields_apart(const bk_batch_req *reqs, uint32_t n, Span *span) {
   uint32_t m = 0;
   for (uint32_t r = 0; r < n; ++r) {
     const bk_batch_req &q = reqs[r];
-    uint64_t bricks = (uint64_t)q.nlist + q.npairs;
-    if (q.plan) bricks = std::max<uint64_t>(bricks, bk::plan_view(q.plan).nbricks);
-    const uintptr_t bytes = bricks * q.step * bk_dtype_size(q.dtype);
-    const uintptr_t lo = reinterpret_cast<uintptr_t>(std::min(q.d_f0, q.d_f1));
-    const uintptr_t hi = reinterpret_cast<uintptr_t>(std::max(q.d_f0, q.d_f1));
-    if (lo + bytes > hi) {  // interleaved
-      span[m++] = {lo, hi + bytes};
+    auto field = [&](const void *p) {
+      const uintptr_t at = reinterpret_cast<uintptr_t>(p);
+      return Span{at, q.plan ? at + (uintptr_t)bk::plan_view(q.plan).nbricks * q.step *
+                                        bk_dtype_size(q.dtype)
+                             : bk::block_end(p)};
+    };
+    const Span lo = field(std::min(q.d_f0, q.d_f1)), hi = field(std::max(q.d_f0, q.d_f1));
+    if (lo.second > hi.first) {  // interleaved, or of one allocation
+      span[m++] = {lo.first, std::max(lo.second, hi.second)};
     } else {
-      span[m++] = {lo, lo + bytes};
-      span[m++] = {hi, hi + bytes};
+      span[m++] = lo;
+      span[m++] = hi;
     }
   }
   std::sort(span, span + m);

@@ -64,6 +64,9 @@ bool box_bound(const PlanView &P, const uint32_t *adj, const uint32_t *pairs,
 // are no longer bound.
 void device_written(const void *p, size_t bytes);
 void device_freed(void *p);
+// The end of the arena block or else the allocation that holds p (UINTPTR_MAX
+// where the runtime knows none).
+uintptr_t block_end(const void *p);
 // Keep cube sweeps over the plan to the marching form, the one the batched
 // kernel runs (the tuner times it for them).
 void plan_march(bk_plan_s *p);
