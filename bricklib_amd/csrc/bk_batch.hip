@@ -377,7 +377,7 @@ int bk_batch_set(bk_batch b, const bk_batch_req *reqs, uint32_t n, bk_stream str
       sg.mask = P.mask;
       sg.nitems = P.nunits;
       sg.kcol = P.kcol;
-      b->h_sweep[g]->levels = std::max(b->h_sweep[g]->levels, P.kcol);
+      b->h_sweep[g]->levels = std::max(b->h_sweep[g]->levels, P.longest);
       if (q.stencil == BK_CUBE125) cube_bricks[q.dtype] += nbricks;
     } else {
       sg.items = q.d_list;

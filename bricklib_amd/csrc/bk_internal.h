@@ -44,6 +44,7 @@ struct PlanView {
   const uint32_t *mask;
   const uint32_t *flat;
   const uint32_t *start;
+  uint32_t longest;  // levels of the longest unit, at most kcol
   uint32_t nbricks;  // bricks of the adjacency the plan was built on
   uint64_t id;       // unique per plan (graph-cache key), never 0
   // periodic box (bk_plan_set_box): its brick ids in grid order, or null
@@ -125,7 +126,7 @@ struct BatchSeg {
 
 struct BatchTable {
   uint32_t nsegs;
-  uint32_t levels;  // levels of the longest plan (cube, block form)
+  uint32_t levels;  // levels of the longest unit (cube, block form)
   uint32_t prefix[kBatchMaxSegs + 1];  // items before segment s
   BatchSeg seg[kBatchMaxSegs];
 };

@@ -36,6 +36,7 @@ struct bk_plan_s {
   int shape = 1;
   uint32_t kcol = 1;
   uint32_t nunits = 0;
+  uint32_t longest = 0;  // levels of the longest unit
   uint32_t ncovered = 0;
   uint32_t *d_arrays = nullptr;  // one allocation holding the arrays below
   uint32_t *d_anchor = nullptr;  // [nunits] level-0 anchor
@@ -80,6 +81,7 @@ const PlanView plan_view(const bk_plan_s *p) {
   v.mask = p->d_mask;
   v.flat = p->d_flat;
   v.start = p->d_start;
+  v.longest = p->longest;
   v.nbricks = p->nbricks;
   v.id = p->id;
   v.box_ids = p->d_box.load(std::memory_order_acquire);  // before what goes with it
@@ -499,6 +501,7 @@ int bk_plan_create(const uint32_t *h_adj, uint32_t nbricks, const uint32_t *h_li
   p->kcol = kcol;
   p->nunits = (uint32_t)A.anchor.size();
   p->ncovered = (uint32_t)A.flat.size();
+  for (uint32_t l : A.len) p->longest = std::max(p->longest, l);
   p->nbricks = nbricks;
   p->id = g_next_plan_id.fetch_add(1);
   (void)hipGetDevice(&p->device);  // the current device owns the arrays below
