@@ -8,7 +8,7 @@
 // the result; the sweeps in between never reach memory.
 //
 // One wave owns a strip of J rows (j) of up to 7 bricks along i and marches
-// along k.  Lane l holds one cell of every row (V = 1).  The 64 cells of a row
+// along k.  Lane l holds one cell of every row.  The 64 cells of a row
 // are the strip's and kHalo halo cells a side, laid round the wave as a ring --
 // strip first, right halo, left halo -- so the i-taps are one-lane wave
 // rotations (DPP) and groups of lanes fall on whole brick rows.  For each sweep
@@ -36,8 +36,8 @@
 // sweep against 0.393 for one sweep per pass (FP32 0.086 against 0.203, BF16
 // 0.089 against 0.117).  Three sweeps per pass: FP64 0.177, FP32 0.107 ms per
 // sweep.  Found on the way: with the strip from the left halo on (lanes
-// across brick edges) and one store per row 0.154; V = 2 in FP32 (fewer
-// rotations, two waves per SIMD instead of three) no faster; issuing the
+// across brick edges) and one store per row 0.154; two cells a lane in FP32
+// (fewer rotations, two waves per SIMD instead of three) no faster; issuing the
 // first five taps of the next row among the last ones of this row, two rows
 // per scheduling group, or loads two planes ahead no faster.
 #include <algorithm>
@@ -78,12 +78,6 @@ struct StepArgs {
   A c[13];
 };
 
-// V adjacent cells of a lane
-template <class A, int V>
-struct Cells {
-  A v[V];
-};
-
 // The value of the next (UP) or previous lane, the wave a ring of 64.
 template <bool UP>
 __device__ __forceinline__ uint32_t wave_turn32(uint32_t x) {
@@ -116,28 +110,27 @@ __device__ __forceinline__ double row_next(double x) {
   return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
-// a lane's V cells from memory
-__device__ __forceinline__ void load_cells(const double *p, Cells<double, 1> &x) { x.v[0] = *p; }
-__device__ __forceinline__ void load_cells(const float *p, Cells<float, 1> &x) { x.v[0] = *p; }
-__device__ __forceinline__ void load_cells(const bf16 *p, Cells<float, 1> &x) {
-  x.v[0] = widen(*p);
-}
+// A cell of a plane.  (A struct: plain floats are allotted otherwise, and the
+// sequences of 7-point sweeps took 1 % longer, FP32 360x216x264 471 -> 475 us,
+// BF16 256^3 318 -> 322.)
+template <class A>
+struct Cell {
+  A v;
+};
 
-// what a store to T and the next sweep's load make of a sweep's values
+// what a store to T and the next sweep's load make of a sweep's value
 // (gfx950's conversion rounds as narrow() does: the same bits for all 2^32
 // inputs)
-template <class T, class A, int V>
-__device__ __forceinline__ void round_cells(Cells<A, V> &x) {
+template <class T, class A>
+__device__ __forceinline__ A rounded(A x) {
   if constexpr (std::is_same<T, bf16>::value) {
     typedef float f2 __attribute__((ext_vector_type(2)));
     typedef __bf16 h2 __attribute__((ext_vector_type(2)));
     f2 t;
-    t.x = x.v[0];
-    t.y = x.v[V - 1];
-    const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(t, h2));
-    x.v[0] = __uint_as_float(u << 16);
-    if (V > 1) x.v[V - 1] = __uint_as_float(u & 0xffff0000u);
+    t.x = t.y = x;
+    return __uint_as_float(__builtin_bit_cast(uint32_t, __builtin_convertvector(t, h2)) << 16);
   }
+  return x;
 }
 
 // Values of the lane `1` or `2` away in its group of four (quad_perm).
@@ -215,16 +208,14 @@ struct RowStore<float> {
   }
 };
 
-template <class T, int TS, int J, int FORM>
+template <class T, int TS, int FORM>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(2)))
 void star_steps(const StepArgs<T> a) {
   using A = typename acc_of<T>::type;
-  constexpr int V = 1;
-  using X = Cells<A, V>;
-  constexpr int NR = J + 2 * TS;  // rows of the input planes
-  static_assert(TS >= 1 && TS <= kHalo && TS <= J && (J == 4 || J == 8),
-                "the halo rows of a side lie in one brick");
+  using X = Cell<A>;
+  constexpr int J = 8, NR = J + 2 * TS;  // rows of the strip and of the input planes
+  static_assert(TS >= 1 && TS <= kHalo, "the halo cells of a row");
   const int lane = threadIdx.x & 63;
   // each wave's older input plane, rows 1 .. NR-2, a lane its own cells
   __shared__ X older_all[4 * (NR - 2) * 64];
@@ -238,15 +229,15 @@ void star_steps(const StepArgs<T> a) {
   const uint32_t seg = w / a.njw;
   if (jg >= a.njg) return;  // wave-uniform; nothing below synchronises waves
 
-  // the strip along i: bricks [c0, c1); lane l the cells l V of it, the last
+  // the strip along i: bricks [c0, c1); lane l cell l of it, the last
   // kHalo cells of the ring those before it (lanes past the right halo hold
   // further cells of the wrapped row, unused)
   const uint32_t c0 = a.nb0 * ch / a.nchunk, c1 = a.nb0 * (ch + 1) / a.nchunk;
   const uint32_t n0 = a.nb0 * 8, n1 = a.nb1 * 8, n2 = a.nb2 * 8;
-  const int off = lane * V < 64 * V - kHalo ? lane * V : (lane - 64) * V;
+  const int off = lane < 64 - kHalo ? lane : lane - 64;
   const uint32_t cell = (uint32_t)((int)(c0 * 8 + n0) + off) % n0;
   const uint32_t bi = cell >> 3, io = cell & 7;
-  const bool mine = (uint32_t)(lane * V) < (c1 - c0) * 8;
+  const bool mine = (uint32_t)lane < (c1 - c0) * 8;
   // rows: the strip's in brick row bj, the halo rows below and above in brick
   // rows bl and bh
   const uint32_t j0 = jg * J;
@@ -278,7 +269,7 @@ void star_steps(const StepArgs<T> a) {
   X ea[NR], eb[NR];  // the last input plane and the one arriving
   auto load_row = [&](int r, X(&e)[NR]) {
     const T *p = r < TS ? pl : (r < TS + J ? pc : ph);
-    load_cells(p + (r - TS) * 8, e[r]);
+    e[r].v = widen(p[(r - TS) * 8]);
   };
 #pragma unroll
   for (int r = 0; r < NR; ++r) load_row(r, eb);
@@ -288,13 +279,11 @@ void star_steps(const StepArgs<T> a) {
 
   X pa[TS][NR], pb[TS][NR];  // the two planes of sweeps 1 .. TS-1
 #pragma unroll
-  for (int r = 0; r < NR; ++r)
+  for (int r = 0; r < NR; ++r) {
+    ea[r].v = A(0);
 #pragma unroll
-    for (int q = 0; q < V; ++q) {
-      ea[r].v[q] = A(0);
-#pragma unroll
-      for (int s = 0; s < TS; ++s) pa[s][r].v[q] = pb[s][r].v[q] = A(0);
-    }
+    for (int s = 0; s < TS; ++s) pa[s][r].v = pb[s][r].v = A(0);
+  }
 
   // values as taps see them: of a kept plane, and of one just computed
   auto tap = [](A x) -> A {
@@ -302,35 +291,25 @@ void star_steps(const StepArgs<T> a) {
     else return x;
   };
   auto keep = [](X x) -> X {
-    if constexpr (FORM == kCondPos) {
-#pragma unroll
-      for (int q = 0; q < V; ++q) x.v[q] = relu_ref(x.v[q]);
-    }
+    if constexpr (FORM == kCondPos) x.v = relu_ref(x.v);
     return x;
   };
   // one sweep at one row: centre m, rows j+1 and j-1, planes k+1 and k-1
   auto point = [&](const X &m, const X &jp, const X &jm, const X &kp, const X &km) {
-    X t, o;
-#pragma unroll
-    for (int q = 0; q < V; ++q) t.v[q] = tap(m.v[q]);
-    const A next = wave_turn<true>(t.v[0]), prev = wave_turn<false>(t.v[V - 1]);
-#pragma unroll
-    for (int q = 0; q < V; ++q) {
-      A acc = a.c[0] * t.v[q];
-      acc = fmadd(a.c[1], q + 1 < V ? t.v[q + 1 < V ? q + 1 : q] : next, acc);
-      acc = fmadd(a.c[2], q > 0 ? t.v[q > 0 ? q - 1 : 0] : prev, acc);
-      acc = fmadd(a.c[3], tap(jp.v[q]), acc);
-      acc = fmadd(a.c[4], tap(jm.v[q]), acc);
-      acc = fmadd(a.c[5], tap(kp.v[q]), acc);
-      acc = fmadd(a.c[6], tap(km.v[q]), acc);
-      if constexpr (FORM != kStar) {
-        const bool sel = a.cond_mode == 0 ? (acc > A(0)) : (m.v[q] > a.theta);
-        acc = sel ? acc : -acc;
-      }
-      o.v[q] = acc;
+    const A t = tap(m.v);
+    const A next = wave_turn<true>(t), prev = wave_turn<false>(t);
+    A acc = a.c[0] * t;
+    acc = fmadd(a.c[1], next, acc);
+    acc = fmadd(a.c[2], prev, acc);
+    acc = fmadd(a.c[3], tap(jp.v), acc);
+    acc = fmadd(a.c[4], tap(jm.v), acc);
+    acc = fmadd(a.c[5], tap(kp.v), acc);
+    acc = fmadd(a.c[6], tap(km.v), acc);
+    if constexpr (FORM != kStar) {
+      const bool sel = a.cond_mode == 0 ? (acc > A(0)) : (m.v > a.theta);
+      acc = sel ? acc : -acc;
     }
-    round_cells<T>(o);
-    return o;
+    return X{rounded<T>(acc)};
   };
 
   // One input plane F (E the one before it): every row through the TS sweeps.
@@ -380,16 +359,14 @@ void star_steps(const StepArgs<T> a) {
           // defined only here, after the older value's last use: the two can
           // share a register (the compiler's own copies sit at the loop's end
           // and doubled the registers held)
-          if (in)
-#pragma unroll
-            for (int q = 0; q < V; ++q) asm volatile("" : "+v"(prv[s][r].v[q]) : "v"(o.v[q]));
+          if (in) asm volatile("" : "+v"(prv[s][r].v) : "v"(o.v));
         }
         if (in) x = s + 1 < TS ? keep(o) : o;
       }
       if (r >= TS && r < TS + J) {
         constexpr int G = RowStore<T>::G;
         const int q = r - TS;
-        rs.put(q % G, x.v[0]);
+        rs.put(q % G, x.v);
         if (q % G == G - 1) rs.store(po + (q - (G - 1)) * 8, lane, st);
       }
       __builtin_amdgcn_sched_barrier(0);  // row by row: bounds the live registers
@@ -674,12 +651,9 @@ __global__ __launch_bounds__(256) void star_steps_block(const StepArgs<T> a) {
         const bool sel = a.cond_mode == 0 ? (acc > A(0)) : (c[p] > a.theta);
         acc = sel ? acc : -acc;
       }
-      Cells<A, 1> o;
-      o.v[0] = acc;
-      round_cells<T>(o);
       if constexpr (R == 2) below[R - 1] = below[0];
       below[0] = m;
-      c[p] = o.v[0];
+      c[p] = rounded<T>(acc);
     }
   }
   if (x >= kHalo && x < kHalo + 8 && y >= kHalo && y < kHalo + 8) {
@@ -692,7 +666,7 @@ __global__ __launch_bounds__(256) void star_steps_block(const StepArgs<T> a) {
 template <class T, int TS, int FORM>
 auto strip_kernel() {
   if constexpr (FORM == kStar13) return &star13_steps<T>;
-  else return &star_steps<T, TS, 8, FORM>;
+  else return &star_steps<T, TS, FORM>;
 }
 
 // How a box is cut into strips of 8 rows and marches along k.  Two workgroups
@@ -774,14 +748,14 @@ const PassModel kModel[4][3] = {
      {{4.4f, 0.8f}, {{6.7f, 3.23f}, {7.07f, 4.91f}},
       {{6.08f, 2.05f, 1.3f, 1.83f}, {5.07f, 2.83f, 1.84f, 2.48f}}},
      {{4.57f, 0.54f}, {{6.8f, 3.81f}, {7.54f, 5.39f}},
-      {{6.32f, 2.15f, 1.42f, 1.85f}, {6.08f, 3.05f, 2.02f, 2.65f}}}},
+      {kNoStrip, kNoStrip}}},
     // cond, clamped values: FP64, FP32, BF16
     {{{4.95f, 1.54f}, {{6.71f, 5.74f}, {7.42f, 7.45f}},
       {{4.02f, 2.14f, 1.54f, 2.19f}, {20.0f, 1.68f, 1.84f, 2.75f}}},
      {{4.38f, 0.81f}, {{6.68f, 3.21f}, {7.06f, 4.89f}},
       {{6.06f, 1.74f, 1.17f, 1.62f}, {10.79f, 2.13f, 1.53f, 2.04f}}},
      {{4.54f, 0.54f}, {{6.74f, 3.8f}, {7.51f, 5.39f}},
-      {{6.19f, 2.03f, 1.32f, 1.72f}, {11.74f, 2.3f, 1.71f, 2.23f}}}},
+      {kNoStrip, kNoStrip}}},
     // 13-point: FP64, FP32, BF16
     {{{4.73f, 1.64f}, {{6.24f, 5.98f}, kNoLine},
       {{5.79f, 1.42f, 1.02f, 2.19f}, kNoStrip}},
@@ -818,10 +792,12 @@ float pass_time(const SweepLaunch &L, const PlanView &P, int ts, bool &block) {
 }
 
 // Strips of four FP64 sweeps with unclamped cond planes spill (0.75 ms a
-// sweep against 0.22 with three): not built.
+// sweep against 0.22 with three), and single sweeps are the faster ones of
+// BF16's cond and 13-point at every size (cond 0.62 us per thousand bricks and
+// sweep by three against 0.54): not built.
 template <class T, int TS, int FORM>
 constexpr bool strip_built() {
-  if (FORM == kStar13) return !std::is_same<T, bf16>::value;
+  if (std::is_same<T, bf16>::value) return FORM == kStar;
   return !(std::is_same<T, double>::value && TS == 4 && FORM == kCondRaw);
 }
 
