@@ -22,6 +22,7 @@ BK_F64, BK_F32, BK_BF16 = 0, 1, 2
 BK_STAR7, BK_STAR13, BK_STAR25, BK_CUBE125, BK_COND7 = 0, 1, 2, 3, 4
 BK_COND_REFERENCE, BK_COND_THRESHOLD = 0, 1
 BK_PLAN_COLUMN, BK_PLAN_QUAD = 1, 4
+BK_PASS_SINGLE, BK_PASS_BLOCKS, BK_PASS_STRIPS = 0, 1, 2
 BK_LAYOUT_8x8x8, BK_LAYOUT_4x8x16, BK_LAYOUT_4x8x16_F88 = 0, 1, 2
 BK_TUNE_ALL_LAYOUTS = 0x7
 BK_TUNE_BATCH_SCHEDULES = 0x100
@@ -221,6 +222,9 @@ SIGNATURES = {
     "bk_sweeps": (C.c_int, [C.POINTER(bk_sweep_desc), vp, C.c_uint32, C.c_int, C.c_int, vp]),
     "bk_sweeps_fused": (C.c_int, [C.POINTER(bk_sweep_desc), vp, vp, vp, C.c_uint32, C.c_int,
                                   C.c_int, vp]),
+    "bk_sweeps_passes": (C.c_int, [C.POINTER(bk_sweep_desc), vp, vp, vp, C.c_uint32, C.c_int,
+                                   C.POINTER(C.c_int), C.POINTER(C.c_int), C.c_int,
+                                   C.POINTER(C.c_int)]),
     "bk_ghost_images": (C.c_int, [longp, u32p, u32p, C.POINTER(C.c_uint32)]),
     "bk_decomp_layout": (C.c_int, [longp, C.c_int, C.c_size_t, C.c_size_t, u32p, u32p,
                                    C.POINTER(C.c_uint32), u32p, C.POINTER(bk_decomp_region),

@@ -794,6 +794,22 @@ def sweeps(st: Stencil, a: Brick, b: Brick, grid: PeriodicGrid, nsweeps: int,
     return b if nsweeps % 2 == 1 else a
 
 
+def sweep_passes(st: Stencil, a: Brick, b: Brick, grid: PeriodicGrid, nsweeps: int,
+                 plan="auto", fused: bool = False) -> list:
+    """The passes that ``sweeps`` of these arguments takes over the fields, as
+    (sweeps, form) pairs (bk_sweeps_passes; forms BK_PASS_*).  The box is
+    declared by the first such sequence itself."""
+    keep: list = []
+    d = _desc(st, b, a, grid, keep, plan=plan)
+    images = tuple(_vp(t.ptr) for t in grid.ghost_images) if fused else (None, None)
+    pairs = _vp(grid.d_pairs.ptr) if grid.d_pairs is not None else None
+    count, cap = C.c_int(), max(int(nsweeps), 1)
+    ts, forms = (C.c_int * cap)(), (C.c_int * cap)()
+    check(load().bk_sweeps_passes(C.byref(d), *images, pairs, grid.npairs, int(nsweeps), ts, forms,
+                                  cap, C.byref(count)))
+    return list(zip(ts[:count.value], forms[:count.value]))
+
+
 def cand_name(c) -> str:
     """A tuner candidate as text: layout, then the schedule."""
     lay = {0: "8x8x8", 1: "4x8x16", 2: "4x8x16/f88"}[c.layout]
@@ -829,6 +845,6 @@ def tune(st: Stencil, cells, dtype: int = BK_F64, ghost: int = 1, steps: int = 5
 __all__ = [
     "tune", "cand_name", "DeviceBuffer", "Stream", "Event", "BrickInfo", "init_grid", "movBrickInfo",
     "BrickStorage", "movBrickStorage", "Brick", "copyToBrick", "copyFromBrick",
-    "PeriodicGrid", "Plan", "plan_host", "sweep", "sweeps", "device_count", "device_sync", "DTYPE_NP",
+    "PeriodicGrid", "Plan", "plan_host", "sweep", "sweeps", "sweep_passes", "device_count", "device_sync", "DTYPE_NP",
     "DTYPE_SIZE", "BK_F64", "BK_F32", "BK_BF16",
 ]

@@ -94,6 +94,7 @@ hipError_t launch_cube_quads(const SweepLaunch &L, const PlanView &P, hipStream_
 // one pass of ts sweeps (3 or 4; radius 2: 2) from L.in to L.out.
 bool steps_fit(const SweepLaunch &L, const PlanView &P);
 void steps_costs(const SweepLaunch &L, const PlanView &P, float cost[5]);
+bool steps_by_blocks(const SweepLaunch &L, const PlanView &P, int ts);  // else by strips
 hipError_t launch_star_steps(const SweepLaunch &L, const PlanView &P, int ts, hipStream_t s);
 
 int plan_fail(int code, const char *msg);

@@ -303,6 +303,28 @@ class SweepSplit {
   }
 };
 
+// The sweeps of each pass of a sequence over a declared box.
+class BoxPasses {
+  bool many_;
+  int left_;
+  float cost_[5] = {};
+  SweepSplit split_;
+
+  const float *costs(const bk::SweepLaunch &L, const bk::PlanView &P) {
+    if (many_) bk::steps_costs(L, P, cost_);
+    return cost_;
+  }
+
+ public:
+  BoxPasses(const bk::SweepLaunch &L, const bk::PlanView &P, int nsweeps)
+      : many_(bk::steps_fit(L, P)), left_(nsweeps), split_(nsweeps - 1, costs(L, P)) {}
+  int next() {  // 0: none left
+    const int ts = left_ <= 1 ? left_ : many_ ? split_.next() : 1;
+    left_ -= ts;
+    return ts;
+  }
+};
+
 // Whether a sequence sweeps a declared box whose tables it uses are bound to it.
 bool box_path(const bk_sweep_desc *d, const uint32_t *pairs, uint32_t npairs, int nsweeps,
               int ghost_iters, const uint32_t *img_off, const uint32_t *img) {
@@ -340,13 +362,10 @@ hipError_t enqueue_sweeps(const bk_sweep_desc *d, const uint32_t *pairs, uint32_
   // several sweeps per pass besides; the last sweep runs by itself.
   if (boxed) {
     const bk::PlanView P = bk::plan_view(d->plan);
-    const bool many = bk::steps_fit(L, P);
-    float cost[5] = {};
-    if (many) bk::steps_costs(L, P, cost);
-    SweepSplit split(nsweeps - 1, cost);
+    BoxPasses passes(L, P, nsweeps);
     bool fwd = true, fresh = false;  // fresh: the input's ghost bricks are up to date
     for (int left = nsweeps; left; fwd = !fwd) {
-      const int ts = left == 1 || !many ? 1 : split.next();
+      const int ts = passes.next();
       left -= ts;
       L.in = fwd ? d->d_in : d->d_out;
       L.in_step = fwd ? d->in_step : d->out_step;
@@ -909,6 +928,36 @@ int bk_sweeps_fused(const bk_sweep_desc *d, const uint32_t *d_img_off, const uin
                 "bk_sweeps");
   return sweeps_impl(d, d_pairs, npairs, nsweeps, 1, d->d_list, d->nlist, d->plan, d_img_off,
                      d_img, use_graph, S(s));
+}
+
+int bk_sweeps_passes(const bk_sweep_desc *d, const uint32_t *d_img_off, const uint32_t *d_img,
+                     const uint32_t *d_pairs, uint32_t npairs, int nsweeps, int *sweeps,
+                     int *forms, int cap, int *npasses) {
+  int rc = check_desc(d, nsweeps > 1);
+  if (rc != BK_OK) return rc;
+  if (nsweeps < 0 || cap < 0 || !npasses || (cap && (!sweeps || !forms)))
+    return fail(BK_ERR_ARG, "bk_sweeps_passes: negative count or null pointer");
+  *npasses = 0;
+  if (desc_empty(d)) return BK_OK;
+  auto put = [&](int ts, int form) {
+    if (*npasses < cap) {
+      sweeps[*npasses] = ts;
+      forms[*npasses] = form;
+    }
+    ++*npasses;
+  };
+  if (!box_path(d, d_pairs, npairs, nsweeps, 1, d_img_off, d_img)) {
+    for (int t = 0; t < nsweeps; ++t) put(1, BK_PASS_SINGLE);
+    return BK_OK;
+  }
+  bk::SweepLaunch L;
+  to_launch(d, L);
+  const bk::PlanView P = bk::plan_view(d->plan);
+  BoxPasses passes(L, P, nsweeps);
+  while (const int ts = passes.next())
+    put(ts, ts == 1 ? BK_PASS_SINGLE
+                    : bk::steps_by_blocks(L, P, ts) ? BK_PASS_BLOCKS : BK_PASS_STRIPS);
+  return BK_OK;
 }
 
 int bk_sweeps_deep(const bk_sweep_desc *d, const uint32_t *d_all, uint32_t nall,

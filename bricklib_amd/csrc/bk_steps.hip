@@ -791,6 +791,16 @@ float pass_time(const SweepLaunch &L, const PlanView &P, int ts, bool &block) {
   return std::min(b, s);
 }
 
+}  // namespace
+
+bool steps_by_blocks(const SweepLaunch &L, const PlanView &P, int ts) {
+  bool block;
+  (void)pass_time(L, P, ts, block);
+  return block;
+}
+
+namespace {
+
 // Strips of four FP64 sweeps with unclamped cond planes spill (0.75 ms a
 // sweep against 0.22 with three), and single sweeps are the faster ones of
 // BF16's cond and 13-point at every size (cond 0.62 us per thousand bricks and
@@ -820,9 +830,7 @@ hipError_t launch_steps_t(const SweepLaunch &L, const PlanView &P, hipStream_t s
   a.theta = (A)L.theta;
   for (int q = 0; q < 13; ++q) a.c[q] = (A)L.coeff[q];
   a.nchunk = a.njg = a.njw = a.ksegs = 0;
-  bool block;
-  (void)pass_time(L, P, TS, block);
-  if (block) {
+  if (steps_by_blocks(L, P, TS)) {
     // half bricks while whole ones would leave half of the 256 CUs without a
     // workgroup (64 bricks: 1.43 us a sweep against 1.58; 216: 1.72 / 1.70)
     if (P.ncovered <= 128)

@@ -90,6 +90,9 @@ typedef struct bk_batch_s *bk_batch; /* batched sweeps (bk_batch_create) */
 typedef struct bk_arena_s *bk_arena; /* field arena (bk_arena_create) */
 
 enum bk_plan_shape { BK_PLAN_COLUMN = 1, BK_PLAN_QUAD = 4 };
+/* Forms of a pass (bk_sweeps_passes): one sweep by the single-sweep kernels,
+ * several by a workgroup a brick (or half brick), several by strips. */
+enum bk_pass_form { BK_PASS_SINGLE = 0, BK_PASS_BLOCKS = 1, BK_PASS_STRIPS = 2 };
 
 /* ---- library, errors, device ------------------------------------------ */
 int bk_version(void);
@@ -425,6 +428,14 @@ int bk_sweeps_deep(const bk_sweep_desc *d, const uint32_t *d_all, uint32_t nall,
 int bk_sweeps_fused(const bk_sweep_desc *d, const uint32_t *d_img_off,
                     const uint32_t *d_img, const uint32_t *d_pairs, uint32_t npairs,
                     int nsweeps, int use_graph, bk_stream s);
+/* The passes over the fields that bk_sweeps (d_img_off NULL) or
+ * bk_sweeps_fused takes for these arguments; nothing is launched.  Pass q
+ * makes sweeps[q] sweeps in the form forms[q]: more than one only over a
+ * declared box with bound tables (bk_plan_bind_box).  *npasses counts all, at
+ * most cap are written.  No counterpart in the reference. */
+int bk_sweeps_passes(const bk_sweep_desc *d, const uint32_t *d_img_off,
+                     const uint32_t *d_img, const uint32_t *d_pairs, uint32_t npairs,
+                     int nsweeps, int *sweeps, int *forms, int cap, int *npasses);
 /* Drop every cached graph (frees their device resources). */
 int bk_graph_cache_clear(void);
 
