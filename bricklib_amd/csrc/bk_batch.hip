@@ -100,7 +100,8 @@ struct bk_batch_s {
   std::unique_ptr<Span[]> span;  // bk_batch_set's: 2 * max_reqs
   bool apart = false;  // the groups of the set may run side by side
   uint64_t bricks = 0;  // of the set's requests with sweeps left
-  // captured runs keyed by (tick count, sweep and refresh group masks); an
+  // captured runs keyed by (tick count, sweep groups with the cube's forms,
+  // refresh groups and whether the groups go side by side); an
   // exec is destroyed only once its last launch has completed, so a caller
   // may queue the next run while the previous one is still on the device
   bk::ExecCache<std::tuple<uint32_t, uint64_t, uint32_t>> graphs{64};

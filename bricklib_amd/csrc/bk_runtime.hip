@@ -352,14 +352,15 @@ hipError_t enqueue_sweeps(const bk_sweep_desc *d, const uint32_t *pairs, uint32_
   L.img_off = img_off;
   L.img = img;
   const size_t es = (size_t)dt_size(d->dtype);
-  // Where the plan's bricks are a periodic box whose ghost bricks this sequence
-  // refreshes before every sweep, sweeps read the periodic image itself and
+  // Over a declared box whose ghost bricks this sequence refreshes before every
+  // sweep, by tables that are the box's, sweeps read the periodic image itself and
   // only the last ones touch ghost bricks: the last sweep's input has them
   // fresh, and in the fused form its output too.  Ten sweeps, us each, with a
   // refresh (fused) every time / now: 25-point FP32 384^3 128 (122) / 110, 13-
   // point FP64 160^3 37.0 (25.5) / 21.6 (20.7), 125-point FP64 160^3 48.9 /
-  // 34.1, 13-point FP32 of 9x7x8 bricks 16.1 (10.7) / 7.0 (6.7).  Stencils of radius 1 take
-  // several sweeps per pass besides; the last sweep runs by itself.
+  // 34.1, 13-point FP32 of 9x7x8 bricks 16.1 (10.7) / 7.0 (6.7).  The 7-point star, cond
+  // and the 13-point star take several sweeps per pass besides; the last sweep runs by
+  // itself.
   if (boxed) {
     const bk::PlanView P = bk::plan_view(d->plan);
     BoxPasses passes(L, P, nsweeps);

@@ -309,9 +309,10 @@ int bk_plan_build_host(const uint32_t *h_adj, uint32_t nbricks,
  * neighbour of every box brick must be the brick of the wrapped box, or a
  * ghost brick that a pair makes its copy -- BK_ERR_UNSUPPORTED otherwise, and
  * the plan stays as it was.  No counterpart in the reference.  Allocates
- * device memory (the ids, two words a brick and, with pairs, an adjacency of
- * its own), filled on s when the call returns; a capture of s is left as it
- * is.  Sequences use the box only with device tables bound to it:
+ * device memory (the ids, two words a brick of the adjacency and, with pairs,
+ * an adjacency of its own of 27 words each: 116 bytes a brick, 250 MB for a
+ * plan of 1024^3 cells), filled on s when the call returns; a capture of s is
+ * left as it is.  Sequences use the box only with device tables bound to it:
  *
  * bk_plan_bind_box compares device tables with the declared box (on s, which
  * it waits for): d_adj, the npairs pairs of d_pairs, and with d_img_off and
@@ -422,7 +423,8 @@ int bk_sweeps_deep(const bk_sweep_desc *d, const uint32_t *d_all, uint32_t nall,
  * output brick into its ghost images (d_img_off / d_img from
  * bk_ghost_images, uploaded), so the next sweep's input is already
  * refreshed.  The same bits as bk_sweeps, with one ghost write per sweep
- * instead of a refresh's read + write.  Star and cond stencils without a
+ * instead of a refresh's read + write (over a box with bound tables only the
+ * last two sweeps do: see bk_plan_bind_box).  Star and cond stencils without a
  * plan (one brick per wave) or with a quad plan; otherwise
  * BK_ERR_UNSUPPORTED. */
 int bk_sweeps_fused(const bk_sweep_desc *d, const uint32_t *d_img_off,
@@ -531,8 +533,10 @@ int bk_batch_destroy(bk_batch batch);
  * them have completed. */
 int bk_batch_set(bk_batch batch, const bk_batch_req *reqs, uint32_t n, bk_stream s);
 /* Run nticks ticks.  With use_graph != 0 the launches are captured once per
- * (nticks, set of non-empty groups) and replayed; the tables are read when
- * the kernels run, so later bk_batch_set calls need no new capture. */
+ * (nticks, set of non-empty groups, form of the cube's kernels, whether the
+ * groups go side by side) and replayed; the tables are read when the kernels
+ * run, so later bk_batch_set calls that leave these as they are need no new
+ * capture. */
 int bk_batch_run(bk_batch batch, uint32_t nticks, int use_graph, bk_stream s);
 
 /* ---- serving loop ------------------------------------------------------ */
