@@ -11,6 +11,7 @@ operation goes through the C-ABI; nothing here computes on the CPU.
 from __future__ import annotations
 
 import ctypes as C
+import itertools
 import struct
 import threading
 from dataclasses import dataclass, field
@@ -42,11 +43,14 @@ def _vp(x) -> C.c_void_p:
 class DeviceBuffer:
     """An HBM allocation owned by Python (freed with the object)."""
 
+    _stamps = itertools.count(1)
+
     def __init__(self, nbytes: int):
         self.nbytes = int(nbytes)
         p = C.c_void_p()
         check(load().bk_alloc(C.c_size_t(self.nbytes), C.byref(p)))
         self.ptr = p.value or 0
+        self.stamp = next(self._stamps)  # of the last upload or clear, among all buffers
 
     @classmethod
     def from_array(cls, arr: np.ndarray, stream=None) -> "DeviceBuffer":
@@ -59,6 +63,7 @@ class DeviceBuffer:
         arr = np.ascontiguousarray(arr)
         if offset + arr.nbytes > self.nbytes:
             raise ValueError("upload past the end of the buffer")
+        self.stamp = next(self._stamps)
         check(load().bk_memcpy_h2d(_vp(self.ptr + offset), _vp(arr), C.c_size_t(arr.nbytes),
                                    _vp(stream)))
 
@@ -74,6 +79,7 @@ class DeviceBuffer:
         return out
 
     def zero(self, stream=None) -> None:
+        self.stamp = next(self._stamps)
         check(load().bk_zero(_vp(self.ptr), C.c_size_t(self.nbytes), _vp(stream)))
 
     def free(self) -> None:
@@ -211,6 +217,7 @@ class BrickStorage:
         es = DTYPE_SIZE[dtype]
         buf.nbytes = ((int(chunks) * int(step) * es + 2047) // 2048) * 2048
         buf.ptr = p.value or 0
+        buf.stamp = next(buf._stamps)
         return cls(buf, int(chunks), int(step), int(dtype))
 
     @property
@@ -338,8 +345,8 @@ class Plan:
                                      _stream_of(stream)))
         self.boxed = True
 
-    def bind_box(self, d_adj: int, d_pairs: int = 0, npairs: int = 0, d_img_off: int = 0,
-                 d_img: int = 0, stream=None) -> None:
+    def bind_box(self, d_adj: int, d_pairs=None, npairs: int = 0, d_img_off=None, d_img=None,
+                 stream=None) -> None:
         """Check these device tables against the declared box and let
         sequences that come with them use it (bk_plan_bind_box), until one of
         them is written through the library or freed."""
@@ -521,9 +528,16 @@ class PeriodicGrid:
         """Ahead of a sequence of sweeps that refresh this grid: declare one
         of its own quad plans a periodic box, once, and bind the tables that
         the sequence comes with."""
-        images = tuple(t.ptr for t in self.ghost_images) if fused else (0, 0)
-        tables = (self.info.dptr, self.d_pairs.ptr if self.d_pairs is not None else 0,
-                  self.npairs, *images)
+        adj, pairs = getattr(self.info, "dev", None), self.d_pairs
+        if adj is None:
+            return
+        off, img = self.ghost_images if fused else (None, None)
+        # (a table that was written into is as good as another: its binding ended)
+        try:
+            tables = ((adj.stamp, pairs and pairs.stamp) if off is None else
+                      (adj.stamp, pairs and pairs.stamp, off.stamp, img.stamp))
+        except AttributeError:  # memory of the caller's own kind
+            tables = tuple(t and getattr(t, "stamp", t.ptr) for t in (adj, pairs, off, img))
         if tables in plan.tables or plan.shape != "quad":
             return
         if not plan.boxed and not any(plan is p for p in list(self._plans.values())):
@@ -534,13 +548,16 @@ class PeriodicGrid:
             try:
                 if not plan.boxed:
                     plan.set_box(self.info, self.nb, self.interior, self.pairs, stream)
-                plan.bind_box(*tables, stream=stream)
+                plan.bind_box(adj.ptr, pairs and pairs.ptr, self.npairs, off and off.ptr,
+                              img and img.ptr, stream=stream)
             except _lib.BrickError as e:
                 if e.code == _lib.BK_ERR_NOMEM:
                     return  # one sweep per pass now; the next sequence tries again
                 if e.code != _lib.BK_ERR_UNSUPPORTED:
                     raise
                 # not a periodic box (changed tables): one sweep per pass with them
+            if len(plan.tables) > 64:
+                plan.tables.clear()
             plan.tables.add(tables)
 
     @property

@@ -35,7 +35,7 @@ class FakePlan:
 
 def _grid(plan):
     g = PeriodicGrid.__new__(PeriodicGrid)
-    g.info, g.d_pairs = SimpleNamespace(dptr=4096), None
+    g.info, g.d_pairs = SimpleNamespace(dev=SimpleNamespace(ptr=4096)), None
     g.pairs = np.empty(0, np.uint32)
     g.interior, g.nb, g._plans = np.arange(8, dtype=np.uint32), (2, 2, 2), {"p": plan}
     return g
