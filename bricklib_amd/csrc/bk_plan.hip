@@ -744,9 +744,13 @@ int bk_plan_bind_box(bk_plan p, const uint32_t *d_adj, const uint32_t *d_pairs,
     const uintptr_t lo = reinterpret_cast<uintptr_t>(t);
     return std::make_pair(lo, t ? lo + 4 * words : lo);
   };
-  bk::bind_box(p->id, {d_adj, c.pairs, d_img_off, d_img,
-                       {span(d_adj, (size_t)nbricks * 27), span(c.pairs, 2 * (size_t)npairs),
-                        span(d_img_off, (size_t)nbricks + 1), span(d_img, npairs)}});
+  try {
+    bk::bind_box(p->id, {d_adj, c.pairs, d_img_off, d_img,
+                         {span(d_adj, (size_t)nbricks * 27), span(c.pairs, 2 * (size_t)npairs),
+                          span(d_img_off, (size_t)nbricks + 1), span(d_img, npairs)}});
+  } catch (const std::bad_alloc &) {
+    return bk::plan_fail(BK_ERR_NOMEM, "bk_plan_bind_box: out of host memory");
+  }
   return BK_OK;
 }
 
